@@ -2453,107 +2453,159 @@ __global__ __launch_bounds__(1024) void k_reduce_max(const double *__restrict__ 
 // x-z mean statistics, PP_MEAN_ZX_FLOW_TG (processing/PP_MEAN_ZX.f90:14-307), channel.  Per
 // row J the 122 statistics are (s): 0..3 U1 (u, v, w, p), 4..6 UP, 7..12 U2 (the reference's
 // upper-triangle storage index), 13..22 U3, 23..31 DVDL1 (3 x 3, row major), 32..40 DVDLP,
-// 41..121 DVDL2 (9 x 9, row major).  Thread (i, J) sums one group of them over k:
-// GRP 0 s = 0..22, GRP 1 s = 23..40, GRP 2..4 the DVDL2 rows l1 = 3 (GRP-2) .. 3 (GRP-2)+2.
-template <int GRP>
-__global__ __launch_bounds__(64) void k_mean_zx(Geo g, const double *__restrict__ q, const double *__restrict__ pr,
-                                                double *__restrict__ part)
+// 41..121 DVDL2 (9 x 9, row major).
+// All of them from one pass over the fields: DVDL2 is symmetric, so the 86 sums (kMeanSums:
+// s = 0..40, then DVDL2's upper triangle by rows) of a column stay in a lane's registers.  A lane
+// owns one column i of row J and a run of KC planes, which it marches carrying plane k's values.
+// The x-neighbours' values come from the neighbouring lanes: a wavefront's 62 inner lanes own
+// columns, and a row's runs follow each other with their two wrapped columns (positions
+// z (L + 2) .. z (L + 2) + L + 1 are columns -1 .. L of run z), so that wavefronts are full for
+// any L.  That leaves 9 loads a point.  With the neighbours loaded too (18 a point, the sums in
+// two side-by-side roles) the texture address unit was busy 79 % of 274 us at 256 x 192 x 256; in
+// five launches over groups of the sums, each reading the fields again and writing 48 MB of
+// per-column partials, it took 1325 us; this pass takes 151 us (2.7 TB/s of the four fields),
+// half of its cycles in FP64 arithmetic, the rest waiting for loads at the two wavefronts per
+// SIMD that 86 sums leave room for.
+// The sums over the lanes are formed by halving: each of six exchanges sends half of the values a
+// lane still holds, 87 exchanges in all, where a butterfly of each value would take 516.
+constexpr int kMeanSums = 86, kMeanCols = 62;
+
+// The value of the next (UP) or previous lane; lane 63 (0) gets a value of no meaning.
+template <bool UP> __device__ __forceinline__ double lane_beside(double v)
 {
-#pragma clang fp contract(off)
-    constexpr int NS = GRP == 0 ? 23 : (GRP == 1 ? 18 : 27);
-    constexpr int S0 = GRP == 0 ? 0 : (GRP == 1 ? 23 : 41 + 27 * (GRP - 2));
-    const int L = g.L, N = g.N;
-    const int i = blockIdx.x * 64 + threadIdx.x, J = blockIdx.y + 1;
-    if (i >= L) return;
-    const size_t hs = (size_t)N * (g.M + 2) * L;
-    const double *U = q, *V = q + hs, *W = q + 2 * hs;
-    const int ip = i == L - 1 ? 0 : i + 1, im = i == 0 ? L - 1 : i - 1;
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), UP ? 0x130 : 0x138, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), UP ? 0x130 : 0x138, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+__global__ __launch_bounds__(64, 2) void k_mean_zx(Geo g, const double *__restrict__ q,
+                                                   const double *__restrict__ pr, double *__restrict__ part, int KC,
+                                                   int NZ, int ntile)
+{
+    const int L = g.L, M = g.M, N = g.N;
+    // (tile, row), rows fastest, dealt to the 8 XCDs in contiguous runs: a row's neighbours are
+    // read through the same L2
+    const int n = M * ntile, per = (n + 7) >> 3, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (id >= n) return;
+    const int J = id % M + 1, tile = id / M;
+    const int pos = min(max(tile * kMeanCols + (int)threadIdx.x - 1, 0), NZ * (L + 2) - 1);
+    const int z = pos / (L + 2), col = pos - z * (L + 2) - 1;
+    const bool mine = threadIdx.x >= 1 && threadIdx.x <= kMeanCols && col >= 0 && col < L &&
+                      tile * kMeanCols + (int)threadIdx.x - 1 < NZ * (L + 2);
+    const int i = col < 0 ? L - 1 : (col == L ? 0 : col);
+    const int k0 = z * KC, k1 = min(k0 + KC, N);
+    const size_t hs = (size_t)N * (M + 2) * L, ps = (size_t)(M + 2) * L;
+    const double *U = q + (size_t)J * L + i, *V = U + hs, *W = V + hs, *P = pr + (size_t)J * L + i;
     const double dycp = g.dyci[J + 1], dyc = g.dyci[J], dyf = g.dyfi[J - 1];
-    double acc[NS];
+    double acc[88];
 #pragma unroll
-    for (int t = 0; t < NS; ++t) acc[t] = 0.0;
-    for (int k = 0; k < N; ++k) {
-        const int kp = k == N - 1 ? 0 : k + 1, km = k == 0 ? N - 1 : k - 1;
-        auto X = [&](const double *f, int ii, int jj, int kk) { return f[hix(g, ii, jj, kk)]; };
-        double u[3];
-        u[0] = X(U, i, J, k) + X(U, ip, J, k);
-        u[1] = X(V, i, J, k) + X(V, i, J + 1, k);
-        u[2] = X(W, i, J, k) + X(W, i, J, kp);
-        const double p = X(pr, i, J, k);
-        if constexpr (GRP == 0) {
+    for (int s = 0; s < 88; ++s) acc[s] = 0.0;
+    {
+        size_t o = (size_t)k0 * ps;
+        const size_t om = (size_t)(k0 == 0 ? N - 1 : k0 - 1) * ps;
+        double ukm = U[om] + lane_beside<true>(U[om]), vkm = V[om] + V[om + L];
+        double ui = U[o], vi = V[o], vt = V[o + L], wi = W[o], wjp = W[o + L], wjm = (W - L)[o];
+        for (int k = k0; k < k1; ++k) {
+            const size_t on = (k == N - 1) ? 0 : o + ps;
+            const double uin = U[on], vin = V[on], vtn = V[on + L], win = W[on], wjpn = W[on + L], wjmn = (W - L)[on];
+            const double uj = U[o + L], um = (U - L)[o], p = P[o];
+            const double uip = lane_beside<true>(ui), w2 = wi + win;
+            const double u[3] = {ui + uip, vi + vt, w2};
+            const double gr[9] = {uip - ui,
+                                  (uj + lane_beside<true>(uj) - u[0]) * dycp + (u[0] - (um + lane_beside<true>(um))) * dyc,
+                                  (uin + lane_beside<true>(uin)) - ukm,
+                                  lane_beside<true>(u[1]) - lane_beside<false>(u[1]),
+                                  (vt - vi) * dyf,
+                                  (vin + vtn) - vkm,
+                                  lane_beside<true>(w2) - lane_beside<false>(w2),
+                                  ((wjp + wjpn) - w2) * dycp + (w2 - (wjm + wjmn)) * dyc,
+                                  win - wi};
+            ukm = u[0];
+            vkm = u[1];
+            ui = uin; vi = vin; vt = vtn; wi = win; wjp = wjpn; wjm = wjmn;
+            o = on;
+            int s2 = 7, s3 = 13, s4 = 41;
+            acc[3] += p;
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
-                acc[a] = acc[a] + u[a];
-                acc[4 + a] = acc[4 + a] + u[a] * p;
-            }
-            acc[3] = acc[3] + p;
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
+                acc[a] += u[a];
+                acc[4 + a] += u[a] * p;
 #pragma unroll
                 for (int b = a; b < 3; ++b) {
-                    const int l = ((a + 1) * (6 - a)) / 2 + (b + 1) - 3;
-                    acc[7 + l - 1] = acc[7 + l - 1] + u[a] * u[b];
+                    const double uu = u[a] * u[b];
+                    acc[s2++] += uu;
+#pragma unroll
+                    for (int c = b; c < 3; ++c) acc[s3++] += uu * u[c];
                 }
+            }
 #pragma unroll
-            for (int a = 0; a < 3; ++a)
+            for (int a = 0; a < 9; ++a) {
+                acc[23 + a] += gr[a];
+                acc[32 + a] += gr[a] * p;
 #pragma unroll
-                for (int b = a; b < 3; ++b)
-#pragma unroll
-                    for (int c = b; c < 3; ++c) {
-                        const int l = (a + 1) * (5 - a) + ((b + 1) * (6 - b)) / 2 + (c + 1) - 8;
-                        acc[13 + l - 1] = acc[13 + l - 1] + u[a] * u[b] * u[c];
-                    }
-        } else {
-            const double ujp0 = X(U, i, J + 1, k) + X(U, ip, J + 1, k), ujm0 = X(U, i, J - 1, k) + X(U, ip, J - 1, k);
-            const double ukp0 = X(U, i, J, kp) + X(U, ip, J, kp), ukm0 = X(U, i, J, km) + X(U, ip, J, km);
-            const double uip2 = X(W, ip, J, k) + X(W, ip, J, kp), uim2 = X(W, im, J, k) + X(W, im, J, kp);
-            const double ujp2 = X(W, i, J + 1, k) + X(W, i, J + 1, kp), ujm2 = X(W, i, J - 1, k) + X(W, i, J - 1, kp);
-            const double uip1 = X(V, ip, J, k) + X(V, ip, J + 1, k), uim1 = X(V, im, J, k) + X(V, im, J + 1, k);
-            const double ukp1 = X(V, i, J, kp) + X(V, i, J + 1, kp), ukm1 = X(V, i, J, km) + X(V, i, J + 1, km);
-            double gr[3][3];
-            gr[0][0] = X(U, ip, J, k) - X(U, i, J, k);
-            gr[0][1] = (ujp0 - u[0]) * dycp + (u[0] - ujm0) * dyc;
-            gr[0][2] = ukp0 - ukm0;
-            gr[1][0] = uip1 - uim1;
-            gr[1][1] = (X(V, i, J + 1, k) - X(V, i, J, k)) * dyf;
-            gr[1][2] = ukp1 - ukm1;
-            gr[2][0] = uip2 - uim2;
-            gr[2][1] = (ujp2 - u[2]) * dycp + (u[2] - ujm2) * dyc;
-            gr[2][2] = X(W, i, J, kp) - X(W, i, J, k);
-            if constexpr (GRP == 1) {
-#pragma unroll
-                for (int a = 0; a < 3; ++a)
-#pragma unroll
-                    for (int b = 0; b < 3; ++b) {
-                        acc[3 * a + b] = acc[3 * a + b] + gr[a][b];
-                        acc[9 + 3 * a + b] = acc[9 + 3 * a + b] + gr[a][b] * p;
-                    }
-            } else {
-#pragma unroll
-                for (int r = 0; r < 3; ++r) {
-                    const int l1 = 3 * (GRP - 2) + r;
-                    const double gl = gr[l1 / 3][l1 % 3];
-#pragma unroll
-                    for (int l2 = 0; l2 < 9; ++l2) acc[9 * r + l2] = acc[9 * r + l2] + gl * gr[l2 / 3][l2 % 3];
-                }
+                for (int b = a; b < 9; ++b) acc[s4++] += gr[a] * gr[b];
             }
         }
     }
 #pragma unroll
-    for (int t = 0; t < NS; ++t) part[((size_t)(J - 1) * 122 + S0 + t) * L + i] = acc[t];
+    for (int s = 0; s < 88; ++s) acc[s] = mine ? acc[s] : 0.0;
+    // sums over the lanes: 86 -> 43 -> 22 -> 11 -> 6 -> 3 -> 2 values held; off, cnt: this lane's
+    int off = 0, cnt = kMeanSums;
+#define CHS_HALVE(H, BIT)                                                           \
+    {                                                                               \
+        const bool up = threadIdx.x & BIT;                                          \
+        _Pragma("unroll") for (int j = 0; j < H; ++j) {                             \
+            const double lo = acc[j], hi = acc[j + H];                              \
+            const double got = __shfl_xor(up ? lo : hi, BIT, 64);                   \
+            acc[j] = (up ? hi : lo) + got;                                          \
+        }                                                                           \
+        acc[H] = 0.0;                                                               \
+        off += up ? H : 0;                                                          \
+        cnt = up ? cnt - H : min(cnt, H);                                           \
+    }
+    CHS_HALVE(43, 32)
+    CHS_HALVE(22, 16)
+    CHS_HALVE(11, 8)
+    CHS_HALVE(6, 4)
+    CHS_HALVE(3, 2)
+    CHS_HALVE(2, 1)
+#undef CHS_HALVE
+    double *o = part + ((size_t)(J - 1) * ntile + tile) * kMeanSums + off;
+    if (cnt > 0) o[0] = acc[0];
+    if (cnt > 1) o[1] = acc[1];
 }
 
-// Row sums of the partials in index order, times the statistic's coefficient.
-__global__ __launch_bounds__(256) void k_mean_zx_sum(int L, int n, const double *__restrict__ part,
-                                                     const double *__restrict__ coef, double *__restrict__ out)
+// The coefficients of the statistics (PP_MEAN_ZX.f90:34-58, :261-292): VL1313_tg = 1 / (NCL1 NCL3)
+// and the 3 x 3 gradient factors, which DVDL2 takes twice.
+struct MeanCoef {
+    double vl, cog[9];
+};
+
+// Row J's 122 statistics from its tiles' sums, added in tile order.
+__global__ __launch_bounds__(128) void k_mean_zx_sum(int ntile, MeanCoef c, const double *__restrict__ part,
+                                                     double *__restrict__ out)
 {
-#pragma clang fp contract(off)
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= n) return;
-    const double *p = part + (size_t)t * L;
-    double s = 0.0;
-    for (int i = 0; i < L; ++i) s = s + p[i];
-    out[t] = s * coef[t % 122];
+    __shared__ double sum[kMeanSums];
+    const int t = threadIdx.x;
+    const double *p = part + (size_t)blockIdx.x * ntile * kMeanSums;
+    if (t < kMeanSums) {
+        double s = 0.0;
+        for (int i = 0; i < ntile; ++i) s += p[(size_t)i * kMeanSums + t];
+        sum[t] = s;
+    }
+    __syncthreads();
+    if (t >= 122) return;
+    int s = t;
+    double f = c.vl;
+    if (t < 13) f = t == 3 ? c.vl : t < 7 ? c.vl * 0.5 : c.vl * (0.5 * 0.5);
+    else if (t < 23) f = c.vl * (0.5 * 0.5 * 0.5);
+    else if (t < 41) f = c.cog[(t - 23) % 9];
+    else {
+        const int a = (t - 41) / 9, b = (t - 41) % 9, lo = min(a, b), hi = max(a, b);
+        s = 41 + lo * 9 - lo * (lo - 1) / 2 + hi - lo;
+        f = c.cog[a] * c.cog[b];
+    }
+    out[(size_t)blockIdx.x * 122 + t] = sum[s] * f;
 }
 
 }  // namespace
@@ -2824,6 +2876,7 @@ struct chs_ctx {
     float *pp32 = nullptr;   // FP32 copy of the Poisson pivots (mixed form, high modes)
     double *pp00 = nullptr;  // (0,0)-mode pivots without FFT99's decoupling (FISHPACK gauge)
     int npartial = 0;
+    double *mean_part = nullptr, *mean_host = nullptr;   // chs_mean_zx_tg: tile sums, pinned result
     void *twx = nullptr, *twz = nullptr;
     void *rtwx = nullptr, *rtwz = nullptr;   // register-FFT pass twiddles (chs_fftr.h), if planned
     chs::FftPlan px, pz;
@@ -3859,9 +3912,10 @@ void chs_destroy(chs_ctx *c)
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void *ptrs[] = {c->cf, c->q, c->qs, c->pr, c->phi, c->div, c->h0, c->rhs, c->rhs2, c->spec, c->pp,
-                    c->pp32, c->pp00, c->partial, c->scal, c->twx, c->twz, c->rtwx, c->rtwz, c->cn_stamp};
+                    c->pp32, c->pp00, c->partial, c->scal, c->twx, c->twz, c->rtwx, c->rtwz, c->cn_stamp, c->mean_part};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    if (c->mean_host) (void)hipHostFree(c->mean_host);
     for (auto &t : c->cn) {
         if (t.gx) (void)hipFree(t.gx);
         if (t.gz) (void)hipFree(t.gz);
@@ -4777,43 +4831,24 @@ extern "C" int chs_mean_zx_tg(chs_ctx *c, double *stats, double *scal)
 {
     if (!c || (!stats && !scal)) return fail(c, CHS_E_ARG, "chs_mean_zx_tg: null argument");
     const int L = c->L, M = c->M, N = c->N;
-    // coefficients (PP_MEAN_ZX.f90:34-58, :261-292): VL1313_tg = 1 / (NCL1 NCL3)
     const double vl = 1.0 / (double)(L * N);
-    const double cog1[3][3] = {{vl * c->dxi, vl * 0.25, vl * 0.25 * c->dzi},
-                               {vl * 0.25 * c->dxi, vl, vl * 0.25 * c->dzi},
-                               {vl * 0.25 * c->dxi, vl * 0.25, vl * c->dzi}};
-    std::vector<double> coef(122);
-    for (int a = 0; a < 3; ++a) coef[a] = vl * 0.5;
-    coef[3] = vl;
-    for (int a = 0; a < 3; ++a) coef[4 + a] = vl * 0.5;
-    for (int t = 0; t < 6; ++t) coef[7 + t] = vl * (0.5 * 0.5);
-    for (int t = 0; t < 10; ++t) coef[13 + t] = vl * (0.5 * 0.5 * 0.5);
-    for (int a = 0; a < 3; ++a)
-        for (int b = 0; b < 3; ++b) coef[23 + 3 * a + b] = coef[32 + 3 * a + b] = cog1[a][b];
-    for (int l1 = 0; l1 < 9; ++l1)
-        for (int l2 = 0; l2 < 9; ++l2) coef[41 + 9 * l1 + l2] = cog1[l1 / 3][l1 % 3] * cog1[l2 / 3][l2 % 3];
-    const size_t n = (size_t)M * 122;
-    double *buf = nullptr;
-    HIPCHK(c, hipMalloc(&buf, sizeof(double) * (n * L + 122 + n)));
-    double *part = buf, *dcoef = buf + n * L, *dout = dcoef + 122;
-    std::vector<double> hout(n);
-    hipError_t e = hipMemcpyAsync(dcoef, coef.data(), sizeof(double) * 122, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) {
-        const dim3 grd((L + 63) / 64, M);
-        hipLaunchKernelGGL(k_mean_zx<0>, grd, dim3(64), 0, c->stream, c->geo, c->q, c->pr, part);
-        hipLaunchKernelGGL(k_mean_zx<1>, grd, dim3(64), 0, c->stream, c->geo, c->q, c->pr, part);
-        hipLaunchKernelGGL(k_mean_zx<2>, grd, dim3(64), 0, c->stream, c->geo, c->q, c->pr, part);
-        hipLaunchKernelGGL(k_mean_zx<3>, grd, dim3(64), 0, c->stream, c->geo, c->q, c->pr, part);
-        hipLaunchKernelGGL(k_mean_zx<4>, grd, dim3(64), 0, c->stream, c->geo, c->q, c->pr, part);
-        hipLaunchKernelGGL(k_mean_zx_sum, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, L, (int)n,
-                           part, dcoef, dout);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipMemcpyAsync(hout.data(), dout, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(buf);
-    if (e != hipSuccess) return fail(c, CHS_E_HIP, std::string("chs_mean_zx_tg: ") + hipGetErrorString(e));
-    if (stats) std::copy(hout.begin(), hout.end(), stats);
+    const MeanCoef mc = {vl, {vl * c->dxi, vl * 0.25, vl * 0.25 * c->dzi, vl * 0.25 * c->dxi, vl, vl * 0.25 * c->dzi,
+                              vl * 0.25 * c->dxi, vl * 0.25, vl * c->dzi}};
+    // planes per lane: 32, fewer where that leaves the GPU's 2048 two-per-SIMD wavefronts short
+    int KC = 32;
+    while (KC > 4 && (long long)M * L * ((N + KC - 1) / KC) < 64LL * 2 * 2048) KC >>= 1;
+    const int NZ = (N + KC - 1) / KC, ntile = ((L + 2) * NZ + kMeanCols - 1) / kMeanCols;
+    const size_t n = (size_t)M * 122, np = (size_t)M * ntile * kMeanSums;
+    // partials and the pinned result, laid out at the first call for this mesh (KC follows from it)
+    if (!c->mean_part) HIPCHK(c, hipMalloc(&c->mean_part, sizeof(double) * np));
+    if (!c->mean_host) HIPCHK(c, hipHostMalloc((void **)&c->mean_host, sizeof(double) * n, hipHostMallocDefault));
+    hipLaunchKernelGGL(k_mean_zx, dim3(8 * ((M * ntile + 7) / 8)), dim3(64), 0, c->stream, c->geo, c->q, c->pr,
+                       c->mean_part, KC, NZ, ntile);
+    hipLaunchKernelGGL(k_mean_zx_sum, dim3(M), dim3(128), 0, c->stream, ntile, mc, c->mean_part, c->mean_host);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const double *hout = c->mean_host;
+    if (stats) std::copy(hout, hout + n, stats);
     if (scal) {   // U1mean_WORK_tg, U1maxx_WORK_tg (PP_MEAN_ZX.f90:294-305), Area_inlet (COORDJR.f90:368-373)
         double um = 0.0, ux = 0.0, area = 0.0;
         for (int J = 1; J <= M; ++J) {

@@ -80,3 +80,19 @@ def test_gpu_matches_oracle_large(pkg):
     st, sc = ch.PP_MEAN_ZX_FLOW_TG()
     check(st, sc, st0, sc0)
     ch.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,M,N", [(4, 4, 4), (60, 5, 6), (64, 4, 36), (120, 7, 34), (150, 9, 128)])
+def test_gpu_lane_and_run_edges(pkg, L, M, N):
+    """Wavefronts of 62 columns over runs of z-planes: lines shorter and longer than a wavefront,
+    runs that wrap a wavefront, a last run cut short, idle lanes; bounds as in ``check``."""
+    co = pkg.channel_setup(L, M, N, STR2=1.7)
+    q, p = pkg.poiseuille_perturbed(co, seed=L + N, amp=0.3)
+    p[:, 1:M + 1, :] = np.random.default_rng(L).standard_normal((N, M, L)) * 0.1
+    o = oracle.OracleTG(setup.Mesh(L, M, N, STR2=1.7), 2800.0)
+    o.set_fields(q, p)
+    ch = pkg.ChannelTG(co, pkg.PLAIN_FP64)
+    ch.upload(q, p)
+    check(*ch.PP_MEAN_ZX_FLOW_TG(), *o.mean_zx())
+    ch.close()
