@@ -34,6 +34,7 @@
 #include "../../include/chapsim_hip.h"
 #include "chs_fft.h"
 #include "chs_fftr.h"
+#include "chs_fftg.h"
 
 using chs::cpx;
 
@@ -1867,12 +1868,21 @@ __global__ __launch_bounds__(1024) void k_ytdma_chunk(Geo g, const double *__res
     k_ytdma_chunk_b<T, C>(g, amph, apph, pp, pp32, pp00, spec, int(blockDim.y), own_blk());
 }
 
+// Where an inverse x-transform puts the solution: the halo field [N][M+2][L] with the Neumann
+// ghost rows of BC_WALL_DPH (BC_WALL.f90:369-386) (pitch (M+2) L, row0 = 0), or a cell field
+// [N][M][L] (pitch M L, row0 = 1), which saves the standalone solve a pass that copies the rows.
+struct PhiOut {
+    double *phi;
+    size_t pitch;
+    int row0;
+};
+
 // Inverse real x-transform of TK z-planes at row J -> phi (halo field) and the Neumann
 // ghost rows of BC_WALL_DPH_tg (BC_WALL.f90:369-386).  Z = A + i B with the Hermitian
 // extension; imaginary parts at kx = 0 and L/2 are not used (FFT99.f90:84-86).
 template <typename T>
-__device__ __forceinline__ void k_fftx_inv_b(Geo g, PoisArgs pa, const cpx<T> *__restrict__ spec,
-                                                  double *__restrict__ phi, int TK, const Blk blk)
+__device__ __forceinline__ void k_fftx_inv_b(Geo g, PoisArgs pa, const cpx<T> *__restrict__ spec, PhiOut out, int TK,
+                                             const Blk blk)
 {
     extern __shared__ unsigned char smem_raw[];
     const int L = g.L, M = g.M, H = g.H, ls = L + 1;
@@ -1903,17 +1913,18 @@ __device__ __forceinline__ void k_fftx_inv_b(Geo g, PoisArgs pa, const cpx<T> *_
         for (int h = 0; h < 2; ++h) {
             const int k = k0 + 2 * p + h;
             const double val = h == 0 ? (double)z.x : (double)z.y;
-            phi[hix(g, i, J, k)] = val;
-            if (J == 1) phi[hix(g, i, 0, k)] = val;
-            if (J == M) phi[hix(g, i, M + 1, k)] = val;
+            double *o = out.phi + (size_t)k * out.pitch + i;
+            o[(size_t)(J - out.row0) * L] = val;
+            if (out.row0 == 0 && J == 1) o[0] = val;
+            if (out.row0 == 0 && J == M) o[(size_t)(M + 1) * L] = val;
         }
     }
 }
 template <typename T>
-__global__ __launch_bounds__(256, 4) void k_fftx_inv(Geo g, PoisArgs pa, const cpx<T> *__restrict__ spec,
-                                                  double *__restrict__ phi, int TK)
+__global__ __launch_bounds__(256, 4) void k_fftx_inv(Geo g, PoisArgs pa, const cpx<T> *__restrict__ spec, PhiOut out,
+                                                     int TK)
 {
-    k_fftx_inv_b<T>(g, pa, spec, phi, TK, own_blk());
+    k_fftx_inv_b<T>(g, pa, spec, out, TK, own_blk());
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2007,8 +2018,8 @@ __global__ __launch_bounds__(64) void k_divg_fftx_r(Geo g, const cpx<T> *__restr
 }
 
 // x inverse: Hermitian extension of the plane pair of each line, complex inverse transform,
-// real parts -> phi with the Neumann ghost rows (BC_WALL.f90:369-386).
-template <typename T, int L>
+// real parts to the solution rows (CELLS: of a cell field, else of the halo field; PhiOut).
+template <typename T, int L, bool CELLS>
 __global__ __launch_bounds__(64) void k_fftx_inv_r(Geo g, const cpx<T> *__restrict__ tw,
                                                    const cpx<T> *__restrict__ spec, double *__restrict__ phi)
 {
@@ -2036,18 +2047,139 @@ __global__ __launch_bounds__(64) void k_fftx_inv_r(Geo g, const cpx<T> *__restri
         for (int r = 0; r < G::R0; ++r) x[b * G::R0 + r] = line[chs::rpad<G::PS>(t + b * G::TL + r * (L / G::R0))];
     chs::wave_lds_sync();
     // the block's planes k0 .. k0+TK-1 from one wave-uniform base: a lane's offset is 32-bit
-    const auto pb = uniform(phi + (size_t)k0 * (M + 2) * L);
-    const unsigned pl = (unsigned)(2 * li) * (unsigned)((M + 2) * L), ps = (unsigned)((M + 2) * L);
+    constexpr int G2 = CELLS ? 0 : 2;   // ghost rows of a plane
+    const auto pb = uniform(phi + (size_t)k0 * (M + G2) * L);
+    const unsigned pl = (unsigned)(2 * li) * (unsigned)((M + G2) * L), ps = (unsigned)((M + G2) * L);
     chs::rfft_line<T, L>(x, line, t, tw, +1, [&](int i, const cpx<T> &z) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const unsigned o = pl + h * ps + (unsigned)i;
             const double val = h == 0 ? (double)z.x : (double)z.y;
-            pb[o + (unsigned)(J * L)] = val;
-            if (J == 1) pb[o] = val;
-            if (J == M) pb[o + (unsigned)((M + 1) * L)] = val;
+            pb[o + (unsigned)((CELLS ? J - 1 : J) * L)] = val;
+            if (!CELLS && J == 1) pb[o] = val;
+            if (!CELLS && J == M) pb[o + (unsigned)((M + 1) * L)] = val;
         }
     });
+}
+
+// ---------------------------------------------------------------------------------------
+// Mixed-radix register passes (chs_fftg.h): the three transform kernels for the lengths without
+// a register plan (factors 3 and 5) and for whatever the register plans serve worse (the rule is
+// poisson_launch's).  Same inputs, outputs, scaling and separation as the kernels above.
+
+// z: NLB contiguous lines [J][kx][:] per block, in place.  Bound by memory: 13 us for the 22 MB in
+// and out at 150x97x120 (N = 120 = 10 x 12), where the LDS transform's three passes with per-element
+// index divisions took 20 us.
+template <typename T, int SIGN>
+__global__ __launch_bounds__(256, 4) void k_fftz_g(Geo g, chs::GPlan P, const cpx<T> *__restrict__ tw,
+                                                   cpx<T> *__restrict__ spec, int NLB)
+{
+    extern __shared__ unsigned char smem_raw[];
+    const int ln = threadIdx.x / P.tpl, j = threadIdx.x - ln * P.tpl;
+    const int l = blockIdx.x * NLB + ln;
+    const bool act = ln < NLB && l < g.M * g.H;
+    cpx<T> *base = spec + (size_t)l * g.N;
+    cpx<T> *line = reinterpret_cast<cpx<T> *>(smem_raw) + (act ? ln : 0) * P.ls;
+    chs::gfft_lines<T, SIGN, false, false>(P, line, j, act, tw, [&](int i) { return base[i]; },
+                                           [&](int k, const cpx<T> &x) { base[k] = x; });
+}
+
+// x forward: block = row J and TK consecutive z-planes (a plane pair per line; planes past N - 1
+// of the last block have no line).  TK = 16 or 8 gives spec runs of 256 or 128 bytes per kx; a
+// block's lines take 20 to 37 KB of LDS and its threads at most 128 VGPRs, so four blocks share a
+// CU.  512x192x512: 348 us (4.6 TB/s) against 562 of the register plan's 32-byte runs.
+template <typename T>
+__global__ __launch_bounds__(256, 4) void k_divg_fftx_g(Geo g, chs::GPlan P, const cpx<T> *__restrict__ tw,
+                                                        const double *__restrict__ dv, double talp,
+                                                        const double *__restrict__ q, double *__restrict__ div,
+                                                        cpx<T> *__restrict__ spec, const double *__restrict__ src,
+                                                        int TK, int nxcd)
+{
+    extern __shared__ unsigned char smem_raw[];
+    cpx<T> *lds = reinterpret_cast<cpx<T> *>(smem_raw);
+    const int L = g.L, N = g.N;
+    // rows J and J+1 (whose v this block also reads) on one XCD, so the re-read hits its L2
+    const int tile = __builtin_amdgcn_readfirstlane(xcd_tile(nxcd, own_blk()));
+    const int J = tile % gridDim.x + 1, k0 = (tile / gridDim.x) * TK;
+    const int ln = threadIdx.x / P.tpl, j = threadIdx.x - ln * P.tpl, ka = k0 + 2 * ln;
+    const bool act = ln < TK / 2 && ka < N;
+    const size_t hs = (size_t)N * (g.M + 2) * L, ps = (size_t)(g.M + 2) * L;
+    const int kc = act ? ka : 0;
+    const double *u = q + kc * ps + (size_t)J * L, *v = u + hs, *w = v + hs;
+    const double *w2 = q + 2 * hs + (size_t)(kc + 2 >= N ? 0 : kc + 2) * ps + (size_t)J * L;
+    const double dyf = g.dyfi[J - 1];
+    const double coe0 = dv ? 1.0 / (dv[0] * talp) : 1.0;   // 1 / (alpha DT) (DIVG_tg)
+    const size_t c0 = cix(g, 0, J, kc), c1 = c0 + (size_t)g.M * L;
+    cpx<T> *line = lds + (act ? ln : 0) * P.ls;
+    chs::gfft_lines<T, -1, false, true>(
+        P, line, j, act, tw,
+        [&](int i) -> cpx<T> {
+            if (src) return {(T)src[c0 + i], (T)src[c1 + i]};
+            const int ip = (i == L - 1) ? 0 : i + 1;
+            const double wm = w[ps + i];
+            const double d0 = divg_cell(u[ip], u[i], v[L + i], v[i], wm, w[i], g.dxi, dyf, g.dzi) * coe0;
+            const double d1 = divg_cell(u[ps + ip], u[ps + i], v[ps + L + i], v[ps + i], w2[i], wm, g.dxi, dyf,
+                                        g.dzi) * coe0;
+            if (div) {
+                div[c0 + i] = d0;
+                div[c1 + i] = d1;
+            }
+            return {(T)d0, (T)d1};
+        },
+        [](int, const cpx<T> &) {});
+    // separate the two real transforms, scale by 1/(L N), write spec[J][kx][k0 .. k0+TK-1]
+    const T scale = T(0.5 / ((double)L * (double)N));
+    const int lz = threadIdx.x & (TK - 1), sh = 31 - __builtin_clz(TK), nk = min(TK, N - k0);
+    const cpx<T> *zl = lds + (lz >> 1) * P.ls;
+    if (lz < nk)
+        for (int kx = threadIdx.x >> sh; kx < g.H; kx += blockDim.x >> sh) {
+            const int kc2 = kx == 0 ? 0 : L - kx;
+            const cpx<T> Z = zl[kx + (kx >> P.ps)], Zc = zl[kc2 + (kc2 >> P.ps)];
+            cpx<T> o;
+            if ((lz & 1) == 0) o = {(Z.x + Zc.x) * scale, (Z.y - Zc.y) * scale};
+            else o = {(Z.y + Zc.y) * scale, (Zc.x - Z.x) * scale};
+            spec[six(g, J, kx, k0 + lz)] = o;
+        }
+}
+
+// x inverse: Hermitian extension of the plane pair of each line, complex inverse transform,
+// real parts to the solution rows (PhiOut).
+template <typename T>
+__global__ __launch_bounds__(256, 4) void k_fftx_inv_g(Geo g, chs::GPlan P, const cpx<T> *__restrict__ tw,
+                                                       const cpx<T> *__restrict__ spec, PhiOut out, int TK)
+{
+    extern __shared__ unsigned char smem_raw[];
+    cpx<T> *lds = reinterpret_cast<cpx<T> *>(smem_raw);
+    const int L = g.L, N = g.N, M = g.M, J = blockIdx.x + 1, k0 = blockIdx.y * TK;
+    {
+        const int np = TK / 2, sh = 31 - __builtin_clz(np), p = threadIdx.x & (np - 1);
+        cpx<T> *zl = lds + p * P.ls;
+        if (k0 + 2 * p < N)
+            for (int kx = threadIdx.x >> sh; kx < g.H; kx += blockDim.x >> sh) {
+                cpx<T> A = spec[six(g, J, kx, k0 + 2 * p)], B = spec[six(g, J, kx, k0 + 2 * p + 1)];
+                const int kc2 = L - kx;
+                if (kx == 0 || kx == L / 2) { A.y = T(0); B.y = T(0); }
+                zl[kx + (kx >> P.ps)] = {A.x - B.y, A.y + B.x};
+                if (kx > 0 && kx < L / 2) zl[kc2 + (kc2 >> P.ps)] = {A.x + B.y, B.x - A.y};
+            }
+    }
+    __syncthreads();
+    const int ln = threadIdx.x / P.tpl, j = threadIdx.x - ln * P.tpl, ka = k0 + 2 * ln;
+    const bool act = ln < TK / 2 && ka < N;
+    cpx<T> *line = lds + (act ? ln : 0) * P.ls;
+    double *pa = out.phi + (size_t)(act ? ka : 0) * out.pitch, *pb = pa + out.pitch;
+    const size_t o = (size_t)(J - out.row0) * L;
+    chs::gfft_lines<T, +1, true, false>(
+        P, line, j, act, tw, [](int) { return cpx<T>{}; },
+        [&](int i, const cpx<T> &z) {
+            const double va = (double)z.x, vb = (double)z.y;
+            pa[o + i] = va;
+            pb[o + i] = vb;
+            if (out.row0 == 0) {
+                if (J == 1) { pa[i] = va; pb[i] = vb; }
+                if (J == M) { pa[o + L + i] = va; pb[o + L + i] = vb; }
+            }
+        });
 }
 
 // Projection of a substep: VELOUPDT_tg (VELO_CORRECTION.f90:31-71), PRCALC_tg
@@ -2361,7 +2493,7 @@ __global__ __launch_bounds__(256) void k_poisson_resid(Geo g, const double *__re
     if (t == 0) part[((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = red[0];
 }
 
-// acc (cells) = [acc +] phi interior rows (halo field)
+// acc (cells) = [acc +] phi interior rows (halo field) [- shift]
 __global__ __launch_bounds__(256) void k_phi_accum(Geo g, const double *__restrict__ phi, double *__restrict__ acc,
                                                    int add, const double *__restrict__ shift)
 {
@@ -2782,11 +2914,11 @@ template <typename T> struct KFftxInv {
         Geo g;
         PoisArgs pa;
         const cpx<T> *spec;
-        double *phi;
+        PhiOut out;
         int TK;
     };
     static constexpr int NT = 256, MINW = 4;
-    static __device__ __forceinline__ void run(const Args &a, Blk blk) { k_fftx_inv_b<T>(a.g, a.pa, a.spec, a.phi, a.TK, blk); }
+    static __device__ __forceinline__ void run(const Args &a, Blk blk) { k_fftx_inv_b<T>(a.g, a.pa, a.spec, a.out, a.TK, blk); }
 };
 struct UpdArgs {
     Geo g;
@@ -2879,6 +3011,8 @@ struct chs_ctx {
     double *mean_part = nullptr, *mean_host = nullptr;   // chs_mean_zx_tg: tile sums, pinned result
     void *twx = nullptr, *twz = nullptr;
     void *rtwx = nullptr, *rtwz = nullptr;   // register-FFT pass twiddles (chs_fftr.h), if planned
+    chs::GPlan gx{}, gxi{}, gz{};            // mixed-radix plans: x forward, x inverse, z (chs_fftg.h)
+    void *gtwx = nullptr, *gtwxi = nullptr, *gtwz = nullptr;   // their twiddles (null: not served)
     chs::FftPlan px, pz;
     CnTab cn[4];
     // launch shapes (chs_set_tuning); 0 = derived from the mesh
@@ -3178,15 +3312,17 @@ int upload_twiddles(chs_ctx *c, int n, void **dst)
     return 0;
 }
 
-template <typename T>
-int upload_rtw(chs_ctx *c, int n, void **dst)
+template <typename V>
+int upload_vec(chs_ctx *c, const std::vector<V> &h, void **dst)
 {
-    const std::vector<cpx<T>> h = chs::rplan_twiddles<T>(n);
-    HIPCHK(c, hipMalloc(dst, sizeof(cpx<T>) * h.size()));
-    HIPCHK(c, hipMemcpyAsync(*dst, h.data(), sizeof(cpx<T>) * h.size(), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMalloc(dst, sizeof(V) * h.size()));
+    HIPCHK(c, hipMemcpyAsync(*dst, h.data(), sizeof(V) * h.size(), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return 0;
 }
+
+template <typename T>
+int upload_rtw(chs_ctx *c, int n, void **dst) { return upload_vec(c, chs::rplan_twiddles<T>(n), dst); }
 
 // z-planes per x-transform block: TK x-lines = TK/2 complex lines, (TK/2)*L <= 2048 complex
 // values (the in-place FFT's register budget), TK a power of two dividing N, at most 16
@@ -3242,15 +3378,40 @@ void divg_fftx_r(int L, dim3 grid, hipStream_t st, const Geo &g, const cpx<T> *t
     }
 }
 template <typename T>
-void fftx_inv_r(int L, dim3 grid, hipStream_t st, const Geo &g, const cpx<T> *tw, const cpx<T> *spec, double *phi)
+void fftx_inv_r(int L, dim3 grid, hipStream_t st, const Geo &g, const cpx<T> *tw, const cpx<T> *spec, PhiOut out)
 {
     switch (L) {
-#define X(n) case n: hipLaunchKernelGGL((k_fftx_inv_r<T, n>), grid, dim3(64), 0, st, g, tw, spec, phi); break;
+#define X(n) \
+    case n: \
+        if (out.row0) hipLaunchKernelGGL((k_fftx_inv_r<T, n, sizeof(T) == 8>), grid, dim3(64), 0, st, g, tw, spec, out.phi); \
+        else hipLaunchKernelGGL((k_fftx_inv_r<T, n, false>), grid, dim3(64), 0, st, g, tw, spec, out.phi); \
+        break;
         CHS_RCASES(X)
 #undef X
     }
 }
 #undef CHS_RCASES
+
+// Blocks of the mixed-radix transforms: at most 256 threads and 40 KB of LDS (four blocks of 4
+// wavefronts on a CU), and fewer lines per block on meshes that would otherwise leave fewer
+// than two blocks per CU.  x: TK planes (two per line); z: lines.
+int gx_planes(const chs::GPlan &P, size_t cs, int M, int N)
+{
+    int tk = 16;
+    while (tk > 2 && ((tk / 2) * P.tpl > 256 || (tk / 2) * P.ls * cs > 40960 ||
+                      (tk > 4 && (long long)M * ((N + tk - 1) / tk) < 512)))
+        tk >>= 1;
+    return tk;
+}
+int gz_lines(const chs::GPlan &P, size_t cs, int lines)
+{
+    int nl = std::max(1, std::min(256 / P.tpl, (int)(40960 / (P.ls * cs))));
+    while (nl > 1 && nl * P.tpl > 64 && (lines + nl - 1) / nl < 512) nl = (nl + 1) / 2;
+    return nl;
+}
+int block_threads(int n) { return (n + 63) / 64 * 64; }
+
+PhiOut halo_phi(const chs_ctx *c) { return {c->phi, (size_t)(c->M + 2) * c->L, 0}; }
 
 // Rows per chunk of k_ytdma_chunk (4, 8 or 16; at most 16 chunks, so M <= 256 — longer
 // chunks exceed the 128 registers a 1024-thread block allows): the tuning value if it fits;
@@ -3271,16 +3432,37 @@ int ytdma_chunk_rows(int want, int M, int lines)
 template <typename T>
 // dv: device DT for the divergence scaling 1 / (talp DT) of a substep (null: a given RHS, src).
 // The RHS is the divergence of the velocity at vel (c->q when null), stored into div (c->div
-// when null; not stored when div_out is false), or the cell field src.
+// when null; not stored when div_out is false), or the cell field src; the solution goes to `to`
+// (c->phi when null).
 void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src, int gauge = 0,
-                    const double *vel = nullptr, bool div_out = true)
+                    const double *vel = nullptr, bool div_out = true, const PhiOut *to = nullptr)
 {
+    const PhiOut out = to ? *to : halo_phi(c);
     const double *qv = vel ? vel : c->q;
     double *dvo = div_out ? c->div : nullptr;
     const Geo &g = c->geo;
     const int L = c->L, M = c->M, N = c->N, H = c->H;
-    const bool rx = c->tune.fft_reg && c->rtwx, rz = c->tune.fft_reg && c->rtwz;
-    const int TKR = 2 * (rx ? chs::rplan_lpw(L) : 1), LPZ = rz ? chs::rplan_lpw(N) : 1;
+    // Transforms (us, one launch; LDS radix 2-5 / register plan / mixed radix):
+    //  z     register plan where N has one (256x192x256: 78 / 34 / 39), else mixed radix
+    //        (N = 120: 20 / - / 13);
+    //  x     register plan where L has one, except where mixed radix is faster: L >= 512, whose plan
+    //        holds one line, so two planes or 32-byte runs of the spectrum, per wavefront
+    //        (512x192x512 forward 520 / 562 / 348, inverse 340 / 270 / 221; the FP32 inverse 188 /
+    //        164 / 182 keeps the plan), and the FP64 forward transform with the divergence of
+    //        L = 128 (128x96x128: 22.3 / 22.3 / 17.2; of a given field the plan is faster); else mixed
+    //        radix (144x103x180 forward 48 / - / 29, inverse 35 / - / 17).
+    // The LDS transforms remain for lengths with no plan of two or three passes of at most 256
+    // threads a line, for fft_reg = 0 and for the batched ensemble.
+    const bool f64 = sizeof(T) == 8, fr = c->tune.fft_reg != 0, gxok = c->gtwx && c->gtwxi;
+    const bool rx = fr && c->rtwx && !(gxok && (L >= 512 || (f64 && L == 128 && !src)));
+    const bool rxi = fr && c->rtwx && !(gxok && f64 && L >= 512);
+    const bool rz = fr && c->rtwz;
+    const bool mx = fr && !rx && gxok, mxi = fr && !rxi && gxok, mz = fr && !rz && c->gtwz;
+    const int TKR = 2 * (c->rtwx ? chs::rplan_lpw(L) : 1), LPZ = rz ? chs::rplan_lpw(N) : 1;
+    const int TKG = gxok ? gx_planes(c->gx, sizeof(cpx<T>), M, N) : 2;
+    const dim3 gxg(M, (N + TKG - 1) / TKG);
+    const int NLG = mz ? gz_lines(c->gz, sizeof(cpx<T>), M * H) : 1;
+    const dim3 gzg((M * H + NLG - 1) / NLG);
     PoisArgs pa{c->px, c->pz, c->twx, c->twz};
     const int TK = c->tune.fftx_tk > 0 ? c->tune.fftx_tk : tk_for(L, N);
     const int NL = c->tune.fftz_nl > 0 ? c->tune.fftz_nl : nlz_for(N);
@@ -3292,6 +3474,10 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
         if (rx)
             divg_fftx_r<T>(L, dim3(M, N / TKR), c->stream, g, (const cpx<T> *)c->rtwx, dv, talp, qv, dvo, spec, src,
                            c->tune.divg_nxcd);
+        else if (mx)
+            hipLaunchKernelGGL(k_divg_fftx_g<T>, gxg, dim3(block_threads(TKG / 2 * c->gx.tpl)),
+                               sizeof(cpx<T>) * (TKG / 2) * c->gx.ls, c->stream, g, c->gx, (const cpx<T> *)c->gtwx, dv,
+                               talp, qv, dvo, spec, src, TKG, c->tune.divg_nxcd);
         else
             hipLaunchKernelGGL(k_divg_fftx<T>, dim3(M, N / TK), dim3(256), shx, c->stream, g, pa, dv, talp, qv, dvo,
                                spec, TK, src);
@@ -3300,6 +3486,9 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
         EvScope ev(c, "fftz_fwd");
         if (rz)
             fftz_r<T>(N, dim3((M * H + LPZ - 1) / LPZ), c->stream, g, (const cpx<T> *)c->rtwz, spec, -1);
+        else if (mz)
+            hipLaunchKernelGGL((k_fftz_g<T, -1>), gzg, dim3(block_threads(NLG * c->gz.tpl)),
+                               sizeof(cpx<T>) * NLG * c->gz.ls, c->stream, g, c->gz, (const cpx<T> *)c->gtwz, spec, NLG);
         else
             hipLaunchKernelGGL(k_fftz<T>, dim3((M * H + NL - 1) / NL), dim3(256), shz, c->stream, g, pa, spec, NL, -1);
     }
@@ -3326,16 +3515,23 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
         EvScope ev(c, "fftz_inv");
         if (rz)
             fftz_r<T>(N, dim3((M * H + LPZ - 1) / LPZ), c->stream, g, (const cpx<T> *)c->rtwz, spec, +1);
+        else if (mz)
+            hipLaunchKernelGGL((k_fftz_g<T, +1>), gzg, dim3(block_threads(NLG * c->gz.tpl)),
+                               sizeof(cpx<T>) * NLG * c->gz.ls, c->stream, g, c->gz, (const cpx<T> *)c->gtwz, spec, NLG);
         else
             hipLaunchKernelGGL(k_fftz<T>, dim3((M * H + NL - 1) / NL), dim3(256), shz, c->stream, g, pa, spec, NL, +1);
     }
     {
         EvScope ev(c, "fftx_inv");
-        if (rx)
-            fftx_inv_r<T>(L, dim3(M, N / TKR), c->stream, g, (const cpx<T> *)c->rtwx, (const cpx<T> *)spec, c->phi);
+        if (rxi)
+            fftx_inv_r<T>(L, dim3(M, N / TKR), c->stream, g, (const cpx<T> *)c->rtwx, (const cpx<T> *)spec, out);
+        else if (mxi)
+            hipLaunchKernelGGL(k_fftx_inv_g<T>, gxg, dim3(block_threads(TKG / 2 * c->gxi.tpl)),
+                               sizeof(cpx<T>) * (TKG / 2) * c->gxi.ls, c->stream, g, c->gxi, (const cpx<T> *)c->gtwxi,
+                               (const cpx<T> *)spec, out, TKG);
         else
             hipLaunchKernelGGL(k_fftx_inv<T>, dim3(M, N / TK), dim3(256), shx, c->stream, g, pa,
-                               (const cpx<T> *)spec, c->phi, TK);
+                               (const cpx<T> *)spec, out, TK);
     }
 }
 
@@ -3589,8 +3785,13 @@ int poisson_device_impl(chs_ctx *c, const double *rhs, double *phi, int nref, do
     const dim3 blk(64, 4), grd((c->L + 63) / 64, (c->M + 3) / 4, c->N);
     const int npart = grd.x * grd.y * grd.z;
     const double *acph = c->cf_acph;
-    poisson_launch<T>(c, nullptr, 1.0, rhs);
-    hipLaunchKernelGGL(k_phi_accum, grd, blk, 0, c->stream, g, c->phi, phi, 0, (const double *)nullptr);
+    if constexpr (sizeof(T) == 8) {   // the inverse transform stores the cells itself
+        const PhiOut cells = {phi, (size_t)c->M * c->L, 1};
+        poisson_launch<T>(c, nullptr, 1.0, rhs, 0, nullptr, true, &cells);
+    } else {   // FP32: one rounding of the inverse transform for every caller
+        poisson_launch<T>(c, nullptr, 1.0, rhs);
+        hipLaunchKernelGGL(k_phi_accum, grd, blk, 0, c->stream, g, c->phi, phi, 0, (const double *)nullptr);
+    }
     for (int r = 0; r < nref; ++r) {
         hipLaunchKernelGGL(k_poisson_resid, grd, blk, 0, c->stream, g, c->d_amph, acph, c->d_apph, rhs, phi,
                            c->div, c->partial);
@@ -3895,6 +4096,18 @@ static int create_impl(const chs_coeffs *cf, int mode, hipStream_t shared, chs_c
     }
     int e = (mode == CHS_MIXED) ? upload_twiddles<float>(c, L, &c->twx) : upload_twiddles<double>(c, L, &c->twx);
     if (!e) e = (mode == CHS_MIXED) ? upload_twiddles<float>(c, N, &c->twz) : upload_twiddles<double>(c, N, &c->twz);
+    // mixed-radix plans: lines of at most 256 threads (k_fftz_g's block)
+    c->gx = chs::gplan(L, false);
+    c->gxi = chs::gplan(L, true);
+    c->gz = chs::gplan(N, false);
+    auto gtw = [&](const chs::GPlan &P, void **dst) {
+        if (e || P.np < 2 || P.np > 3 || P.tpl > 256) return;
+        e = (mode == CHS_MIXED) ? upload_vec(c, chs::gplan_twiddles<float>(P), dst)
+                                : upload_vec(c, chs::gplan_twiddles<double>(P), dst);
+    };
+    gtw(c->gx, &c->gtwx);
+    gtw(c->gxi, &c->gtwxi);
+    gtw(c->gz, &c->gtwz);
     // register FFTs: x needs a plan for L and N divisible by the plane pairs of one wavefront
     int rad[8];
     if (!e && chs::rplan_radices(L, rad) && N % (2 * chs::rplan_lpw(L)) == 0)
@@ -3912,7 +4125,7 @@ void chs_destroy(chs_ctx *c)
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void *ptrs[] = {c->cf, c->q, c->qs, c->pr, c->phi, c->div, c->h0, c->rhs, c->rhs2, c->spec, c->pp,
-                    c->pp32, c->pp00, c->partial, c->scal, c->twx, c->twz, c->rtwx, c->rtwz, c->cn_stamp, c->mean_part};
+                    c->pp32, c->pp00, c->partial, c->scal, c->twx, c->twz, c->rtwx, c->rtwz, c->gtwx, c->gtwxi, c->gtwz, c->cn_stamp, c->mean_part};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->mean_host) (void)hipHostFree(c->mean_host);
@@ -4620,7 +4833,7 @@ int ens_make_launches(chs_ens *e, const double *dt, const double *cvisc, EnsLaun
             Pmax = std::max(Pmax, P);
             ayt.push_back({g, c->d_amph, c->d_apph, c->pp, mixed ? c->pp32 : (const float *)nullptr, spec, P, C});
             gyt.push_back(dim3((H * N + 63) / 64));
-            afxi.push_back({g, pa, (const cpx<W> *)spec, c->phi, TK});
+            afxi.push_back({g, pa, (const cpx<W> *)spec, halo_phi(c), TK});
             const dim3 gu((L + 63) / 64, (M + 3) / 4, (N + KU - 1) / KU);
             aupd.push_back({g, s, c->phi, c->qs, c->q, c->pr, KU, c->partial});
             gupd.push_back(gu);

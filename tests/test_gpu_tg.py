@@ -376,3 +376,33 @@ def test_config1_100_steps_match_oracle(pkg):
     assert worst["p"] < 1e-10, worst
     assert div < 1e-12
     ch.close()
+
+
+# Mixed-radix transforms (chs_fftg.h): two- and three-pass plans in x and z, plane blocks cut short
+# (N = 18, 50, 90), lines of 256 threads, FP64 plans that replace the register ones (128, 512), and
+# a length with no plan of three passes (1250, LDS transforms).
+MIXED_RADIX_MESHES = [(18, 5, 18), (150, 6, 120), (162, 4, 250), (200, 5, 50), (128, 7, 90), (512, 5, 30),
+                      (30, 4, 2048), (2048, 4, 6), (1250, 4, 20), (54, 9, 486)]
+
+
+@pytest.mark.parametrize("L,M,N", MIXED_RADIX_MESHES)
+def test_mixed_radix_poisson_matches_oracle_and_device_output(pkg, L, M, N):
+    """The solve against the oracle (bounds as test_poisson_matches_oracle), and the device entry
+    point's cell output equal to the host one's, which goes through the halo field."""
+    print(f"mixed-radix poisson {L}x{M}x{N}", flush=True)
+    mesh = setup.Mesh(L, M, N, STR2=1.9)
+    r = np.random.default_rng(L + N).standard_normal((N, M, L))
+    w = (1.0 / mesh.DYFI)[None, :, None]
+    r -= np.sum(r * w) / (np.sum(w) * L * N)
+    ref = oracle.OracleTG(mesh, 2800.0).poisson(r)
+    for mode, tol in ((pkg.PLAIN_FP64, 1e-10), (pkg.MIXED, 1e-5)):
+        ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=1.9), mode)
+        phi = ch.poisson(r)
+        assert rel(phi, ref) < tol, (mode, rel(phi, ref))
+        d_r, d_p = pkg.DeviceArray.from_host(r), pkg.DeviceArray(r.shape)
+        ch.poisson_device(d_r.ptr, d_p.ptr, 0, False)
+        ch.sync()
+        assert np.array_equal(d_p.to_host(), phi)
+        for d in (d_r, d_p):
+            d.free()
+        ch.close()
