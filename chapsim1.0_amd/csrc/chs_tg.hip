@@ -1868,6 +1868,124 @@ __global__ __launch_bounds__(1024) void k_ytdma_chunk(Geo g, const double *__res
     k_ytdma_chunk_b<T, C>(g, amph, apph, pp, pp32, pp00, spec, int(blockDim.y), own_blk());
 }
 
+// k_ytdma_wide: k_ytdma_chunk with a wavefront's lanes split between 16 lines (256-byte runs of a
+// spectrum row) and four chunks, so that a block of at most 1024 threads covers 64 chunks of C
+// rows: M <= 64 C, where k_ytdma_chunk ends at 16 chunks of 16.  The shorter chunks leave registers
+// for two to four blocks on a CU, whose loads (all of a chunk's rows at once) cover each other's
+// sweeps: 256x192x256 70 -> 48 us (5.3 TB/s); 512x384x512 886 -> 424 us (4.7 TB/s), which one
+// thread per line spent on reading every row twice in a serial sweep.
+template <typename T, int C>
+__global__ __launch_bounds__(1024, 4) void k_ytdma_wide(Geo g, const double *__restrict__ amph,
+                                                        const double *__restrict__ apph,
+                                                        const double *__restrict__ pp,
+                                                        const float *__restrict__ pp32,
+                                                        const double *__restrict__ pp00, cpx<T> *__restrict__ spec)
+{
+    constexpr int LN = 16;
+    extern __shared__ unsigned char smem_raw[];
+    const int M = g.M, HN = g.H * g.N, P = blockDim.x / LN;
+    double *am = reinterpret_cast<double *>(smem_raw), *ap = am + M;
+    double *xr = ap + M, *xi = xr + P * LN, *xl = xi + P * LN;
+    for (int t = threadIdx.x; t < M; t += blockDim.x) {
+        am[t] = t == 0 ? 0.0 : amph[t];
+        ap[t] = apph[t];
+    }
+    const int lane = threadIdx.x & (LN - 1), q = threadIdx.x / LN;
+    const int t = blockIdx.x * LN + lane;
+    const bool act = t < HN;
+    const int tt = act ? t : HN - 1;   // lanes past the last line solve a copy of it, unstored
+    const int kx = tt / g.N, kz = tt - kx * g.N;
+    const bool zero = kx == 0 && kz == 0;
+    const bool pin = zero && pp00;      // TRID0: x_M = 0, unmodified pivots pp00[J-1]
+    const bool z99 = zero && !pp00;     // FFT99: RHS(1) = 0, row 1 decoupled
+    // FP32 pivots (mixed form) for all but the lowest modes, as k_ytdma
+    const bool low = !pp32 || (kx <= 1 && (kz <= 1 || kz == g.N - 1));
+    const int j0 = q * C, n = max(0, min(C, M - j0));   // rows j0 .. j0 + n - 1, 0-based
+    cpx<T> *sp = spec + (size_t)j0 * HN + tt;
+    const size_t po = (size_t)j0 * HN + tt;
+    double rr[C], ri[C], pv[C];
+#pragma unroll
+    for (int u = 0; u < C; ++u)
+        if (u < n) {
+            const cpx<T> v = sp[(size_t)u * HN];
+            rr[u] = (double)v.x;
+            ri[u] = (double)v.y;
+            pv[u] = pin ? pp00[j0 + u] : (low ? pp[po + (size_t)u * HN] : (double)pp32[po + (size_t)u * HN]);
+        }
+    __syncthreads();   // am, ap
+    double gr = 0.0, gi = 0.0, lam = 1.0;
+#pragma unroll
+    for (int u = 0; u < C; ++u)
+        if (u < n) {
+            const double a = am[j0 + u];
+            const bool r0 = z99 && j0 + u == 0;
+            gr = ((r0 ? 0.0 : rr[u]) - a * gr) * pv[u];
+            gi = ((r0 ? 0.0 : ri[u]) - a * gi) * pv[u];
+            lam = -(a * pv[u]) * lam;
+            rr[u] = gr;
+            ri[u] = gi;
+        }
+    xr[threadIdx.x] = gr;
+    xi[threadIdx.x] = gi;
+    xl[threadIdx.x] = lam;
+    __syncthreads();
+    double inr = 0.0, ini = 0.0;
+    for (int e = lane; e < (int)threadIdx.x; e += LN) {
+        inr = xr[e] + xl[e] * inr;
+        ini = xi[e] + xl[e] * ini;
+    }
+    lam = 1.0;
+#pragma unroll
+    for (int u = 0; u < C; ++u)
+        if (u < n) {
+            lam = -(am[j0 + u] * pv[u]) * lam;
+            rr[u] += lam * inr;
+            ri[u] += lam * ini;
+        }
+    // backward sweep from x_in = 0
+    double xhr = 0.0, xhi = 0.0, mu = 1.0;
+#pragma unroll
+    for (int u = C - 1; u >= 0; --u)
+        if (u < n) {
+            const int j = j0 + u;
+            const double h = ((z99 && j == 0) ? 0.0 : ap[j]) * pv[u];
+            if (pin && j == M - 1) {
+                xhr = 0.0;
+                xhi = 0.0;
+            } else {
+                xhr = rr[u] - h * xhr;
+                xhi = ri[u] - h * xhi;
+            }
+            mu = -h * mu;
+            rr[u] = xhr;
+            ri[u] = xhi;
+        }
+    __syncthreads();   // every chunk has read the forward end values
+    xr[threadIdx.x] = xhr;
+    xi[threadIdx.x] = xhi;
+    xl[threadIdx.x] = mu;
+    __syncthreads();
+    double xir = 0.0, xii = 0.0;
+    for (int e = (P - 1) * LN + lane; e > (int)threadIdx.x; e -= LN) {
+        xir = xr[e] + xl[e] * xir;
+        xii = xi[e] + xl[e] * xii;
+    }
+    mu = 1.0;
+#pragma unroll
+    for (int u = C - 1; u >= 0; --u)
+        if (u < n) {
+            const int j = j0 + u;
+            mu = -(((z99 && j == 0) ? 0.0 : ap[j]) * pv[u]) * mu;
+            rr[u] += mu * xir;
+            ri[u] += mu * xii;
+        }
+    if (act) {
+#pragma unroll
+        for (int u = 0; u < C; ++u)
+            if (u < n) sp[(size_t)u * HN] = {(T)rr[u], (T)ri[u]};
+    }
+}
+
 // Where an inverse x-transform puts the solution: the halo field [N][M+2][L] with the Neumann
 // ghost rows of BC_WALL_DPH (BC_WALL.f90:369-386) (pitch (M+2) L, row0 = 0), or a cell field
 // [N][M][L] (pitch M L, row0 = 1), which saves the standalone solve a pass that copies the rows.
@@ -3411,6 +3529,17 @@ int gz_lines(const chs::GPlan &P, size_t cs, int lines)
 }
 int block_threads(int n) { return (n + 63) / 64 * 64; }
 
+// Rows per chunk of k_ytdma_wide, 0 where k_ytdma_chunk or k_ytdma runs: automatic (want = -1)
+// only, and M <= 1024 (64 chunks of 16).  k_ytdma_chunk keeps M <= 128 (128x96x128: 15.8 us
+// against 16.4 to 21.5 with 4 to 16 rows) and, up to the 256 rows it covers, fft_reg = 0, whose
+// steps the batched launches reproduce.  us by rows per chunk 8 / 12 / 16, and before:
+// 256x192x256 68 / 48 / 57, 70; 250x300x250 108 / 94 / 122; 512x384x512 425 / 449 / 545, 886.
+int ytdma_wide_rows(int want, int fft_reg, int M)
+{
+    if (want >= 0 || M > 1024 || M <= 128 || (M <= 256 && !fft_reg)) return 0;
+    return M <= 320 || (M > 512 && M <= 768) ? 12 : (M <= 512 ? 8 : 16);
+}
+
 PhiOut halo_phi(const chs_ctx *c) { return {c->phi, (size_t)(c->M + 2) * c->L, 0}; }
 
 // Rows per chunk of k_ytdma_chunk (4, 8 or 16; at most 16 chunks, so M <= 256 — longer
@@ -3496,13 +3625,23 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
         EvScope ev(c, "ytdma");
         const float *p32 = c->mode == CHS_MIXED ? c->pp32 : (const float *)nullptr;
         const double *p00 = gauge ? (const double *)c->pp00 : (const double *)nullptr;
-        const int C = ytdma_chunk_rows(c->tune.ytdma_c, M, H * N);
+        const int CW = ytdma_wide_rows(c->tune.ytdma_c, c->tune.fft_reg, M);
+        const int C = CW ? 0 : ytdma_chunk_rows(c->tune.ytdma_c, M, H * N);
         if (C > 0) {
             const dim3 grid((H * N + 63) / 64), blk(64, (M + C - 1) / C);
             switch (C) {
 #define CHS_YTC(cc) case cc: hipLaunchKernelGGL((k_ytdma_chunk<T, cc>), grid, blk, 0, c->stream, g, c->d_amph, c->d_apph, c->pp, p32, p00, spec); break;
                 CHS_YTC(4) CHS_YTC(8) CHS_YTC(16)
 #undef CHS_YTC
+            }
+        } else if (CW > 0) {
+            const int P = (M + CW - 1) / CW;
+            const dim3 grid((H * N + 15) / 16), blk(16 * ((P + 3) / 4 * 4));
+            const size_t sh = sizeof(double) * (2 * (size_t)M + 3 * blk.x);
+            switch (CW) {
+#define CHS_YTW(cc) case cc: hipLaunchKernelGGL((k_ytdma_wide<T, cc>), grid, blk, sh, c->stream, g, c->d_amph, c->d_apph, c->pp, p32, p00, spec); break;
+                CHS_YTW(8) CHS_YTW(12) CHS_YTW(16)
+#undef CHS_YTW
             }
         } else {
             const int bs = c->tune.ytdma_bs;

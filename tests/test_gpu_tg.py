@@ -406,3 +406,24 @@ def test_mixed_radix_poisson_matches_oracle_and_device_output(pkg, L, M, N):
         for d in (d_r, d_p):
             d.free()
         ch.close()
+
+
+@pytest.mark.parametrize("M", [129, 131, 192, 256, 257, 320, 321, 512, 513, 769, 1024, 1025])
+def test_wide_ytdma_matches_serial_lines(pkg, M):
+    """The y-Thomas with 16-line runs (M > 128; chunks of 8, 12 and 16 rows, the last one short)
+    against one thread per line (ytdma_c = 0), both gauges.  The split sweeps differ from the serial
+    one by rounding only; the (0, 0) mode's Neumann sweep amplifies it by at most the condition
+    M^2 / 4 of that line (1e-16 * 2.6e5 = 3e-11 at M = 1024)."""
+    L, N = 36, 30
+    r = np.random.default_rng(M).standard_normal((N, M, L))
+    co = pkg.channel_setup(L, M, N, STR2=1.9)
+    w = (1.0 / co["dyfi"])[None, :, None]
+    r -= np.sum(r * w) / (np.sum(w) * L * N)
+    for mode, tol in ((pkg.PLAIN_FP64, 1e-10), (pkg.MIXED, 1e-5)):
+        ch = pkg.ChannelTG(co, mode)
+        got = [ch.poisson(r), ch.FISHPACK_POIS3D_SIMPLE(r)]
+        ch.set_tuning(ytdma_c=0)
+        ref = [ch.poisson(r), ch.FISHPACK_POIS3D_SIMPLE(r)]
+        for a, b in zip(got, ref):
+            assert rel(a, b) < tol, (mode, rel(a, b))
+        ch.close()
