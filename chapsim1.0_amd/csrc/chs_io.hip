@@ -1131,31 +1131,40 @@ __device__ __forceinline__ void io_cn_x_jac(const IoDev &d, double dp, double fa
     if (valid) ioh<W>(d)[C * cs + cx(d, e, J, k)] = (W)x;
 }
 
-// MOMFA1_X_io for L = 64 P (P = 1..8): one wavefront per x-line, lane l holding points
+// MOMFA1_X_io for L = n P with n <= 64 lanes: one wavefront per x-line, lane l < n holding points
 // l P .. l P + P - 1; the neighbours across lanes come by cross-lane shuffles, so a line needs
 // no block barrier and a wavefront's loads are all issued together.  Coefficients and sweeps
-// as io_cn_x_jac (rho is the line's own maximum).
-template <int C, int P, typename W, bool FD>
+// as io_cn_x_jac (rho is the line's own maximum).  RG: n < 64, the other lanes carry identity
+// rows (L = 90: 45 lanes of 2 points; 90x71x120: 112 us of one thread per line, whose
+// lanes read 720 bytes apart, -> 21 us for the three).
+template <int C, int P, typename W, bool FD, bool RG>
 __device__ __forceinline__ void io_cn_x_wave(const IoDev &d, double dp, double facoe)
 {
 #pragma clang fp contract(off)
-    const int M = d.M, j0 = C == 1 ? 2 : 1, nj = M - j0 + 1, nl = nj * d.N;
+    const int M = d.M, n = RG ? d.L / P : 64, j0 = C == 1 ? 2 : 1, nj = M - j0 + 1, nl = nj * d.N;
     const int lane = threadIdx.x & 63;
     const int line = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     if (line >= nl) return;   // the whole wavefront
     const int J = j0 + line % nj, k = line / nj;
     const size_t hs = hsz(d), cs = csz(d);
-    const int lm = (lane + 63) & 63, lp = (lane + 1) & 63;
+    const bool own = !RG || lane < n;
+    const int lm = RG ? (lane == 0 ? n - 1 : lane - 1) : (lane + 63) & 63;
+    const int lp = RG ? (lane >= n - 1 ? 0 : lane + 1) : (lane + 1) & 63;
     const double *F0 = (C == 0 ? d.m1 : d.mstg + (C - 1) * hs) + hx(d, lane * P, J, k);
     const double *F1 = d.dstg + C * hs + hx(d, lane * P, J, k);
     W *R = ioh<W>(d) + C * cs + cx(d, lane * P, J, k);
     double f0[P], f1[P], r[P];
 #pragma unroll
     for (int j = 0; j < P; ++j) {
-        f0[j] = F0[j];
-        f1[j] = F1[j];
-        r[j] = R[j];
-        if constexpr (C == 0) r[j] = r[j] - dp;
+        f0[j] = 0.0;
+        f1[j] = 1.0;
+        r[j] = 0.0;
+        if (own) {
+            f0[j] = F0[j];
+            f1[j] = F1[j];
+            r[j] = R[j];
+            if constexpr (C == 0) r[j] = r[j] - dp;
+        }
     }
     const double f0m = __shfl(f0[P - 1], lm), f0p = __shfl(f0[0], lp);
     const double f1m = __shfl(f1[P - 1], lm), f1p = __shfl(f1[0], lp);
@@ -1176,7 +1185,11 @@ __device__ __forceinline__ void io_cn_x_wave(const IoDev &d, double dp, double f
         }
         a[j] = qd<FD>(amu, dm);
         c[j] = qd<FD>(apu, dq);
-        const double b = 1.0 - qd<FD>(amu + apu, f1[j]);
+        double b = 1.0 - qd<FD>(amu + apu, f1[j]);
+        if (!own) {
+            a[j] = c[j] = 0.0;
+            b = 1.0;
+        }
         ib[j] = qd<FD>(1.0, b);
         rho = nanmax(rho, (fabs(a[j]) + fabs(c[j])) * fabs(ib[j]));
     }
@@ -1200,17 +1213,19 @@ __device__ __forceinline__ void io_cn_x_wave(const IoDev &d, double dp, double f
 #pragma unroll
         for (int j = 0; j < P; ++j) x[j] = xn[j];
     }
+    if (own) {
 #pragma unroll
-    for (int j = 0; j < P; ++j) R[j] = (W)x[j];
+        for (int j = 0; j < P; ++j) R[j] = (W)x[j];
+    }
 }
 
-template <int P, typename W, bool FD>
+template <int P, typename W, bool FD, bool RG>
 __global__ __launch_bounds__(256) void k_io_cn_x_wave(IoDev d, const double *__restrict__ dpg_dev, double dpg,
                                                       double facoe)
 {
-    if (blockIdx.y == 0) io_cn_x_wave<0, P, W, FD>(d, dpg_dev ? dpg_dev[0] : dpg, facoe);
-    else if (blockIdx.y == 1) io_cn_x_wave<1, P, W, FD>(d, 0.0, facoe);
-    else io_cn_x_wave<2, P, W, FD>(d, 0.0, facoe);
+    if (blockIdx.y == 0) io_cn_x_wave<0, P, W, FD, RG>(d, dpg_dev ? dpg_dev[0] : dpg, facoe);
+    else if (blockIdx.y == 1) io_cn_x_wave<1, P, W, FD, RG>(d, 0.0, facoe);
+    else io_cn_x_wave<2, P, W, FD, RG>(d, 0.0, facoe);
 }
 
 template <typename W>
@@ -1256,15 +1271,6 @@ __device__ __forceinline__ void io_cn_z_line(const IoDev &d, int l, double facoe
     auto rhs = [&](int k) { return (double)R[cx(d, i, J, k)]; };
     auto out = [&](int k, double x) { R[cx(d, i, J, k)] = (W)x; };
     thomas_cyc(N, coef, rhs, out, Wk, Wk + cs, Wk + 2 * cs, (size_t)nl);
-}
-
-template <typename W>
-__global__ __launch_bounds__(128) void k_io_cn_z(IoDev d, double facoe)
-{
-    const int l = blockIdx.x * 128 + threadIdx.x;
-    if (blockIdx.y == 0) io_cn_z_line<0, W>(d, l, facoe);
-    else if (blockIdx.y == 1) io_cn_z_line<1, W>(d, l, facoe);
-    else io_cn_z_line<2, W>(d, l, facoe);
 }
 
 // MOMFA3_Y_io (MOMFA_io.f90:268-406): y-lines over rows 1..M with zero boundary values, then
@@ -1337,32 +1343,46 @@ __global__ __launch_bounds__(128) void k_io_cn_y(IoDev d, const double *__restri
     else io_cn_y_line<2, W>(d, gs, l, facoe);
 }
 
-// MOMFA2_Z_io with P consecutive z-points per thread (N a multiple of P): a block holds T
-// x-columns of one row J, thread (lt, chunk) at lt + T chunk, so a wave reads runs of T
-// consecutive x; only the chunk edges go through LDS (coefficient neighbours, then the Jacobi
-// sweeps' neighbours).
-template <int C, int P, typename W, bool FD>
-__device__ __forceinline__ void io_cn_z_jac(const IoDev &d, double facoe, double *lds)
+// MOMFA2_Z_io with P consecutive z-points per thread: a block holds T x-columns of one row J,
+// thread (lt, chunk) at lt + T chunk, so a wave reads runs of T consecutive x; only the chunk
+// edges go through LDS (coefficient neighbours, then the Jacobi sweeps' neighbours).  The
+// threads past T NT (the block is whole wavefronts) carry identity rows.  RG: N is not a multiple
+// of P and the last chunk holds the n = N - (NT - 1) P points left (90x71x120, 15 chunks in blocks
+// of 256 threads: 135 us of one thread per line -> 24 us; 54 MB in, 18 MB out).
+template <int C, int P, typename W, bool FD, bool RG>
+__device__ __forceinline__ void io_cn_z_jac(const IoDev &d, double facoe, double *lds, int T)
 {
 #pragma clang fp contract(off)
     const int L = d.L, M = d.M, N = d.N, j0 = C == 1 ? 2 : 1;
-    const int NT = N / P, T = blockDim.x / NT, lt = threadIdx.x % T, tt = threadIdx.x / T;
+    const int NT = (N + P - 1) / P, lt = threadIdx.x % T, tt = threadIdx.x / T;
     const int ng = (L + T - 1) / T;
     const int i = (blockIdx.x % ng) * T + lt, J = j0 + blockIdx.x / ng;
-    const bool valid = i < L && J <= M;
+    const bool valid = i < L && J <= M && tt < NT;
     const size_t hs = hsz(d), cs = csz(d);
     const int S = blockDim.x;
     double *e0 = lds, *e1 = lds + S, *e2 = lds + 2 * S, *e3 = lds + 3 * S;
     unsigned long long *word = reinterpret_cast<unsigned long long *>(lds + 4 * S);
     const int k0 = tt * P;
-    const int sl = ((tt + NT - 1) % NT) * T + lt, sr = ((tt + 1) % NT) * T + lt;   // neighbour chunks
+    const int n = RG ? min(P, N - k0) : P;   // this chunk's points (RG: its last is j = n - 1)
+    const int sl = (tt == 0 ? NT - 1 : min(tt, NT) - 1) * T + lt, sr = (tt >= NT - 1 ? 0 : tt + 1) * T + lt;   // neighbour chunks
+    auto last = [&](const double (&v)[P]) {
+        double x = v[P - 1];
+        if constexpr (RG) {
+#pragma unroll
+            for (int j = 0; j < P - 1; ++j) {
+                x = j == n - 1 ? v[j] : x;
+                asm("" : "+v"(x));   // keeps the selects: as v[n - 1] the array would go to scratch
+            }
+        }
+        return x;
+    };
     double f0[P], f1[P], r[P];
 #pragma unroll
     for (int j = 0; j < P; ++j) {
         f0[j] = 0.0;
         f1[j] = 1.0;
         r[j] = 0.0;
-        if (valid) {
+        if (valid && (!RG || j < n)) {
             const size_t o = hx(d, i, J, k0 + j);
             f0[j] = C == 2 ? d.m1[o] : d.mstg[(C + 1) * hs + o];
             f1[j] = d.dstg[C * hs + o];
@@ -1370,16 +1390,17 @@ __device__ __forceinline__ void io_cn_z_jac(const IoDev &d, double facoe, double
         }
     }
     e0[threadIdx.x] = f0[0];
-    e1[threadIdx.x] = f0[P - 1];
+    e1[threadIdx.x] = last(f0);
     e2[threadIdx.x] = f1[0];
-    e3[threadIdx.x] = f1[P - 1];
+    e3[threadIdx.x] = last(f1);
     __syncthreads();
     const double f0m = e1[sl], f1m = e3[sl], f0p = e0[sr], f1p = e2[sr];
     double a[P], c[P], ib[P], rho = 0.0;
 #pragma unroll
     for (int j = 0; j < P; ++j) {
-        const double vm = j > 0 ? f0[j - 1] : f0m, vp = j < P - 1 ? f0[j + 1] : f0p;
-        const double dm = j > 0 ? f1[j - 1] : f1m, dq = j < P - 1 ? f1[j + 1] : f1p;
+        const bool end = j == P - 1 || (RG && j == n - 1);
+        const double vm = j > 0 ? f0[j - 1] : f0m, vp = end ? f0p : f0[j + 1 < P ? j + 1 : j];
+        const double dm = j > 0 ? f1[j - 1] : f1m, dq = end ? f1p : f1[j + 1 < P ? j + 1 : j];
         double amu, apu;
         if constexpr (C == 2) {
             const double coe1 = facoe * 4.0 / 3.0 * d.dzqi;
@@ -1393,7 +1414,7 @@ __device__ __forceinline__ void io_cn_z_jac(const IoDev &d, double facoe, double
         a[j] = qd<FD>(amu, dm);
         c[j] = qd<FD>(apu, dq);
         double b = 1.0 - qd<FD>(amu + apu, f1[j]);
-        if (!valid) {
+        if (!valid || (RG && j >= n)) {
             a[j] = c[j] = 0.0;
             b = 1.0;
         }
@@ -1414,13 +1435,14 @@ __device__ __forceinline__ void io_cn_z_jac(const IoDev &d, double facoe, double
         // one barrier per sweep
         double *w0 = (it & 1) ? e2 : e0, *w1 = (it & 1) ? e3 : e1;
         w0[threadIdx.x] = x[0];
-        w1[threadIdx.x] = x[P - 1];
+        w1[threadIdx.x] = last(x);
         __syncthreads();
         const double xl = w1[sl], xr = w0[sr];
         double xn[P];
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-            const double xm = j > 0 ? x[j - 1] : xl, xp = j < P - 1 ? x[j + 1] : xr;
+            const bool end = j == P - 1 || (RG && j == n - 1);
+            const double xm = j > 0 ? x[j - 1] : xl, xp = end ? xr : x[j + 1 < P ? j + 1 : j];
             xn[j] = (r[j] - a[j] * xm - c[j] * xp) * ib[j];
         }
 #pragma unroll
@@ -1428,38 +1450,41 @@ __device__ __forceinline__ void io_cn_z_jac(const IoDev &d, double facoe, double
     }
     if (valid) {
 #pragma unroll
-        for (int j = 0; j < P; ++j) ioh<W>(d)[C * cs + cx(d, i, J, k0 + j)] = (W)x[j];
+        for (int j = 0; j < P; ++j)
+            if (!RG || j < n) ioh<W>(d)[C * cs + cx(d, i, J, k0 + j)] = (W)x[j];
     }
 }
 
-template <typename W, bool FD, int P>
-__global__ __launch_bounds__(1024) void k_io_cn_z_jac(IoDev d, double facoe)
+template <typename W, bool FD, int P, bool RG>
+__global__ __launch_bounds__(1024) void k_io_cn_z_jac(IoDev d, double facoe, int T)
 {
     extern __shared__ double lds[];
-    if (blockIdx.y == 0) io_cn_z_jac<0, P, W, FD>(d, facoe, lds);
-    else if (blockIdx.y == 1) io_cn_z_jac<1, P, W, FD>(d, facoe, lds);
-    else io_cn_z_jac<2, P, W, FD>(d, facoe, lds);
+    if (blockIdx.y == 0) io_cn_z_jac<0, P, W, FD, RG>(d, facoe, lds, T);
+    else if (blockIdx.y == 1) io_cn_z_jac<1, P, W, FD, RG>(d, facoe, lds, T);
+    else io_cn_z_jac<2, P, W, FD, RG>(d, facoe, lds, T);
 }
 
 // MOMFA3_Y_io + the G update with P consecutive rows per thread (NT = ceil(M / P) chunks per
 // column, rows past M are identity rows): a block holds T x-columns of one z-plane, thread
-// (lt, chunk) at lt + T chunk; coefficients as io_cn_y_line builds them; writes every row of
-// the new G of its columns.
+// (lt, chunk) at lt + T chunk (threads past T NT, to whole wavefronts, carry identity rows);
+// coefficients as io_cn_y_line builds them; writes every row of the new G of its columns
+// (90x71x120, 9 chunks: 62 us of one thread per line -> 35 us).
 template <int C, int P, typename W, bool FD>
-__device__ __forceinline__ void io_cn_y_jac(const IoDev &d, const double *__restrict__ gs, double facoe, double *lds)
+__device__ __forceinline__ void io_cn_y_jac(const IoDev &d, const double *__restrict__ gs, double facoe, double *lds,
+                                            int T)
 {
 #pragma clang fp contract(off)
     const int L = d.L, M = d.M;
-    const int NT = (M + P - 1) / P, T = blockDim.x / NT, lt = threadIdx.x % T, tt = threadIdx.x / T;
+    const int NT = (M + P - 1) / P, lt = threadIdx.x % T, tt = threadIdx.x / T;
     const int ng = (L + T - 1) / T;
     const int i = (blockIdx.x % ng) * T + lt, k = blockIdx.x / ng;
-    const bool valid = i < L;
+    const bool valid = i < L && tt < NT;
     const size_t hs = hsz(d), cs = csz(d);
     const int S = blockDim.x;
     double *e0 = lds, *e1 = lds + S, *e2 = lds + 2 * S, *e3 = lds + 3 * S;
     unsigned long long *word = reinterpret_cast<unsigned long long *>(lds + 4 * S);
     const int J0 = tt * P + 1;
-    const int sl = tt > 0 ? (tt - 1) * T + lt : -1, sr = tt < NT - 1 ? (tt + 1) * T + lt : -1;
+    const int sl = tt > 0 && tt < NT ? (tt - 1) * T + lt : -1, sr = tt < NT - 1 ? (tt + 1) * T + lt : -1;
     const double *DS = d.dstg + C * hs, *FM = C == 1 ? d.m1 : d.mstg + C * hs;
     double f0[P], f1[P], r[P];
 #pragma unroll
@@ -1573,12 +1598,12 @@ __device__ __forceinline__ void io_cn_y_jac(const IoDev &d, const double *__rest
 }
 
 template <typename W, bool FD, int P>
-__global__ __launch_bounds__(1024) void k_io_cn_y_jac(IoDev d, const double *__restrict__ gs, double facoe)
+__global__ __launch_bounds__(1024) void k_io_cn_y_jac(IoDev d, const double *__restrict__ gs, double facoe, int T)
 {
     extern __shared__ double lds[];
-    if (blockIdx.y == 0) io_cn_y_jac<0, P, W, FD>(d, gs, facoe, lds);
-    else if (blockIdx.y == 1) io_cn_y_jac<1, P, W, FD>(d, gs, facoe, lds);
-    else io_cn_y_jac<2, P, W, FD>(d, gs, facoe, lds);
+    if (blockIdx.y == 0) io_cn_y_jac<0, P, W, FD>(d, gs, facoe, lds, T);
+    else if (blockIdx.y == 1) io_cn_y_jac<1, P, W, FD>(d, gs, facoe, lds, T);
+    else io_cn_y_jac<2, P, W, FD>(d, gs, facoe, lds, T);
 }
 
 // DIVG_io (DIVG.f90:54-137), iWeightedPre = 0: rows 1..M.
@@ -2098,13 +2123,23 @@ void io_momentum_launch(chs_io *m, const double *gs, double tg, double tr, doubl
         // here (each reads Q, the properties and its own increment), so they run side by side.
         const double facoe = 0.5 * ta * dt * d.cvisc;
         const int L = m->L, M = m->M, N = m->N;
-        const int PX = L / 64;   // x-line points per lane of the wavefront-per-line solve
-        if (m->cnx_wave && L % 64 == 0 && (PX == 1 || PX == 2 || PX == 4 || PX == 8)) {
+        // x: one wavefront per line where L is a multiple n P of at most 64 lanes (the fewest points
+        // per lane); else a block per line for powers of two, else a thread per line
+        int PX = 0;
+        if (m->cnx_wave && L <= 640)
+            for (int q : {1, 2, 3, 4, 5, 6, 8, 9, 10})
+                if (PX == 0 && L % q == 0 && L / q <= 64) PX = q;
+        if (PX && !(L < 32 && (L & (L - 1)) == 0)) {
             const dim3 gx((M * N + 3) / 4, 3);
-            if (PX == 1) hipLaunchKernelGGL((k_io_cn_x_wave<1, W, false>), gx, dim3(256), 0, m->stream, d, dpg_dev, dpg, facoe);
-            else if (PX == 2) hipLaunchKernelGGL((k_io_cn_x_wave<2, W, false>), gx, dim3(256), 0, m->stream, d, dpg_dev, dpg, facoe);
-            else if (PX == 4) hipLaunchKernelGGL((k_io_cn_x_wave<4, W, false>), gx, dim3(256), 0, m->stream, d, dpg_dev, dpg, facoe);
-            else hipLaunchKernelGGL((k_io_cn_x_wave<8, W, false>), gx, dim3(256), 0, m->stream, d, dpg_dev, dpg, facoe);
+#define CHS_IOX(q) \
+    case q: \
+        if (L == 64 * q) hipLaunchKernelGGL((k_io_cn_x_wave<q, W, false, false>), gx, dim3(256), 0, m->stream, d, dpg_dev, dpg, facoe); \
+        else hipLaunchKernelGGL((k_io_cn_x_wave<q, W, false, true>), gx, dim3(256), 0, m->stream, d, dpg_dev, dpg, facoe); \
+        break;
+            switch (PX) {
+                CHS_IOX(1) CHS_IOX(2) CHS_IOX(3) CHS_IOX(4) CHS_IOX(5) CHS_IOX(6) CHS_IOX(8) CHS_IOX(9) CHS_IOX(10)
+            }
+#undef CHS_IOX
         } else if ((L & (L - 1)) == 0 && L >= 4 && L <= 512) {
             const int T = L >= 256 ? 1 : 256 / L;   // x-lines per block
             hipLaunchKernelGGL(k_io_cn_x_jac<W>, dim3((M * N + T - 1) / T, 3), dim3(T * L),
@@ -2113,33 +2148,38 @@ void io_momentum_launch(chs_io *m, const double *gs, double tg, double tr, doubl
             hipLaunchKernelGGL(k_io_cn_x<W>, dim3((M * N + 127) / 128, 3), dim3(128), 0, m->stream, d, dpg_dev, dpg,
                                facoe);
         }
-        // line points per thread of the z and y kernels (4 or 8)
+        // z and y: T x-columns by NT chunks of P line points per thread (4 or 8), rounded up to whole
+        // wavefronts; N <= 2048 leaves z at most 512 chunks
         const int Pz = m->cnz_p, Py = m->cny_p;
-        const int NTz = N / Pz;   // z: block = Tz x-columns x NTz chunks, whole waves
-        int Tz = (N % Pz == 0 && NTz >= 2 && NTz <= 1024) ? std::min(m->cnz_cols ? m->cnz_cols : m->cn_cols, 1024 / NTz) : 0;
-        if (Tz > 0) Tz -= Tz % (64 / std::gcd(NTz, 64));
-        if (Tz > 0) {
-            const int ng = (L + Tz - 1) / Tz;
-            const dim3 gz(ng * M, 3), bz(Tz * NTz);
-            const size_t sz = sizeof(double) * (4 * Tz * NTz + 1);
-            if (Pz == 8 && m->cn_fastdiv) hipLaunchKernelGGL((k_io_cn_z_jac<W, true, 8>), gz, bz, sz, m->stream, d, facoe);
-            else if (Pz == 8) hipLaunchKernelGGL((k_io_cn_z_jac<W, false, 8>), gz, bz, sz, m->stream, d, facoe);
-            else if (m->cn_fastdiv) hipLaunchKernelGGL((k_io_cn_z_jac<W, true, 4>), gz, bz, sz, m->stream, d, facoe);
-            else hipLaunchKernelGGL((k_io_cn_z_jac<W, false, 4>), gz, bz, sz, m->stream, d, facoe);
-        } else {
-            hipLaunchKernelGGL(k_io_cn_z<W>, dim3((M * L + 127) / 128, 3), dim3(128), 0, m->stream, d, facoe);
+        {
+            const int NT = (N + Pz - 1) / Pz, T = std::min(m->cnz_cols ? m->cnz_cols : m->cn_cols, 1024 / NT);
+            const int S = (T * NT + 63) / 64 * 64;
+            const dim3 gz((L + T - 1) / T * M, 3), bz(S);
+            const size_t sz = sizeof(double) * (4 * S + 1);
+            const int sel = (m->cn_fastdiv ? 4 : 0) + (Pz == 8 ? 2 : 0) + (N % Pz ? 1 : 0);
+            switch (sel) {
+#define CHS_IOZ(fd, p, rg) hipLaunchKernelGGL((k_io_cn_z_jac<W, fd, p, rg>), gz, bz, sz, m->stream, d, facoe, T); break;
+            case 0: CHS_IOZ(false, 4, false)
+            case 1: CHS_IOZ(false, 4, true)
+            case 2: CHS_IOZ(false, 8, false)
+            case 3: CHS_IOZ(false, 8, true)
+            case 4: CHS_IOZ(true, 4, false)
+            case 5: CHS_IOZ(true, 4, true)
+            case 6: CHS_IOZ(true, 8, false)
+            default: CHS_IOZ(true, 8, true)
+#undef CHS_IOZ
+            }
         }
-        const int NTy = (M + Py - 1) / Py;   // y: block = Ty x-columns x NTy chunks, whole waves
-        int Ty = NTy <= 1024 ? std::min(m->cny_cols ? m->cny_cols : m->cn_cols, 1024 / NTy) : 0;
-        if (Ty > 0) Ty -= Ty % (64 / std::gcd(NTy, 64));
-        if (Ty > 0) {
+        const int NTy = (M + Py - 1) / Py;
+        if (NTy <= 1024) {
+            const int Ty = std::min(m->cny_cols ? m->cny_cols : m->cn_cols, 1024 / NTy), S = (Ty * NTy + 63) / 64 * 64;
             const int ng = (L + Ty - 1) / Ty;
-            const dim3 gy(ng * N, 3), by(Ty * NTy);
-            const size_t sy = sizeof(double) * (4 * Ty * NTy + 1 + 2 * (M + 2));
-            if (Py == 8 && m->cn_fastdiv) hipLaunchKernelGGL((k_io_cn_y_jac<W, true, 8>), gy, by, sy, m->stream, d, gs, facoe);
-            else if (Py == 8) hipLaunchKernelGGL((k_io_cn_y_jac<W, false, 8>), gy, by, sy, m->stream, d, gs, facoe);
-            else if (m->cn_fastdiv) hipLaunchKernelGGL((k_io_cn_y_jac<W, true, 4>), gy, by, sy, m->stream, d, gs, facoe);
-            else hipLaunchKernelGGL((k_io_cn_y_jac<W, false, 4>), gy, by, sy, m->stream, d, gs, facoe);
+            const dim3 gy(ng * N, 3), by(S);
+            const size_t sy = sizeof(double) * (4 * S + 1 + 2 * (M + 2));
+            if (Py == 8 && m->cn_fastdiv) hipLaunchKernelGGL((k_io_cn_y_jac<W, true, 8>), gy, by, sy, m->stream, d, gs, facoe, Ty);
+            else if (Py == 8) hipLaunchKernelGGL((k_io_cn_y_jac<W, false, 8>), gy, by, sy, m->stream, d, gs, facoe, Ty);
+            else if (m->cn_fastdiv) hipLaunchKernelGGL((k_io_cn_y_jac<W, true, 4>), gy, by, sy, m->stream, d, gs, facoe, Ty);
+            else hipLaunchKernelGGL((k_io_cn_y_jac<W, false, 4>), gy, by, sy, m->stream, d, gs, facoe, Ty);
         } else {
             hipLaunchKernelGGL(k_io_cn_y<W>, dim3((L * N + 127) / 128, 3), dim3(128), 0, m->stream, d, gs, facoe);
         }

@@ -3130,7 +3130,7 @@ struct chs_ctx {
     void *twx = nullptr, *twz = nullptr;
     void *rtwx = nullptr, *rtwz = nullptr;   // register-FFT pass twiddles (chs_fftr.h), if planned
     chs::GPlan gx{}, gxi{}, gz{};            // mixed-radix plans: x forward, x inverse, z (chs_fftg.h)
-    void *gtwx = nullptr, *gtwxi = nullptr, *gtwz = nullptr;   // their twiddles (null: not served)
+    void *gtw = nullptr, *gtwx = nullptr, *gtwxi = nullptr, *gtwz = nullptr;   // their twiddles (null: not served)
     chs::FftPlan px, pz;
     CnTab cn[4];
     // launch shapes (chs_set_tuning); 0 = derived from the mesh
@@ -3436,6 +3436,28 @@ int upload_vec(chs_ctx *c, const std::vector<V> &h, void **dst)
     HIPCHK(c, hipMalloc(dst, sizeof(V) * h.size()));
     HIPCHK(c, hipMemcpyAsync(*dst, h.data(), sizeof(V) * h.size(), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+}
+
+// The twiddles of the three mixed-radix plans in one allocation (c->gtw); a plan the kernels do not
+// take (other than two or three passes, more than 256 threads a line) gets none.
+template <typename T>
+int upload_gtw(chs_ctx *c)
+{
+    std::vector<cpx<T>> h;
+    size_t off[3];
+    const chs::GPlan *P[3] = {&c->gx, &c->gxi, &c->gz};
+    for (int i = 0; i < 3; ++i) {
+        off[i] = h.size();
+        if (P[i]->np < 2 || P[i]->np > 3 || P[i]->tpl > 256) continue;
+        const std::vector<cpx<T>> t = chs::gplan_twiddles<T>(*P[i]);
+        h.insert(h.end(), t.begin(), t.end());
+    }
+    if (h.empty()) return 0;
+    if (int e = upload_vec(c, h, &c->gtw)) return e;
+    void **dst[3] = {&c->gtwx, &c->gtwxi, &c->gtwz};
+    for (int i = 0; i < 3; ++i)
+        if ((i < 2 ? off[i + 1] : h.size()) > off[i]) *dst[i] = (cpx<T> *)c->gtw + off[i];
     return 0;
 }
 
@@ -4239,14 +4261,7 @@ static int create_impl(const chs_coeffs *cf, int mode, hipStream_t shared, chs_c
     c->gx = chs::gplan(L, false);
     c->gxi = chs::gplan(L, true);
     c->gz = chs::gplan(N, false);
-    auto gtw = [&](const chs::GPlan &P, void **dst) {
-        if (e || P.np < 2 || P.np > 3 || P.tpl > 256) return;
-        e = (mode == CHS_MIXED) ? upload_vec(c, chs::gplan_twiddles<float>(P), dst)
-                                : upload_vec(c, chs::gplan_twiddles<double>(P), dst);
-    };
-    gtw(c->gx, &c->gtwx);
-    gtw(c->gxi, &c->gtwxi);
-    gtw(c->gz, &c->gtwz);
+    if (!e) e = (mode == CHS_MIXED) ? upload_gtw<float>(c) : upload_gtw<double>(c);
     // register FFTs: x needs a plan for L and N divisible by the plane pairs of one wavefront
     int rad[8];
     if (!e && chs::rplan_radices(L, rad) && N % (2 * chs::rplan_lpw(L)) == 0)
@@ -4264,7 +4279,7 @@ void chs_destroy(chs_ctx *c)
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void *ptrs[] = {c->cf, c->q, c->qs, c->pr, c->phi, c->div, c->h0, c->rhs, c->rhs2, c->spec, c->pp,
-                    c->pp32, c->pp00, c->partial, c->scal, c->twx, c->twz, c->rtwx, c->rtwz, c->gtwx, c->gtwxi, c->gtwz, c->cn_stamp, c->mean_part};
+                    c->pp32, c->pp00, c->partial, c->scal, c->twx, c->twz, c->rtwx, c->rtwz, c->gtw, c->cn_stamp, c->mean_part};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->mean_host) (void)hipHostFree(c->mean_host);

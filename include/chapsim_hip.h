@@ -512,11 +512,12 @@ int chs_substep_io_momentum(chs_io *m, int ns, double dt);
  * per block of the LDS-staged staggered-property kernel of chs_io_props (default 16; 0 selects
  * the per-point kernel); "mom_rows": rows per 64 x 4 block of the per-point kernel (4
  * default, 2, 1; the block's other rows of threads take further z-planes); "cn_cols": most
- * x-columns per block of the Crank-Nicolson z and y Jacobi solves (1..64, default 16; rounded
- * down to whole wavefronts, the sequential solves where that leaves none), "cnz_cols" and
+ * x-columns per block of the Crank-Nicolson z and y Jacobi solves (1..64, default 16; the block is
+ * padded to whole wavefronts), "cnz_cols" and
  * "cny_cols" the same for one direction (0: cn_cols), "cnz_p" / "cny_p" their line points per
  * thread (8 default, or 4); "cnx_wave": the x-solve one wavefront
- * per line (1, default, for L = 64, 128, 256, 512) or one block per line (0); "cn_fastdiv":
+ * per line (1, default, where L is a multiple of at most 64 lanes of 1..10 points) or one block
+ * (powers of two up to 512) or thread per line (0); "cn_fastdiv":
  * the z and y solves' coefficients by Newton reciprocals (1, default) or IEEE division (0),
  * which changes them by an ulp, below the 1e-17 the sweeps resolve.  Otherwise results change
  * only through the summation order of the mass-flux partials.  CHS_E_ARG for an unknown key

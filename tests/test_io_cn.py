@@ -590,3 +590,35 @@ def test_gpu_io_fishpack_gauge(pkg, vis):
     with pytest.raises(pkg.ChsError):
         ch._check(pkg.lib().chs_io_set_poisson(ch._h, 2), "chs_io_set_poisson")
     ch.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,M,N,kv", [(90, 5, 30, {}), (54, 9, 50, {}), (60, 71, 90, {}), (250, 4, 10, {}),
+                                      (450, 4, 6, {}), (96, 13, 54, dict(cnz_p=4, cny_p=4)),
+                                      (36, 17, 20, dict(cn_cols=1)), (150, 6, 1280, dict(cn_cols=5)),
+                                      (90, 8, 30, dict(cn_fastdiv=0, cnz_p=4))])
+def test_gpu_cn_ragged_line_solves(pkg, L, M, N, kv):
+    """The x-solve on fewer than 64 lanes (L / P for P = 1 ... 10), z-lines whose last chunk is short
+    and blocks that are not whole wavefronts, against the per-line bounds of
+    test_gpu_cn_matches_oracle."""
+    print(f"io cn ragged {L}x{M}x{N} {kv}", flush=True)
+    mesh = setup.Mesh(L, M, N, STR2=2.0)
+    st = oracle.io_initial_field(mesh, 90 + L)
+    m1 = cn_viscosity(st, 90 + L, False)
+    REN, dt = 4000.0, 5e-4
+    o = oracle.OracleIO(mesh, REN, gravity=1, f_a=0.02, flow_driven=1, vis_scheme=1)
+    o.set_state(dict(st, M1=m1))
+    ch = pkg.ChannelIO(pkg.channel_setup(L, M, N, STR2=2.0), REN, gravity=1, f_a=0.02, flow_driven=1, vis_scheme=1)
+    ch.set_tuning(**kv)
+    ch.upload(**st, M1=m1)
+    for ns in (1, 2):
+        o.props(ns)
+        o.substep(ns, dt)
+        ch.ioprops(ns)
+        ch.SOLVERRK3_MOM_io(ns, dt)
+    f = ch.download()
+    for k in ("G", "Q"):
+        for c in range(3):
+            assert rel(f[k][c], o.f[k][c]) < 1e-11, (k, c, rel(f[k][c], o.f[k][c]))
+    assert rel(f["PR"], o.f["PR"]) < 1e-10, rel(f["PR"], o.f["PR"])
+    ch.close()
