@@ -548,6 +548,14 @@ __device__ __forceinline__ void bare_barrier()
     asm volatile("" ::: "memory");
 }
 
+// Wavefronts per SIMD that k_conv_rhs_dma's registers are held to: its blocks take 37 KB of LDS per
+// 64 columns (BY = 4), so that four blocks of 4 wavefronts (BXW = 1) or two of 8 (BXW = 2) share a
+// CU if they keep within 128 VGPRs.
+template <typename W> constexpr int conv_dma_waves(int by, int bxw, bool rg)
+{
+    return by == 4 && bxw <= 2 && (rg || sizeof(W) == 8) ? 4 : 1;
+}
+
 // k_conv_rhs_dma: the arithmetic of k_conv_rhs_lds with the state planes moved into LDS by
 // direct global-to-LDS loads (global_load_lds_dwordx4: a lane moves 16 bytes and a wavefront
 // one 1 KB chunk, with no register in between) into three rotating plane buffers [u v w p]
@@ -559,27 +567,32 @@ __device__ __forceinline__ void bare_barrier()
 // wavefront's loads of plane k+1 (vmcnt(0)) and barrier (then every wavefront's have landed,
 // and plane k-1's buffer is free: its x-solve is done), issue plane k+2, compute, barrier
 // (plane k read), write the RHS rows, barrier, x-solve.
-template <typename W, int BY, int BXW>
-__global__ __launch_bounds__(64 * BXW * BY) void k_conv_rhs_dma(Geo g, Sub s, const double *__restrict__ q,
+// RG: any even L <= 64 BXW and any M.  A block's rows of a plane are one run of memory, copied in
+// chunks whatever the row length; lanes past L and rows past M compute on repeated values and
+// store nothing.
+template <typename W, int BY, int BXW, bool RG = false>
+__global__ __launch_bounds__(64 * BXW * BY, conv_dma_waves<W>(BY, BXW, RG)) void k_conv_rhs_dma(Geo g, Sub s, const double *__restrict__ q,
                                                           const double *__restrict__ pr, W *__restrict__ h0,
                                                           W *__restrict__ rhs, double *__restrict__ partial,
                                                           int KC, int nxcd, const W *__restrict__ gx, int Dx)
 {
-    constexpr int L = 64 * BXW, R = BY + 2, NT = L * BY, NW = NT / 64;
-    constexpr int FS = R * L, PB = 4 * FS;        // doubles per field slab, per plane buffer
+    constexpr int LX = 64 * BXW, R = BY + 2, NT = LX * BY, NW = NT / 64;
+    constexpr int FS = R * LX, PB = 4 * FS;        // doubles per field slab, per plane buffer
     constexpr int NCH = PB / 128;                 // 1 KB chunks per plane buffer
     static_assert(FS % 128 == 0 && NCH % NW == 0, "a chunk lies in one field; chunks split evenly");
     constexpr int CPW = NCH / NW;                 // chunks per wavefront per plane
-    constexpr int XH = 16, LP = L + 2 * XH;       // RHS rows carry XH wrapped points each side
+    constexpr int XH = 16, LP = LX + 2 * XH;       // RHS rows carry XH wrapped points each side
     static_assert(3 * BY * LP * sizeof(W) <= PB * sizeof(double) && NT <= PB, "RHS rows fit a buffer");
     __shared__ double b0[PB], b1[PB], b2[PB];
     const int tile = __builtin_amdgcn_readfirstlane(xcd_tile(nxcd, own_blk()));
     const int ty = (tile / gridDim.x) % gridDim.y, tz = tile / (gridDim.x * gridDim.y);
-    const int i = threadIdx.x, t = __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int lane = i & 63, wv = __builtin_amdgcn_readfirstlane((t * L + i) >> 6);
+    const int N = g.N, M = g.M, L = RG ? g.L : LX;
+    const int i = RG ? min((int)threadIdx.x, L - 1) : (int)threadIdx.x;
+    const int t = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((t * LX + (int)threadIdx.x) >> 6);
     const int J0 = ty * BY + 1;
-    const int J = __builtin_amdgcn_readfirstlane(J0 + t);
-    const int N = g.N, M = g.M;
+    const int J = __builtin_amdgcn_readfirstlane(RG ? min(J0 + t, M) : J0 + t);
+    const bool own = !RG || ((int)threadIdx.x < L && J0 + t <= M);   // this thread's point is its own
     const size_t hs = (size_t)N * (M + 2) * L, cs = (size_t)N * M * L;
     const int kbeg = tz * KC, kend = min(N, kbeg + KC);
     const int ip = (i == L - 1) ? 0 : i + 1, im = (i == 0) ? L - 1 : i - 1;
@@ -591,13 +604,25 @@ __global__ __launch_bounds__(64 * BXW * BY) void k_conv_rhs_dma(Geo g, Sub s, co
     // plane kk of rows J0-1 .. J0+BY into buffer B: chunk ch (wave-uniform) is LDS elements
     // ch*128 .. ch*128+127, lane l moves elements ch*128 + 2l and + 2l + 1
     auto dma = [&](double *B, int kk) {
+        if constexpr (RG) {   // the rows are one run of memory: nf chunks a field, the last one's lanes
+                              // past the run (or past row M + 1) reload its last values
+            const int nf = (R * L + 127) >> 7, end = min(R, M + 3 - J0) * L - 2;
+            for (int ch = wv; ch < 4 * nf; ch += NW) {
+                const int f = ch / nf, cf = ch - f * nf;
+                const double *src = (const double *)uniform(grow(f, J0 - 1, kk)) + min(cf * 128 + 2 * lane, end);
+                __builtin_amdgcn_global_load_lds((const void *)src,
+                                                 (__attribute__((address_space(3))) void *)(B + f * FS + cf * 128),
+                                                 16, 0, 0);
+            }
+            return;
+        }
 #pragma unroll
         for (int c = 0; c < CPW; ++c) {
             const int ch = wv * CPW + c;
             const int f = (ch * 128) / FS, cf = ch - f * (FS / 128);   // field, chunk within it
             const double *src;
-            if constexpr (L % 128 == 0) {   // a chunk is part of one row: uniform base + lane
-                constexpr int CR = L / 128;
+            if constexpr (LX % 128 == 0) {   // a chunk is part of one row: uniform base + lane
+                constexpr int CR = LX / 128;
                 src = (const double *)(uniform(grow(f, J0 - 1 + cf / CR, kk) + (cf % CR) * 128) + 2 * lane);
             } else {                        // a chunk spans rows: row and x per lane
                 const int e = cf * 128 + 2 * lane, rr = e / L;
@@ -609,6 +634,7 @@ __global__ __launch_bounds__(64 * BXW * BY) void k_conv_rhs_dma(Geo g, Sub s, co
     };
     auto put = [&](W *xs, int cc, W v) {
         W *row = xs + (cc * BY + t) * LP + XH;
+        if (RG && (int)threadIdx.x >= L) return;
         row[i] = v;
         if (i < XH) row[L + i] = v;
         if (i >= L - XH) row[i - L] = v;
@@ -636,10 +662,11 @@ __global__ __launch_bounds__(64 * BXW * BY) void k_conv_rhs_dma(Geo g, Sub s, co
         const int r = t + 1;
         double rsum = 0.0;
         W hn[3];
+        const bool hist = s.troh != 0.0;   // NS = 0, 1: the history is not read
         auto hload = [&](int kk) {
             const size_t cc0 = ((size_t)kk * M + (J - 1)) * L;
 #pragma unroll
-            for (int f = 0; f < 3; ++f) hn[f] = uniform(h0 + f * cs + cc0)[i];
+            for (int f = 0; f < 3; ++f) hn[f] = hist ? uniform(h0 + f * cs + cc0)[i] : W(0);
         };
         hload(kbeg);
         auto plane = [&](int k, auto cbc) {
@@ -676,7 +703,7 @@ __global__ __launch_bounds__(64 * BXW * BY) void k_conv_rhs_dma(Geo g, Sub s, co
                 cu = conv;
                 const W pgm = (W)((p0 - pim) * g.dxi * coep);
                 ru = (rhsc + (W)(coev * lap)) * dt - pgm;
-                rsum += (double)ru;
+                if (own) rsum += (double)ru;
             }
             asm volatile("" ::: "memory");
             // ---- v (CONVECTION_Y.f90:37-84), stored for rows J >= 2 ----
@@ -714,9 +741,11 @@ __global__ __launch_bounds__(64 * BXW * BY) void k_conv_rhs_dma(Geo g, Sub s, co
                 const W pgm = (W)((p0 - p_m) * g.dzi * coep);
                 rw = (rhsc + (W)(coev * lap)) * dt - pgm;
             }
-            hr0[i] = cu;
-            if (J >= 2) hr1[i] = cv;
-            hr2[i] = cw;
+            if (own) {
+                hr0[i] = cu;
+                if (J >= 2) hr1[i] = cv;
+                hr2[i] = cw;
+            }
             u_m = u_c; v_m = v_c; w_m = w_c; p_m = p0; uip_m = uip; vjp_m = vjp;
             bare_barrier();   // plane k read by every wavefront (its reads have returned: their
                               // values are used above), so its buffer takes the RHS rows
@@ -733,7 +762,7 @@ __global__ __launch_bounds__(64 * BXW * BY) void k_conv_rhs_dma(Geo g, Sub s, co
                 const W *ln = xs + (cc * BY + t) * LP + XH + i;
                 W acc = gx[0] * ln[0];
                 for (int d = 1; d <= Dx; ++d) acc += gx[d] * (ln[d] + ln[-d]);   // Dx <= XH
-                uniform(rhs + cc * cs + c0)[i] = acc;
+                if (own) uniform(rhs + cc * cs + c0)[i] = acc;
             }
             // plane k+1's history values, loaded a plane ahead: no vector-memory wait inside a
             // plane is then behind that plane's in-flight state loads
@@ -756,7 +785,7 @@ __global__ __launch_bounds__(64 * BXW * BY) void k_conv_rhs_dma(Geo g, Sub s, co
     static_assert((P2 & (P2 - 1)) == 0, "block size 2^n or 3 * 2^n");
     __syncthreads();
     double *red = b0;
-    const int tid = t * L + i;
+    const int tid = t * LX + (int)threadIdx.x;
     red[tid] = mf;
     __syncthreads();
     if (P2 < NT) {
@@ -3137,7 +3166,7 @@ struct chs_ctx {
     // (defaults: the fastest shapes on MI355X for a 256 x 192 x 256 channel; cnx_nlx 0 means
     // 2048 / L lines)
     struct {
-        int conv_by = 4, conv_kc = 16;  // k_conv_rhs rows per block, z-planes per thread
+        int conv_by = 4, conv_kc = 0;   // k_conv_rhs rows per block, z-planes per thread (0: by the mesh)
         int conv_bx = 1;                // k_conv_rhs wavefronts along x per block (1 or 4)
         int conv_fence = 0;             // 1: all of a plane's loads stay ahead of its arithmetic
         int cnx_nlx = 0;                // k_cn_x lines per block
@@ -3152,7 +3181,7 @@ struct chs_ctx {
         int conv_lds = 2;                   // k_conv_rhs_lds rows per block (1, 2, 4; 0 = k_conv_rhs)
         int conv_dma = 4;                   // k_conv_rhs_dma rows per block (2, 4; 0 = k_conv_rhs_lds)
         int divg_nxcd = 8;                  // XCDs the k_divg_fftx_r rows are grouped for (1 = off)
-        int cny3_ky = 48;                   // k_cn_y3_march rows per chunk (0 = M; -1 = one launch per component)
+        int cny3_ky = -2;                   // k_cn_y3_march rows per chunk (-2 by the mesh; 0 = M; -1 = one launch per component)
         int upd_kz = 4;                     // k_update z-planes per thread
         int upd_by = 4;                     // k_update rows per block (1, 2, 4, 8, 16)
         int upd_nxcd = 1;                   // k_update tiles grouped for this many XCDs (1: launch order;
@@ -3160,7 +3189,7 @@ struct chs_ctx {
         int upd_w2 = 1;                     // k_update2 (two points per lane) where L % 128 == 0 (0 = k_update)
         int cnzy = 1;                       // z and y solves fused (k_cn_zy_march): 1 where L % 64 == 0
                                             // and N % 16 == 0, 2 on every mesh, 0 = two kernels
-        int cnzy_ky = 48;                   // k_cn_zy_march rows per chunk (0 = M)
+        int cnzy_ky = -1;                   // k_cn_zy_march rows per chunk (-1 by the mesh; 0 = M)
         int cnzy_nxcd = 8;                  // k_cn_zy_march tiles grouped for this many XCDs
     } tune;
     int tune_gen = 0;   // bumped by every chs_set_tuning / chs_set_refinement (graphs are re-made)
@@ -3549,6 +3578,47 @@ int gz_lines(const chs::GPlan &P, size_t cs, int lines)
     while (nl > 1 && nl * P.tpl > 64 && (lines + nl - 1) / nl < 512) nl = (nl + 1) / 2;
     return nl;
 }
+// z-planes per block of k_conv_rhs_dma (4 rows): its blocks fill the GPU in rounds of 256 CUs times the
+// blocks a CU holds, and a block reads two planes more than it computes, so the march is the one
+// with the least rounds x (planes + 2), the longest of equals.  256x192x256 52 planes (240 blocks in one
+// round, 6 % fewer plane loads than 16 planes in three: 285 -> 250 us, FP32 201 -> 183); 64x64x64
+// 4 (34 -> 17 us with 256 blocks in place of 64); 144x103x180 20 (118 -> 83 us with 234 blocks in
+// place of 312).
+int conv_march(int M, int N, int bxw, int waves)
+{
+    const long long cap = 256LL * (waves == 4 ? (bxw == 1 ? 4 : 2) : (bxw == 1 ? 2 : 1));
+    const long long rows = (M + 3) / 4;
+    int best = 4;
+    long long cost = -1;
+    for (int kc = 4; kc <= 64 && kc <= N; ++kc) {
+        const long long t = (rows * ((N + kc - 1) / kc) + cap - 1) / cap * (kc + 2);
+        if (cost < 0 || t <= cost) { cost = t; best = kc; }
+    }
+    return best;
+}
+// Rows per chunk of the marching y-solves: 48, fewer where the blocks would not fill the GPU.  A
+// chunk reads and computes the 2 D rows beside its own, so shorter ones cost more rows; with few
+// blocks the march's length is the time.
+int cny3_rows(int want, int L, int M, int N)
+{
+    if (want >= 0) return want > 0 ? want : M;
+    for (int ky : {48, 32, 24})   // 16 wavefronts (4 blocks) per CU
+        if ((long long)((L + 63) / 64) * N * 3 * ((M + ky - 1) / ky) >= 16 * 256) return ky;
+    return 16;
+}
+int cnzy_rows(int want, int L, int M, int N, int KB, int D)
+{
+    if (want >= 0) return want > 0 ? want : M;
+    const long long tiles = 3LL * ((L + 63) / 64) * ((N + KB - 1) / KB);
+    if (tiles * ((M + 47) / 48) >= 512) return 48;   // two blocks per CU
+    int best = 48;
+    long long cost = -1;
+    for (int ky : {48, 32, 24, 16, 12}) {   // rounds of 512 blocks x rows marched
+        const long long t = (tiles * ((M + ky - 1) / ky) + 511) / 512 * (ky + 2 * D + 4);
+        if (ky > D && (cost < 0 || t < cost)) { cost = t; best = ky; }
+    }
+    return best;
+}
 int block_threads(int n) { return (n + 63) / 64 * 64; }
 
 // Rows per chunk of k_ytdma_wide, 0 where k_ytdma_chunk or k_ytdma runs: automatic (want = -1)
@@ -3749,7 +3819,8 @@ int substep_impl(chs_ctx *c, int ns, double dt, double cvisc, bool host_dt = tru
     const size_t cs = (size_t)N * M * L;
     W *h0 = (W *)c->h0, *rhs = (W *)c->rhs, *rhs2 = (W *)c->rhs2;
     const dim3 blk(64, 4), grd((L + 63) / 64, (M + 3) / 4, N);
-    const int BY = c->tune.conv_by, KC = c->tune.conv_kc, BX = c->tune.conv_bx;
+    const int BY = c->tune.conv_by, BX = c->tune.conv_bx;
+    int KC = c->tune.conv_kc;
     CnTab &t = c->cn[ns];
     const int KZ = c->tune.cnz_kz, KY = c->tune.cny_ky;
     const bool zmarch = !t.fullz && t.Dz <= 8;
@@ -3759,21 +3830,36 @@ int substep_impl(chs_ctx *c, int ns, double dt, double cvisc, bool host_dt = tru
     // x-solve inside k_conv_rhs: whole x-lines of 1..4 wavefronts, a short x-inverse band, and
     // the z-marching kernel to take the deferred mass-flux correction
     const int FY = c->tune.conv_fx;   // rows per block of the fused kernel (0: not fused)
-    const bool fx = FY > 0 && M % FY == 0 && !xz && zmarch && L % 64 == 0 && L * FY <= 512 && !t.fullx &&
+    const bool fx0 = FY > 0 && M % FY == 0 && !xz && zmarch && L % 64 == 0 && L * FY <= 512 && !t.fullx &&
                     t.Dx <= 16;
     // state staged through LDS (k_conv_rhs_lds): LY rows of whole x-lines per block
     const int LY = c->tune.conv_lds;
     // state planes moved into LDS by direct loads (k_conv_rhs_dma): DY rows per block
     const int DY = c->tune.conv_dma;
-    const bool dma = fx && DY > 0 && M % DY == 0 && L <= 256 && L * DY <= 1024;
-    const bool lds = !dma && fx && LY > 0 && M % LY == 0 && L <= 256 && L * LY <= 1024;
+    const bool dma = fx0 && DY > 0 && M % DY == 0 && L <= 256 && L * DY <= 1024;
+    const bool lds = !dma && fx0 && LY > 0 && M % LY == 0 && L <= 256 && L * LY <= 1024;
+    // the same on ragged tiles: rows of 32 to 256 points in blocks of 64 BXW x 4 threads, the last rows
+    // past M idle.  us with the x-solve, FP64 / FP32, against the per-column kernel and k_cn_x:
+    // 150x97x120 53 / 44 and 90 / 66; 96x80x96 31 / 24 and 45 / 44; 250x150x200 229 / 145 and
+    // 319 / 258; 256x97x256 173 / 114 against 216 / 172 of the 2-row kernel
+    const bool rgd = !dma && c->tune.conv_fx > 0 && DY == 4 && !xz && zmarch && L >= 32 && L <= 256 && !t.fullx &&
+                     t.Dx <= 16;
+    const bool fx = fx0 || rgd;   // the x-solve runs inside the convection kernel
     const int RY = dma ? DY : LY;
-    const dim3 blkc = (dma || lds) ? dim3(L, RY) : fx ? dim3(L, FY) : dim3(64 * BX, BY);
-    const dim3 grdc = (dma || lds) ? dim3(1, M / RY, (N + KC - 1) / KC)
+    if (KC == 0) KC = (rgd || (dma && DY == 4)) ? conv_march(M, N, (L + 63) / 64, conv_dma_waves<W>(4, (L + 63) / 64, rgd)) : std::min(16, N);
+    const dim3 blkc = rgd ? dim3(64 * ((L + 63) / 64), 4) : (dma || lds) ? dim3(L, RY) : fx ? dim3(L, FY) : dim3(64 * BX, BY);
+    const dim3 grdc = rgd ? dim3(1, (M + 3) / 4, (N + KC - 1) / KC) : (dma || lds) ? dim3(1, M / RY, (N + KC - 1) / KC)
                       : fx         ? dim3(1, M / FY, (N + KC - 1) / KC)
                                    : dim3((L + 64 * BX - 1) / (64 * BX), (M + BY - 1) / BY, (N + KC - 1) / KC);
     const int npart = grdc.x * grdc.y * grdc.z;
-    if (dma) {
+    if (rgd) {
+        EvScope ev(c, "conv_rhs");
+        switch ((L + 63) / 64) {
+#define CHS_RCASE(bx) case bx: hipLaunchKernelGGL((k_conv_rhs_dma<W, 4, bx, true>), grdc, blkc, 0, c->stream, g, s, c->q, c->pr, h0, rhs, c->partial, KC, c->tune.nxcd, (const W *)t.gx, t.Dx); break;
+            CHS_RCASE(1) CHS_RCASE(2) CHS_RCASE(3) CHS_RCASE(4)
+#undef CHS_RCASE
+        }
+    } else if (dma) {
         EvScope ev(c, "conv_rhs");
         switch (DY * 10 + L / 64) {
 #define CHS_DCASE(by, bx) case by * 10 + bx: hipLaunchKernelGGL((k_conv_rhs_dma<W, by, bx>), grdc, blkc, 0, c->stream, g, s, c->q, c->pr, h0, rhs, c->partial, KC, c->tune.nxcd, (const W *)t.gx, t.Dx); break;
@@ -3835,7 +3921,7 @@ int substep_impl(chs_ctx *c, int ns, double dt, double cvisc, bool host_dt = tru
     // the block's side planes; batches of 2 FP64 / 4 FP32 rows, so that two blocks fit a CU
     // (48 KB of LDS each at Dz <= 4, and at most 64 VGPRs)
     constexpr int ZYKB = 16, ZYBT = sizeof(W) == 8 ? 2 : 4;
-    const int KZY = c->tune.cnzy_ky > 0 ? c->tune.cnzy_ky : M;
+    const int KZY = cnzy_rows(c->tune.cnzy_ky, L, M, N, ZYKB, Dym);
     // (by default only on whole tiles: on the ensemble's uneven meshes the ragged tiles made the
     // pass slower than the two kernels)
     const bool full = L % 64 == 0 && N % ZYKB == 0;
@@ -3869,10 +3955,10 @@ int substep_impl(chs_ctx *c, int ns, double dt, double cvisc, bool host_dt = tru
             hipLaunchKernelGGL(k_cn_z<W>, grd, blk, 0, c->stream, g, (const W *)t.gz, t.Dz, t.fullz, rhs, rhs2, comp);
         }
     }
-    const int KY3 = c->tune.cny3_ky > 0 ? c->tune.cny3_ky : M;
+    const int KY3 = cny3_rows(c->tune.cny3_ky, L, M, N);
     if (zy) {
         // the y-solves ran inside k_cn_zy_march
-    } else if (c->tune.cny3_ky >= 0 && Dym <= 8 && KY3 > Dym && ysame) {
+    } else if (c->tune.cny3_ky != -1 && Dym <= 8 && KY3 > Dym && ysame) {
         EvScope ev(c, "cn_y");
         const dim3 gy((L + 63) / 64, (N + 3) / 4, 3 * ((M + KY3 - 1) / KY3));
         const W *b0 = (const W *)t.by[0], *b1 = (const W *)t.by[1], *b2 = (const W *)t.by[2];
@@ -4880,7 +4966,7 @@ bool ens_batchable(const chs_ens *e)
         for (int ns = 1; ns <= 3; ++ns) {
             const CnTab &t = c->cn[ns];
             if (t.fullz || t.Dz > 8 || t.Dy[0] > 8 || t.Dy[1] != t.Dy[0] || t.Dy[2] != t.Dy[0]) return false;
-            if (c->M > 256 || c->nref_step != 0 || c->tune.cny3_ky < 0 ||
+            if (c->M > 256 || c->nref_step != 0 || c->tune.cny3_ky == -1 ||
                 ytdma_chunk_rows(c->tune.ytdma_c, c->M, c->H * c->N) == 0)
                 return false;
             if (c->tune.cny3_ky > 0 && c->tune.cny3_ky <= t.Dy[0]) return false;
@@ -4957,8 +5043,8 @@ int ens_make_launches(chs_ens *e, const double *dt, const double *cvisc, EnsLaun
             const int L = c->L, M = c->M, N = c->N, H = c->H;
             W *h0 = (W *)c->h0, *rhs = (W *)c->rhs, *rhs2 = (W *)c->rhs2;
             cpx<W> *spec = (cpx<W> *)c->spec;
-            const int KC = c->tune.conv_kc, KZ = c->tune.cnz_kz, KU = c->tune.upd_kz;
-            const int KY3 = c->tune.cny3_ky > 0 ? c->tune.cny3_ky : M;
+            const int KC = c->tune.conv_kc > 0 ? c->tune.conv_kc : std::min(16, N), KZ = c->tune.cnz_kz, KU = c->tune.upd_kz;
+            const int KY3 = cny3_rows(c->tune.cny3_ky, L, M, N);
             const int NLX = c->tune.cnx_nlx > 0 ? c->tune.cnx_nlx : ((2048 / L) < 1 ? 1 : 2048 / L);
             const int TK = c->tune.fftx_tk > 0 ? c->tune.fftx_tk : tk_for(L, N);
             const int NL = c->tune.fftz_nl > 0 ? c->tune.fftz_nl : nlz_for(N);

@@ -136,7 +136,8 @@ int chs_set_refinement(chs_ctx *ctx, int nref_step, int nref_projection);
  * "conv_bx" wavefronts along x per k_conv_rhs block (1 or 4, conv_bx * conv_by <= 16; 1),
  * "conv_fence" 1 to keep all of a z-plane's loads ahead of its arithmetic in k_conv_rhs (FP64 0,
  * mixed 1),
- * "conv_kc" z-planes marched per k_conv_rhs thread (1..N; 16), "cnx_nlx" x-lines per CN-x
+ * "conv_kc" z-planes marched per k_conv_rhs thread (1..N; by default chosen by the mesh for the
+ * direct-to-LDS kernel, else 16), "cnx_nlx" x-lines per CN-x
  * block (0 = 2048/L), "cnz_kz" / "cny_ky" march lengths of the z / y CN stencils (FP64 16 / 48,
  * mixed 8 / 32),
  * "fftx_tk" z-planes per x-transform block (0 = derived; even, divides N, TK/2*L <= 2048),
@@ -153,11 +154,11 @@ int chs_set_refinement(chs_ctx *ctx, int nref_step, int nref_projection);
  * threads per block of the Poisson y-solve (64 default, 128, 256) and "ytdma_rb" its rows per
  * load batch (8, 16 default), "ytdma_c" rows per chunk of the chunked y-Thomas (-1 = chosen by
  * the mesh, 0 = unchunked), "conv_dma" rows per block of the direct-to-LDS convection kernel
- * (4 default, 2; 0 = off), "cny3_ky" rows per chunk of the fused three-component y-solve (48;
+ * (4 default, 2; 0 = off), "cny3_ky" rows per chunk of the fused three-component y-solve (by default 16 to 48 by the mesh;
  * 0 = M, -1 = one launch per component), "cnzy" 1 (default) to run the z and y Crank-Nicolson
  * solves in one pass where L is a multiple of 64 and N of 16, 2 on every mesh (ragged tiles), 0
  * for the two kernels (the pass needs z and y band half-widths of at most 8), "cnzy_ky" its rows
- * per chunk (48; 0 = M), "cnzy_nxcd" the XCDs its tiles
+ * per chunk (by default 12 to 48 by the mesh; 0 = M), "cnzy_nxcd" the XCDs its tiles
  * are grouped for (8), "divg_nxcd" and "upd_nxcd" the XCDs the divergence
  * transform's and the correction's tiles are grouped for (8 and 1; 1 = dispatch order), "upd_kz"
  * z-planes each correction thread marches (4) and "upd_by" its rows per block (4), "upd_w2" 1

@@ -427,3 +427,49 @@ def test_wide_ytdma_matches_serial_lines(pkg, M):
         for a, b in zip(got, ref):
             assert rel(a, b) < tol, (mode, rel(a, b))
         ch.close()
+
+
+@pytest.mark.parametrize("L,M,N,REN,dt", [(32, 5, 10, 2000.0, 1.0e-3), (36, 4, 6, 4000.0, 5.0e-4), (60, 7, 50, 4000.0, 5.0e-4),
+                                          (64, 9, 20, 4000.0, 5.0e-4), (96, 6, 16, 4000.0, 5.0e-4), (128, 13, 18, 4000.0, 5.0e-4),
+                                          (150, 10, 36, 4000.0, 5.0e-4), (192, 11, 12, 4000.0, 5.0e-4), (250, 5, 24, 4000.0, 5.0e-4),
+                                          (256, 6, 100, 4000.0, 5.0e-4)])
+def test_ragged_convection_tiles_match_oracle(pkg, L, M, N, REN, dt):
+    """The direct-to-LDS convection kernel on ragged tiles (each width class, rows past M, a single
+    row left, marches cut short) over two RK3 steps against the oracle, and against the
+    per-column kernel (conv_dma = 0, conv_fx = 0) to rounding.  Bounds as
+    test_projection_and_steps_match_oracle; the two routes differ by the order of the mass-flux
+    sum and the banded x-solve's last bits: 1e-13 of the velocity."""
+    print(f"ragged convection {L}x{M}x{N}", flush=True)
+    mesh, ch, o = make(pkg, L, M, N, 1.8, REN)
+    _, ch2, _ = make(pkg, L, M, N, 1.8, REN)
+    ch2.set_tuning(conv_dma=0, conv_lds=0, conv_fx=0)
+    for c in (ch, ch2):
+        c.SOLVERRK3_MOM_tg(0, dt, 1.0 / REN)
+        for _ in range(2):
+            c.rk3_step(dt, 1.0 / REN)
+    o.substep(0, dt)
+    for _ in range(2):
+        o.step(dt)
+    q, p = ch.download()
+    q2, p2 = ch2.download()
+    assert max(rel(q[c], o.q[c]) for c in range(3)) < 1e-10
+    assert rel(p, o.pr) < 1e-9
+    assert max(rel(q[c], q2[c]) for c in range(3)) < 1e-13
+    ch.close()
+    ch2.close()
+
+
+@pytest.mark.parametrize("L,M,N,mode", [(64, 64, 64, "plain"), (64, 30, 32, "mixed"), (72, 33, 40, "plain"), (72, 33, 40, "mixed")])
+def test_y_chunks_by_mesh_change_no_bit(pkg, L, M, N, mode):
+    """The rows per chunk of the marching y-solves, chosen by the mesh, change no result: equal to
+    48-row chunks bit for bit."""
+    q, p = oracle.initial_field(setup.Mesh(L, M, N, STR2=1.8), 3)
+    out = []
+    for kv in ({}, dict(cnzy_ky=min(48, M), cny3_ky=min(48, M))):
+        ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=1.8), pkg.MIXED if mode == "mixed" else pkg.PLAIN_FP64)
+        ch.set_tuning(**kv)
+        ch.upload(q, p)
+        ch.rk3_step(1.0e-3, 1.0 / 2800.0)
+        out.append(ch.download())
+        ch.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
