@@ -1764,10 +1764,12 @@ struct chs_io {
     double *buf = nullptr;
     int npart = 0, flow_driven = 1;
     int mom_rows = 4;   // rows per momentum block (4, 2 or 1; the rest of its 4 rows of threads are z-planes)
-    int mom_kz = 32;    // z-planes per block of the LDS-staged momentum kernel (0: the per-point kernel)
+    int mom_kz = -1;    // z-planes per block of the LDS-staged momentum kernel (0: the per-point kernel; -1: by
+                        // the mesh)
     int mom_by = 4;     // rows per block of the LDS-staged momentum kernel (4 or 8)
     int mom_nxcd = 8;   // XCDs the LDS-staged momentum kernel groups its tiles for (1: launch order)
-    int props_kc = 16;  // z-planes per block of the LDS-staged staggered properties (0: per-point kernel)
+    int props_kc = 4;   // z-planes per block of the LDS-staged staggered properties (0: per-point kernel; 4
+                        // against 16: 256x128x256 252 and 256 us, 90x71x120 22 and 29)
     int cnz_cols = 0, cny_cols = 0;   // cn_cols for the z or the y solve alone (0: cn_cols)
     int cnz_p = 8, cny_p = 8;         // line points per thread of the z and y solves (4 or 8; 8:
                                       // 6.21 -> 6.09 (z) and 6.14 (y) ms per heated CN step)
@@ -2094,7 +2096,15 @@ void io_momentum_launch(chs_io *m, const double *gs, double tg, double tr, doubl
     auto a16 = [](const void *q) { return q == nullptr || ((uintptr_t)q & 15) == 0; };
     const bool aligned = m->L % 2 == 0 && a16(gs) && a16(d.q) && a16(d.mstg) && a16(d.m0) && a16(d.m1) &&
                          a16(d.pr) && a16(d.divu);
-    const int TY = m->mom_rows, TZ = 4 / TY, KZ = aligned ? m->mom_kz : 0, BY = m->mom_by, NX = m->mom_nxcd;
+    const int TY = m->mom_rows, TZ = 4 / TY, BY = m->mom_by, NX = m->mom_nxcd;
+    int KZ = aligned ? m->mom_kz : 0;
+    if (KZ < 0) {
+        // 32 planes where that leaves two rounds of two blocks per CU, else fewer (momentum part, us,
+        // with 32 / 16 / 8 / 4: 256x128x256 945 / 953 / 964 / 993; 150x97x120 291 / 276 / 263 / 261;
+        // 90x71x120 164 / 144 / 138 / 133)
+        KZ = 32;
+        while (KZ > 4 && (size_t)((m->L + 63) / 64) * ((m->M + BY - 1) / BY) * ((m->N + KZ - 1) / KZ) < 1024) KZ >>= 1;
+    }
     const dim3 gmom = KZ > 0 ? dim3((m->L + 63) / 64, (m->M + BY - 1) / BY, (m->N + KZ - 1) / KZ)
                              : dim3((m->L + 63) / 64, (m->M + TY - 1) / TY, (m->N + TZ - 1) / TZ);
     const int npart = (int)(gmom.x * gmom.y * gmom.z);   // at most the 64 x 4 row-block count

@@ -538,11 +538,45 @@ __device__ void eng_cell_props(const EngDev &e, const PropDev &p, size_t h0, int
     eng_cells_props<1>(e, p, &h0, &act, err, xdh, xh);
 }
 
+// BC_WALL_THERMAL(IMAIND) (BC_WALL.f90:622-643) at the ghost cell (i, k) of wall w (0 bottom, 1 top):
+// iso-flux walls extrapolate DH to the ghost row and look up H, T, D, M, K, Cp there
+// (BC_WALL_Isoflux :575-615); iso-thermal walls take the wall state and DH = H D
+// (BC_WALL_IsoTHERMAL :484-538).
+__device__ void eng_wall(const EngDev &e, const PropDev &p, int *err, int w, int i, int k)
+{
+#pragma clang fp contract(off)
+    const int M = e.M;
+    const size_t h0 = ehx(e, i, w == 0 ? 0 : M + 1, k);
+    if ((w == 0 ? e.wall_type0 : e.wall_type1) == 1) {
+        if (w == 0)
+            e.dh[h0] = 2.0 * e.dh[ehx(e, i, 1, k)] - e.wff[2] * e.dh[ehx(e, i, 2, k)] -
+                       e.wfb[2] * e.dh[ehx(e, i, 1, k)];
+        else
+            e.dh[h0] = 2.0 * e.dh[ehx(e, i, M, k)] - e.wff[e.top_face] * e.dh[ehx(e, i, M, k)] -
+                       e.wfb[e.top_face] * e.dh[ehx(e, i, M - 1, k)];
+        eng_cell_props(e, p, h0, err, p.dhh.x, p.ht.x);
+    } else {
+        e.t[h0] = e.ws[w][0];
+        e.h[h0] = e.ws[w][1];
+        e.d[h0] = e.ws[w][2];
+        e.m[h0] = e.ws[w][3];
+        e.k[h0] = e.ws[w][4];
+        e.dh[h0] = e.h[h0] * e.d[h0];
+    }
+}
+
 // THERM_PROP_UPDATE (THERM_PROP_UPDATE.f90:124-168) over rows j0..j1.  With lds != 0 the two
-// searched tables (2 n doubles of dynamic LDS) are staged per block first.
-__global__ __launch_bounds__(256) void k_eng_props(EngDev e, PropDev p, int j0, int j1, int *err, int lds)
+// searched tables (2 n doubles of dynamic LDS) are staged per block first.  walls: the launch has one
+// more row of blocks, which does BC_WALL_THERMAL (it reads DH only, which this kernel does not
+// write elsewhere): a launch of its own took 10 to 13 us of latency per stage.
+__global__ __launch_bounds__(256) void k_eng_props(EngDev e, PropDev p, int j0, int j1, int *err, int lds, int walls)
 {
     extern __shared__ double tab[];
+    if (walls && blockIdx.y == gridDim.y - 1) {   // thread rows: wall w = ty & 1 of planes k, k + gridDim.z
+        const int i = blockIdx.x * 64 + threadIdx.x, k = blockIdx.z + (threadIdx.y >> 1) * gridDim.z;
+        if (i < e.L && k < e.N) eng_wall(e, p, err, threadIdx.y & 1, i, k);
+        return;
+    }
     const double *xdh = p.dhh.x, *xh = p.ht.x;
     if (lds) {
         for (int t = threadIdx.x + 64 * threadIdx.y; t < p.n; t += 256) {
@@ -563,36 +597,13 @@ __global__ __launch_bounds__(256) void k_eng_props(EngDev e, PropDev p, int j0, 
     eng_cells_props<2>(e, p, h0, act, err, xdh, xh);
 }
 
-// BC_WALL_THERMAL(IMAIND) (BC_WALL.f90:622-643): iso-flux walls extrapolate DH to the ghost
-// row and look up H, T, D, M, K, Cp there (BC_WALL_Isoflux :575-615); iso-thermal walls take
-// the wall state and DH = H D (BC_WALL_IsoTHERMAL :484-538).  One thread per (i, k).
+// One thread per ghost cell (i, k) of each wall, for a property update that covered the ghost rows
+// too (rows 0..M+1, the start-up); otherwise the walls ride in k_eng_props' own launch.
 __global__ __launch_bounds__(256) void k_eng_walls(EngDev e, PropDev p, int *err)
 {
-#pragma clang fp contract(off)
     const int i = blockIdx.x * 256 + threadIdx.x;
-    const int k = blockIdx.y;
     if (i >= e.L) return;
-    const int M = e.M;
-    for (int w = 0; w < 2; ++w) {
-        const int J = w == 0 ? 0 : M + 1;
-        const size_t h0 = ehx(e, i, J, k);
-        if ((w == 0 ? e.wall_type0 : e.wall_type1) == 1) {
-            if (w == 0)
-                e.dh[h0] = 2.0 * e.dh[ehx(e, i, 1, k)] - e.wff[2] * e.dh[ehx(e, i, 2, k)] -
-                           e.wfb[2] * e.dh[ehx(e, i, 1, k)];
-            else
-                e.dh[h0] = 2.0 * e.dh[ehx(e, i, M, k)] - e.wff[e.top_face] * e.dh[ehx(e, i, M, k)] -
-                           e.wfb[e.top_face] * e.dh[ehx(e, i, M - 1, k)];
-            eng_cell_props(e, p, h0, err, p.dhh.x, p.ht.x);
-        } else {
-            e.t[h0] = e.ws[w][0];
-            e.h[h0] = e.ws[w][1];
-            e.d[h0] = e.ws[w][2];
-            e.m[h0] = e.ws[w][3];
-            e.k[h0] = e.ws[w][4];
-            e.dh[h0] = e.h[h0] * e.d[h0];
-        }
-    }
+    for (int w = 0; w < 2; ++w) eng_wall(e, p, err, w, i, blockIdx.y);
 }
 
 }  // namespace
@@ -620,7 +631,7 @@ struct chs_eng {
     double *d0 = nullptr, *m0 = nullptr;   // DENSITY0, Viscousity0 (swapped with e.d, e.m each substep)
     double *gown = nullptr;                 // own G (e.g1.. may point at a momentum context's G)
     int rhs_lds = 1;                        // energy RHS from LDS-staged planes (k_eng_rhs_lds)
-    int rhs_kc = 32;                        // its z-planes per block
+    int rhs_kc = 0;                         // its z-planes per block (0: by the mesh)
     int rhs_nxcd = 8;                       // XCDs its tiles are grouped for
     std::string errmsg;
 };
@@ -659,13 +670,14 @@ void eng_own_g(chs_eng *e)
 
 void eng_props_and_walls(chs_eng *e, int j0, int j1)
 {
-    const dim3 blk(64, 4), grd((e->L + 63) / 64, (j1 - j0 + 4) / 4, (e->N + 1) / 2);
+    const bool own = j0 >= 1 && j1 <= e->M;   // the ghost rows are the walls' alone
+    const dim3 blk(64, 4), grd((e->L + 63) / 64, (j1 - j0 + 4) / 4 + (own ? 1 : 0), (e->N + 1) / 2);
     // without bucket indexes the bisections run on LDS copies of the two searched tables;
     // with them, a search touches two or three entries, which the caches serve
     const size_t sh = 2 * sizeof(double) * (size_t)e->prop->p.n;
     const int lds = sh <= 64 * 1024 && (e->prop->p.bdh.nb == 0 || e->prop->p.bh.nb == 0);
-    hipLaunchKernelGGL(k_eng_props, grd, blk, lds ? sh : 0, e->stream, e->e, e->prop->p, j0, j1, e->err, lds);
-    hipLaunchKernelGGL(k_eng_walls, dim3((e->L + 255) / 256, e->N), dim3(256), 0, e->stream, e->e, e->prop->p,
+    hipLaunchKernelGGL(k_eng_props, grd, blk, lds ? sh : 0, e->stream, e->e, e->prop->p, j0, j1, e->err, lds, own);
+    if (!own) hipLaunchKernelGGL(k_eng_walls, dim3((e->L + 255) / 256, e->N), dim3(256), 0, e->stream, e->e, e->prop->p,
                        e->err);
 }
 
@@ -788,7 +800,11 @@ int chs_substep_eng(chs_eng *e, int ns, double dt)
     auto a16 = [](const void *q) { return ((uintptr_t)q & 15) == 0; };
     if (e->rhs_lds && e->L % 2 == 0 && a16(e->e.h) && a16(e->e.k) && a16(e->e.t) && a16(e->e.g1) && a16(e->e.g2) &&
         (e->hs % 2) == 0) {
-        const int KC = e->rhs_kc;
+        // planes per block: 32 where that leaves four blocks per CU (256x128x256: 417 us with 32 planes,
+        // 421 with 8, the whole substep), else fewer, down to 8 (90x71x120: 102 and 83 us)
+        int KC = e->rhs_kc > 0 ? e->rhs_kc : 32;
+        while (e->rhs_kc == 0 && KC > 8 && (size_t)((e->L + 63) / 64) * ((e->M + 3) / 4) * ((e->N + KC - 1) / KC) < 1024)
+            KC >>= 1;
         const dim3 grd((e->L + 63) / 64, (e->M + 3) / 4, (e->N + KC - 1) / KC);
         hipLaunchKernelGGL(k_eng_rhs_lds<4>, grd, dim3(64, 4), 0, e->stream, e->e, e->tgam[ns] * dt, e->troh[ns] * dt,
                            KC, e->rhs_nxcd);

@@ -361,7 +361,7 @@ int chs_substep_eng(chs_eng *e, int ns, double dt);
 /* Launch shape of the energy substep's right-hand side (no counterpart in the reference): key
  * "rhs_lds" 1 (default) for the kernel that stages H, K, T, G_x, G_y per z-plane in LDS, 0 for
  * the one reading them per point (identical results); "rhs_kc" its z-planes per block (1..1024,
- * default 32); "rhs_nxcd" the XCDs its tiles are grouped for (1..64, default 8).  CHS_E_ARG for
+ * by default 8 to 32 by the mesh); "rhs_nxcd" the XCDs its tiles are grouped for (1..64, default 8).  CHS_E_ARG for
  * an unknown key or a value out of range. */
 int chs_eng_set_tuning(chs_eng *e, const char *key, int value);
 
@@ -507,10 +507,10 @@ int chs_substep_io_momentum(chs_io *m, int ns, double dt);
 
 /* Launch shape of the main-domain momentum kernel, as chs_set_tuning is for the turbulence
  * generator; no counterpart in the reference.  Key "mom_kz": z-planes each block of the
- * LDS-staged momentum kernel marches (default 32; 0 selects the per-point kernel);
+ * LDS-staged momentum kernel marches (by default 4 to 32 by the mesh; 0 selects the per-point kernel);
  * "mom_by": its rows per block (4 default, or 8); "mom_nxcd": XCDs its tiles are grouped for
  * (default 8; 1 keeps launch order; also used by the staggered properties); "props_kc": z-planes
- * per block of the LDS-staged staggered-property kernel of chs_io_props (default 16; 0 selects
+ * per block of the LDS-staged staggered-property kernel of chs_io_props (default 4; 0 selects
  * the per-point kernel); "mom_rows": rows per 64 x 4 block of the per-point kernel (4
  * default, 2, 1; the block's other rows of threads take further z-planes); "cn_cols": most
  * x-columns per block of the Crank-Nicolson z and y Jacobi solves (1..64, default 16; the block is
