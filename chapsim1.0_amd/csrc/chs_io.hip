@@ -25,6 +25,7 @@ int chs_internal_poisson_in_place(chs_ctx *c, const double *rhs, int gauge);
 const double *chs_internal_phi(chs_ctx *c);
 void chs_internal_eng_fields(chs_eng *e, hipStream_t *s, double **d0, double **m0, double **m, double **g);
 void chs_internal_eng_set_g(chs_eng *e, const double *g);
+hipError_t chs_internal_eng_wait(chs_eng *e, hipStream_t other);
 double *chs_internal_eng_density(chs_eng *e);
 
 namespace {
@@ -2325,7 +2326,9 @@ int chs_heated_substep(chs_eng *e, chs_io *m, int ns, double dt)
     hipStream_t es;
     double *ed0, *em0, *em, *eg;
     chs_internal_eng_fields(e, &es, &ed0, &em0, &em, &eg);
-    hipError_t he = hipStreamSynchronize(m->stream);   // G of the last momentum substep is final
+    // the energy substep follows the last momentum substep, whose G it reads, on the GPU: the host
+    // waits once a stage (for the energy's range check) and not for each stream
+    hipError_t he = chs_internal_eng_wait(e, m->stream);
     if (he != hipSuccess) return io_hip(m, he, "chs_heated_substep");
     chs_internal_eng_set_g(e, m->d.g);                 // the energy reads the current G in place
     int rc = chs_substep_eng(e, ns, dt);               // synchronous

@@ -74,14 +74,38 @@ __device__ __forceinline__ int spl_index_b(const BucketDev &bk, const double *x,
     return I;
 }
 
+// Table-range flags: one int per bit in pinned host memory, written only by a lookup outside its
+// table, so a caller that has waited for the stream reads them without a copy.
+constexpr int kErrBits = 16;
+__device__ void raise_flags(int *err, int mask)
+{
+    for (int b = 0; b < kErrBits; ++b)
+        if (mask >> b & 1) err[b] = 1;
+}
+// The flags raised since the last call, cleared (host; the stream that may write them is idle).
+int take_flags(int *err)
+{
+    int mask = 0;
+    for (int b = 0; b < kErrBits; ++b)
+        if (err[b]) mask |= 1 << b;
+    for (int b = 0; b < kErrBits; ++b) err[b] = 0;
+    return mask;
+}
+hipError_t alloc_flags(int **err)
+{
+    hipError_t e = hipHostMalloc((void **)err, sizeof(int) * kErrBits, hipHostMallocDefault);
+    if (e == hipSuccess) take_flags(*err);
+    return e;
+}
+
 // spline_interpolation_* (thermo_properties_table_searching.f90:678-723 and siblings):
 // range check (tolerance 1e-8), bisection I = 1, J = N+1, then
 // Y(I) + DX*(B(I) + DX*(C(I) + DX*D(I))).
 __device__ double spl_eval(const SplineDev &s, const BucketDev &bk, int n, double xv, int *err, int bit)
 {
 #pragma clang fp contract(off)
-    if ((xv - s.x[s.imin - 1]) < -1.0e-8) atomicOr(err, bit);
-    if ((xv - s.x[s.imax - 1]) > 1.0e-8) atomicOr(err, bit << 8);
+    if ((xv - s.x[s.imin - 1]) < -1.0e-8) raise_flags(err, bit);
+    if ((xv - s.x[s.imax - 1]) > 1.0e-8) raise_flags(err, bit << 8);
     const int I = spl_index_b(bk, s.x, n, xv);
     const double dx = xv - s.x[I - 1];
     return s.y[I - 1] + dx * (s.b[I - 1] + dx * (s.c[I - 1] + dx * s.d[I - 1]));
@@ -493,8 +517,8 @@ __device__ void eng_cells_props(const EngDev &e, const PropDev &p, const size_t 
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         if (!act[c]) continue;
-        if ((dv[c] - p.dhh.x[p.dhh.imin - 1]) < -1.0e-8) atomicOr(err, 1);
-        if ((dv[c] - p.dhh.x[p.dhh.imax - 1]) > 1.0e-8) atomicOr(err, 1 << 8);
+        if ((dv[c] - p.dhh.x[p.dhh.imin - 1]) < -1.0e-8) raise_flags(err, 1);
+        if ((dv[c] - p.dhh.x[p.dhh.imax - 1]) > 1.0e-8) raise_flags(err, 1 << 8);
     }
     spl_index_lock<C>(p.bdh, xdh, p.n, dv, I);
 #pragma unroll
@@ -509,8 +533,8 @@ __device__ void eng_cells_props(const EngDev &e, const PropDev &p, const size_t 
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         if (!act[c]) continue;
-        if ((hv[c] - p.ht.x[p.ht.imin - 1]) < -1.0e-8) atomicOr(err, 2 | 4 | 8 | 16 | 32);
-        if ((hv[c] - p.ht.x[p.ht.imax - 1]) > 1.0e-8) atomicOr(err, (2 | 4 | 8 | 16 | 32) << 8);
+        if ((hv[c] - p.ht.x[p.ht.imin - 1]) < -1.0e-8) raise_flags(err, 2 | 4 | 8 | 16 | 32);
+        if ((hv[c] - p.ht.x[p.ht.imax - 1]) > 1.0e-8) raise_flags(err, (2 | 4 | 8 | 16 | 32) << 8);
     }
     spl_index_lock<C>(p.bh, xh, p.n, hv, I);
 #pragma unroll
@@ -633,6 +657,7 @@ struct chs_eng {
     int rhs_lds = 1;                        // energy RHS from LDS-staged planes (k_eng_rhs_lds)
     int rhs_kc = 0;                         // its z-planes per block (0: by the mesh)
     int rhs_nxcd = 8;                       // XCDs its tiles are grouped for
+    hipEvent_t after = nullptr;             // the momentum stream's last work (chs_internal_eng_wait)
     std::string errmsg;
 };
 
@@ -648,13 +673,10 @@ int eng_fail(chs_eng *e, int code, const std::string &msg)
 // Reads and clears the table-range flags of the last launches (the reference STOPs there).
 int eng_check(chs_eng *e, const char *what)
 {
-    int herr = 0;
     hipError_t he = hipGetLastError();
-    if (he == hipSuccess) he = hipMemcpyAsync(&herr, e->err, sizeof(int), hipMemcpyDeviceToHost, e->stream);
     if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
     if (he != hipSuccess) return eng_fail(e, CHS_E_HIP, std::string(what) + ": " + hipGetErrorString(he));
-    if (herr) {
-        (void)hipMemsetAsync(e->err, 0, sizeof(int), e->stream);
+    if (const int herr = take_flags(e->err)) {
         return eng_fail(e, CHS_E_RANGE, std::string(what) + ": DH outside the property table (flags " +
                                            std::to_string(herr) + ")");
     }
@@ -707,9 +729,8 @@ int chs_eng_create(const chs_coeffs *c, const chs_prop_table *table, const chs_e
     const size_t nb = 12 * e->hs + cs + 2 * (size_t)N * L + 4 * (size_t)(M + 2);
     hipError_t he = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
     if (he == hipSuccess) he = hipMalloc(&e->buf, sizeof(double) * nb);
-    if (he == hipSuccess) he = hipMalloc(&e->err, sizeof(int));
+    if (he == hipSuccess) he = alloc_flags(&e->err);
     if (he == hipSuccess) he = hipMemsetAsync(e->buf, 0, sizeof(double) * nb, e->stream);
-    if (he == hipSuccess) he = hipMemsetAsync(e->err, 0, sizeof(int), e->stream);
     std::vector<double> geo(4 * (size_t)(M + 2), 0.0);
     for (int J = 1; J <= M; ++J) geo[J] = c->dyfi[J - 1];
     for (int J = 1; J <= M + 1; ++J) {
@@ -754,7 +775,8 @@ void chs_eng_destroy(chs_eng *e)
     if (!e) return;
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     if (e->buf) (void)hipFree(e->buf);
-    if (e->err) (void)hipFree(e->err);
+    if (e->err) (void)hipHostFree(e->err);
+    if (e->after) (void)hipEventDestroy(e->after);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     if (e->prop) chs_prop_destroy(e->prop);
     delete e;
@@ -939,7 +961,7 @@ int chs_prop_create(const chs_prop_table *t, chs_prop **out)
     }
     hipError_t e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&p->dev, sizeof(double) * pack.size());
-    if (e == hipSuccess) e = hipMalloc(&p->err, sizeof(int));
+    if (e == hipSuccess) e = alloc_flags(&p->err);
     if (e == hipSuccess) e = hipMemcpyAsync(p->dev, pack.data(), sizeof(double) * pack.size(),
                                             hipMemcpyHostToDevice, p->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(p->stream);
@@ -1028,7 +1050,7 @@ void chs_prop_destroy(chs_prop *p)
     if (p->dev) (void)hipFree(p->dev);
     if (p->buckets) (void)hipFree(p->buckets);
     if (p->recs) (void)hipFree(p->recs);
-    if (p->err) (void)hipFree(p->err);
+    if (p->err) (void)hipHostFree(p->err);
     if (p->stream) (void)hipStreamDestroy(p->stream);
     delete p;
 }
@@ -1043,18 +1065,15 @@ int chs_prop_update_from_dh(chs_prop *p, long n, const double *dh, double *out)
     }
     if (n == 0) return CHS_OK;
     double *d_in = nullptr, *d_out = nullptr;
-    int herr = 0;
     hipError_t e = hipMalloc(&d_in, sizeof(double) * n);
     if (e == hipSuccess) e = hipMalloc(&d_out, sizeof(double) * 7 * n);
     if (e == hipSuccess) e = hipMemcpyAsync(d_in, dh, sizeof(double) * n, hipMemcpyHostToDevice, p->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(p->err, 0, sizeof(int), p->stream);
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_prop_from_dh, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, p->stream, p->p, n,
                            d_in, d_out, p->err);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(out, d_out, sizeof(double) * 7 * n, hipMemcpyDeviceToHost, p->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(&herr, p->err, sizeof(int), hipMemcpyDeviceToHost, p->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(p->stream);
     if (d_in) (void)hipFree(d_in);
     if (d_out) (void)hipFree(d_out);
@@ -1062,7 +1081,7 @@ int chs_prop_update_from_dh(chs_prop *p, long n, const double *dh, double *out)
         p->errmsg = std::string("chs_prop_update_from_dh: ") + hipGetErrorString(e);
         return CHS_E_HIP;
     }
-    if (herr) {
+    if (const int herr = take_flags(p->err)) {
         p->errmsg = "chs_prop_update_from_dh: value outside the property table (flags " + std::to_string(herr) + ")";
         return CHS_E_RANGE;
     }
@@ -1086,6 +1105,15 @@ __attribute__((visibility("hidden"))) void chs_internal_eng_fields(chs_eng *e, h
 
 // The current DENSITY of an energy context (CFL_io reads it).
 __attribute__((visibility("hidden"))) double *chs_internal_eng_density(chs_eng *e) { return e->e.d; }
+
+// Makes an energy context's stream wait for what another stream has been given so far (no host wait).
+__attribute__((visibility("hidden"))) hipError_t chs_internal_eng_wait(chs_eng *e, hipStream_t other)
+{
+    hipError_t he = hipSuccess;
+    if (!e->after) he = hipEventCreateWithFlags(&e->after, hipEventDisableTiming);
+    if (he == hipSuccess) he = hipEventRecord(e->after, other);
+    return he == hipSuccess ? hipStreamWaitEvent(e->stream, e->after, 0) : he;
+}
 
 // Point an energy context's G at a momentum context's G array (3 halo fields) instead of
 // copying it (NULL: back to the context's own array, as chs_eng_upload and
