@@ -80,3 +80,24 @@ def test_gpu_rejects_bad_arguments(pkg):
         pkg.tdma_lines(0, z, z + 1, z, z)          # cyclic line of 2 points
     with pytest.raises(pkg.ChsError):
         pkg.tdma_lines(7, z, z + 1, z, z)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n", [2, 3, 4, 15, 16, 17, 18, 32, 33, 34, 320, 321, 1280, 1281])
+def test_gpu_chunk_and_wavefront_edges(pkg, kind, n):
+    """Chunks of 16 points with the last one short or holding the cyclic solver's last unknown alone,
+    the longest lines of each LDS size and the first beyond them, and wavefronts with one line, all
+    but one and one more than 64: bit for bit against the oracle, on both entry points."""
+    if n < 3 and kind in (0, 3):
+        pytest.skip("a cyclic line needs 3 points")
+    for nl in (1, 63, 65):
+        rng = np.random.default_rng(1000 * kind + n + nl)
+        isz, jsz = (n, nl) if kind in (0, 2) else (nl, n)
+        A, C_ = rng.uniform(-1, 1, (2, jsz, isz))
+        B = 2.5 + rng.uniform(0, 1, (jsz, isz))
+        R = rng.standard_normal((jsz, isz))
+        bc = rng.standard_normal((2, nl))
+        ref = oracle.tdma_lines(kind, A, B, C_, R, bc)
+        assert np.array_equal(pkg.tdma_lines(kind, A, B, C_, R, bc), ref), (n, nl)
+        assert np.array_equal(pkg.tdma_lines(kind, A, B, C_, R, bc, noalloc=True), ref), (n, nl)
