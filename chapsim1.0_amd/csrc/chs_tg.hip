@@ -3581,7 +3581,7 @@ int gz_lines(const chs::GPlan &P, size_t cs, int lines)
 // z-planes per block of k_conv_rhs_dma (4 rows): its blocks fill the GPU in rounds of 256 CUs times the
 // blocks a CU holds, and a block reads two planes more than it computes, so the march is the one
 // with the least rounds x (planes + 2), the longest of equals.  256x192x256 52 planes (240 blocks in one
-// round, 6 % fewer plane loads than 16 planes in three: 285 -> 250 us, FP32 201 -> 183); 64x64x64
+// round, 6 % fewer plane loads than 16 planes in three: 285 -> 250 us, FP32 189 -> 182); 64x64x64
 // 4 (34 -> 17 us with 256 blocks in place of 64); 144x103x180 20 (118 -> 83 us with 234 blocks in
 // place of 312).
 int conv_march(int M, int N, int bxw, int waves)
@@ -3626,9 +3626,13 @@ int block_threads(int n) { return (n + 63) / 64 * 64; }
 // against 16.4 to 21.5 with 4 to 16 rows) and, up to the 256 rows it covers, fft_reg = 0, whose
 // steps the batched launches reproduce.  us by rows per chunk 8 / 12 / 16, and before:
 // 256x192x256 68 / 48 / 57, 70; 250x300x250 108 / 94 / 122; 512x384x512 425 / 449 / 545, 886.
-int ytdma_wide_rows(int want, int fft_reg, int M)
+// The FP32 spectrum keeps 16 rows up to M = 256, as k_ytdma_chunk: the FP64 sweeps round to FP32 at the
+// end, and other chunks move a few of those roundings, which p shows by 3e-6 of its size
+// (256x192x256: 77 us in k_ytdma_chunk, 58 here).
+int ytdma_wide_rows(int want, int fft_reg, int M, bool f64)
 {
     if (want >= 0 || M > 1024 || M <= 128 || (M <= 256 && !fft_reg)) return 0;
+    if (!f64 && M <= 256) return 16;
     return M <= 320 || (M > 512 && M <= 768) ? 12 : (M <= 512 ? 8 : 16);
 }
 
@@ -3717,7 +3721,7 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
         EvScope ev(c, "ytdma");
         const float *p32 = c->mode == CHS_MIXED ? c->pp32 : (const float *)nullptr;
         const double *p00 = gauge ? (const double *)c->pp00 : (const double *)nullptr;
-        const int CW = ytdma_wide_rows(c->tune.ytdma_c, c->tune.fft_reg, M);
+        const int CW = ytdma_wide_rows(c->tune.ytdma_c, c->tune.fft_reg, M, f64);
         const int C = CW ? 0 : ytdma_chunk_rows(c->tune.ytdma_c, M, H * N);
         if (C > 0) {
             const dim3 grid((H * N + 63) / 64), blk(64, (M + C - 1) / C);

@@ -473,3 +473,20 @@ def test_y_chunks_by_mesh_change_no_bit(pkg, L, M, N, mode):
         out.append(ch.download())
         ch.close()
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("L,M,N", [(64, 132, 64), (128, 192, 64), (64, 256, 50), (48, 161, 128)])
+def test_fp32_wide_ytdma_changes_no_bit(pkg, L, M, N):
+    """The mixed form's chunked y-solve keeps its 16-row chunks (M = 129 .. 256) in the kernel with 16
+    lines per wavefront: the same sums in the same order as with 64 lines (ytdma_c = 16), bit for bit."""
+    q, p = oracle.initial_field(setup.Mesh(L, M, N, STR2=1.8), 3)
+    out = []
+    for kv in ({}, dict(ytdma_c=16)):
+        ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=1.8), pkg.MIXED)
+        ch.set_tuning(**kv)
+        ch.upload(q, p)
+        for _ in range(2):
+            ch.rk3_step(1.0e-3, 1.0 / 2800.0)
+        out.append(ch.download())
+        ch.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
