@@ -2231,6 +2231,115 @@ __global__ __launch_bounds__(256, 4) void k_fftz_g(Geo g, chs::GPlan P, const cp
                                            [&](int k, const cpx<T> &x) { base[k] = x; });
 }
 
+// z-transform, y-Thomas and inverse z-transform of one kx in a block whose LDS holds the spectrum's
+// M x N plane (FP64, at most 160 KB): one launch and one trip through memory where the three kernels
+// make three, for small meshes, whose kernels are mostly launch and latency.  The Thomas lines go as
+// in k_ytdma_wide: thread (kz, q) takes the C rows of chunk q into registers (and the plane's LDS
+// then holds the chunks' end values).  Grid: L/2 + 1 blocks; bound
+// by the latency of its dependent phases.  us for the three kernels / this one, each launch timed
+// with about 3 us of events: 64x64x64 23.2 / 16.5, 96x80x96 33.0 / 22.8, 72x66x108 29.5 / 22.4,
+// 90x71x120 31.6 / 24.2, 192x71x120 41.6 / 25.9.
+constexpr int kPlaneCpx = 10240;   // complex values in 160 KB
+template <int C>
+__global__ __launch_bounds__(1024) void k_spec_plane(Geo g, chs::GPlan P, const cpx<double> *__restrict__ tw,
+                                                     const double *__restrict__ amph, const double *__restrict__ apph,
+                                                     const double *__restrict__ pp, const double *__restrict__ pp00,
+                                                     cpx<double> *__restrict__ spec, int PC)
+{
+    __shared__ cpx<double> pl[kPlaneCpx];
+    const int M = g.M, N = g.N, kx = blockIdx.x;
+    const size_t st = (size_t)g.H * N;
+    cpx<double> *base = spec + (size_t)kx * N;
+    const int ln = threadIdx.x / P.tpl, j = threadIdx.x - ln * P.tpl;
+    const bool act = ln < M;
+    cpx<double> *line = pl + (act ? ln : 0) * P.ls, *row = base + (size_t)(act ? ln : 0) * st;
+    chs::gfft_lines<double, -1, false, true>(P, line, j, act, tw, [&](int i) { return row[i]; },
+                                             [](int, const cpx<double> &) {});
+    {
+        const int q = threadIdx.x / N, kz = threadIdx.x - q * N, j0 = q * C;
+        const int n = q < PC ? max(0, min(C, M - j0)) : 0;   // rows j0 .. j0 + n - 1, 0-based
+        const int kp = kz + (kz >> P.ps);
+        const bool zero = kx == 0 && kz == 0, pin = zero && pp00, z99 = zero && !pp00;   // gauges as k_ytdma_chunk
+        double rr[C], ri[C], pv[C];
+#pragma unroll
+        for (int u = 0; u < C; ++u)
+            if (u < n) {
+                const cpx<double> v = pl[(j0 + u) * P.ls + kp];
+                rr[u] = v.x;
+                ri[u] = v.y;
+                pv[u] = pin ? pp00[j0 + u] : pp[(size_t)(j0 + u) * st + (size_t)kx * N + kz];
+            }
+        double gr = 0.0, gi = 0.0, lam = 1.0;
+#pragma unroll
+        for (int u = 0; u < C; ++u)
+            if (u < n) {
+                const double a = j0 + u == 0 ? 0.0 : amph[j0 + u];
+                const bool r0 = z99 && j0 + u == 0;
+                gr = ((r0 ? 0.0 : rr[u]) - a * gr) * pv[u];
+                gi = ((r0 ? 0.0 : ri[u]) - a * gi) * pv[u];
+                lam = -(a * pv[u]) * lam;
+                rr[u] = gr;
+                ri[u] = gi;
+            }
+        __syncthreads();   // the plane is in registers
+        double *xr = reinterpret_cast<double *>(pl), *xi = xr + 1024, *xl = xi + 1024;
+        xr[threadIdx.x] = gr;
+        xi[threadIdx.x] = gi;
+        xl[threadIdx.x] = lam;
+        __syncthreads();
+        double inr = 0.0, ini = 0.0;
+        for (int e = kz; e < (int)threadIdx.x; e += N) {
+            inr = xr[e] + xl[e] * inr;
+            ini = xi[e] + xl[e] * ini;
+        }
+        lam = 1.0;
+#pragma unroll
+        for (int u = 0; u < C; ++u)
+            if (u < n) {
+                lam = -((j0 + u == 0 ? 0.0 : amph[j0 + u]) * pv[u]) * lam;
+                rr[u] += lam * inr;
+                ri[u] += lam * ini;
+            }
+        double xhr = 0.0, xhi = 0.0, mu = 1.0;
+#pragma unroll
+        for (int u = C - 1; u >= 0; --u)
+            if (u < n) {
+                const double h = ((z99 && j0 + u == 0) ? 0.0 : apph[j0 + u]) * pv[u];
+                if (pin && j0 + u == M - 1) {
+                    xhr = 0.0;
+                    xhi = 0.0;
+                } else {
+                    xhr = rr[u] - h * xhr;
+                    xhi = ri[u] - h * xhi;
+                }
+                mu = -h * mu;
+                rr[u] = xhr;
+                ri[u] = xhi;
+            }
+        __syncthreads();   // every chunk has read the forward end values
+        xr[threadIdx.x] = xhr;
+        xi[threadIdx.x] = xhi;
+        xl[threadIdx.x] = mu;
+        __syncthreads();
+        double xir = 0.0, xii = 0.0;
+        for (int e = (PC - 1) * N + kz; e > (int)threadIdx.x; e -= N) {
+            xir = xr[e] + xl[e] * xir;
+            xii = xi[e] + xl[e] * xii;
+        }
+        mu = 1.0;
+        __syncthreads();   // the end values are read: the plane's LDS takes its rows again
+#pragma unroll
+        for (int u = C - 1; u >= 0; --u)
+            if (u < n) {
+                mu = -(((z99 && j0 + u == 0) ? 0.0 : apph[j0 + u]) * pv[u]) * mu;
+                pl[(j0 + u) * P.ls + kp] = {rr[u] + mu * xir, ri[u] + mu * xii};
+            }
+        __syncthreads();
+    }
+    chs::gfft_lines<double, +1, true, false>(P, line, j, act, tw, [](int) { return cpx<double>{}; },
+                                             [&](int k, const cpx<double> &x) { row[k] = x; });
+}
+
 // x forward: block = row J and TK consecutive z-planes (a plane pair per line; planes past N - 1
 // of the last block have no line).  TK = 16 or 8 gives spec runs of 256 or 128 bytes per kx; a
 // block's lines take 20 to 37 KB of LDS and its threads at most 128 VGPRs, so four blocks share a
@@ -3182,13 +3291,13 @@ struct chs_ctx {
         int conv_dma = 4;                   // k_conv_rhs_dma rows per block (2, 4; 0 = k_conv_rhs_lds)
         int divg_nxcd = 8;                  // XCDs the k_divg_fftx_r rows are grouped for (1 = off)
         int cny3_ky = -2;                   // k_cn_y3_march rows per chunk (-2 by the mesh; 0 = M; -1 = one launch per component)
-        int upd_kz = 4;                     // k_update z-planes per thread
+        int upd_kz = 0;                     // k_update z-planes per thread (0: by the mesh)
         int upd_by = 4;                     // k_update rows per block (1, 2, 4, 8, 16)
         int upd_nxcd = 1;                   // k_update tiles grouped for this many XCDs (1: launch order;
                                             // 8 measured equal at 256x192x256)
         int upd_w2 = 1;                     // k_update2 (two points per lane) where L % 128 == 0 (0 = k_update)
-        int cnzy = 1;                       // z and y solves fused (k_cn_zy_march): 1 where L % 64 == 0
-                                            // and N % 16 == 0, 2 on every mesh, 0 = two kernels
+        int cnzy = -1;                      // z and y solves fused (k_cn_zy_march): -1 by the mesh, 1 where
+                                            // L % 64 == 0 and N % 16 == 0, 2 on every mesh, 0 = two kernels
         int cnzy_ky = -1;                   // k_cn_zy_march rows per chunk (-1 by the mesh; 0 = M)
         int cnzy_nxcd = 8;                  // k_cn_zy_march tiles grouped for this many XCDs
     } tune;
@@ -3598,13 +3707,13 @@ int conv_march(int M, int N, int bxw, int waves)
 }
 // Rows per chunk of the marching y-solves: 48, fewer where the blocks would not fill the GPU.  A
 // chunk reads and computes the 2 D rows beside its own, so shorter ones cost more rows; with few
-// blocks the march's length is the time.
+// blocks the march's length is the time (96x80x96, rows 48 / 16 / 8: 23.5 / 14.4 / 13.0 us).
 int cny3_rows(int want, int L, int M, int N)
 {
     if (want >= 0) return want > 0 ? want : M;
-    for (int ky : {48, 32, 24})   // 16 wavefronts (4 blocks) per CU
+    for (int ky : {48, 32, 24, 16, 12})   // 16 wavefronts (4 blocks) per CU
         if ((long long)((L + 63) / 64) * N * 3 * ((M + ky - 1) / ky) >= 16 * 256) return ky;
-    return 16;
+    return 9;   // more than the widest band (8)
 }
 int cnzy_rows(int want, int L, int M, int N, int KB, int D)
 {
@@ -3618,6 +3727,13 @@ int cnzy_rows(int want, int L, int M, int N, int KB, int D)
         if (ky > D && (cost < 0 || t < cost)) { cost = t; best = ky; }
     }
     return best;
+}
+// z-planes each correction thread marches: 4, 2 where that leaves fewer than four blocks (of 4 rows)
+// per CU (64x64x64 10.0 -> 8.8 us).
+int upd_planes(int want, int L, int M, int N)
+{
+    if (want > 0) return want;
+    return (long long)((L + 63) / 64) * ((M + 3) / 4) * ((N + 3) / 4) < 1024 ? 2 : 4;
 }
 int block_threads(int n) { return (n + 63) / 64 * 64; }
 
@@ -3634,6 +3750,14 @@ int ytdma_wide_rows(int want, int fft_reg, int M, bool f64)
     if (want >= 0 || M > 1024 || M <= 128 || (M <= 256 && !fft_reg)) return 0;
     if (!f64 && M <= 256) return 16;
     return M <= 320 || (M > 512 && M <= 768) ? 12 : (M <= 512 ? 8 : 16);
+}
+
+// Rows per chunk of k_spec_plane (4, 8 or 12; 1024 / N chunks), 0 where a plane does not fit.
+int plane_rows(const chs::GPlan &P, int M, int N)
+{
+    if (N > 512 || M * P.tpl > 1024 || M * P.ls > kPlaneCpx) return 0;
+    const int c = (M + 1024 / N - 1) / (1024 / N);
+    return c <= 4 ? 4 : (c <= 8 ? 8 : (c <= 12 ? 12 : 0));
 }
 
 PhiOut halo_phi(const chs_ctx *c) { return {c->phi, (size_t)(c->M + 2) * c->L, 0}; }
@@ -3707,7 +3831,19 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
             hipLaunchKernelGGL(k_divg_fftx<T>, dim3(M, N / TK), dim3(256), shx, c->stream, g, pa, dv, talp, qv, dvo,
                                spec, TK, src);
     }
-    {
+    // the whole z-y-z part of a kx in one block where its plane fits
+    const int PLC = f64 && fr && c->gtwz && c->tune.ytdma_c < 0 ? plane_rows(c->gz, M, N) : 0;
+    if constexpr (sizeof(T) == 8) if (PLC > 0) {
+        EvScope ev(c, "spec_plane");
+        const int PC = 1024 / N, nt = block_threads(std::max(M * c->gz.tpl, N * PC));
+        const double *p00 = gauge ? (const double *)c->pp00 : (const double *)nullptr;
+        switch (PLC) {
+#define CHS_PLC(cc) case cc: hipLaunchKernelGGL((k_spec_plane<cc>), dim3(H), dim3(nt), 0, c->stream, g, c->gz, (const cpx<T> *)c->gtwz, c->d_amph, c->d_apph, c->pp, p00, spec, PC); break;
+            CHS_PLC(4) CHS_PLC(8) CHS_PLC(12)
+#undef CHS_PLC
+        }
+    }
+    if (PLC == 0) {
         EvScope ev(c, "fftz_fwd");
         if (rz)
             fftz_r<T>(N, dim3((M * H + LPZ - 1) / LPZ), c->stream, g, (const cpx<T> *)c->rtwz, spec, -1);
@@ -3717,7 +3853,7 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
         else
             hipLaunchKernelGGL(k_fftz<T>, dim3((M * H + NL - 1) / NL), dim3(256), shz, c->stream, g, pa, spec, NL, -1);
     }
-    {
+    if (PLC == 0) {
         EvScope ev(c, "ytdma");
         const float *p32 = c->mode == CHS_MIXED ? c->pp32 : (const float *)nullptr;
         const double *p00 = gauge ? (const double *)c->pp00 : (const double *)nullptr;
@@ -3746,7 +3882,7 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
                                c->d_apph, c->pp, p32, p00, spec);
         }
     }
-    {
+    if (PLC == 0) {
         EvScope ev(c, "fftz_inv");
         if (rz)
             fftz_r<T>(N, dim3((M * H + LPZ - 1) / LPZ), c->stream, g, (const cpx<T> *)c->rtwz, spec, +1);
@@ -3929,7 +4065,12 @@ int substep_impl(chs_ctx *c, int ns, double dt, double cvisc, bool host_dt = tru
     // (by default only on whole tiles: on the ensemble's uneven meshes the ragged tiles made the
     // pass slower than the two kernels)
     const bool full = L % 64 == 0 && N % ZYKB == 0;
-    const bool zy = (c->tune.cnzy == 2 || (c->tune.cnzy == 1 && full)) && !xz && zmarch && 2 * t.Dz <= ZYKB &&
+    // FP64 below 2^22 points: the fields stay in the caches and the pass's barriers cost more than the
+    // traffic it saves (us, fused / two kernels: 64x64x64 31 / 19, 128x128x128 62 / 55, 256x128x128
+    // 100 / 100, 256x96x192 104 / 113, 256x192x256 225 / 307)
+    const bool small = sizeof(W) == 8 && (size_t)L * M * N < (size_t(1) << 22);
+    const int want = c->tune.cnzy >= 0 ? c->tune.cnzy : (small ? 0 : 1);
+    const bool zy = (want == 2 || (want == 1 && full)) && !xz && zmarch && 2 * t.Dz <= ZYKB &&
                     t.Dz <= 8 && ysame && Dym <= 8 && KZY > Dym;
     if (zy) {
         EvScope ev(c, "cn_zy");
@@ -3987,7 +4128,7 @@ int substep_impl(chs_ctx *c, int ns, double dt, double cvisc, bool host_dt = tru
     // FP64-residual refinement (mixed form): the divergence of the corrected velocity drives
     // another solve and correction; the CFL then comes from the final field
     const int nref = ns == 0 ? c->nref_projection : c->nref_step;
-    const int KU = c->tune.upd_kz, UY = c->tune.upd_by;
+    const int UY = c->tune.upd_by, KU = upd_planes(c->tune.upd_kz, L, M, N);
     const bool u2 = c->tune.upd_w2 && L % 128 == 0;   // two points per lane
     const dim3 gu(u2 ? L / 128 : (L + 63) / 64, (M + UY - 1) / UY, (N + KU - 1) / KU), blku(64, UY);
     if (u2) {
@@ -5047,7 +5188,7 @@ int ens_make_launches(chs_ens *e, const double *dt, const double *cvisc, EnsLaun
             const int L = c->L, M = c->M, N = c->N, H = c->H;
             W *h0 = (W *)c->h0, *rhs = (W *)c->rhs, *rhs2 = (W *)c->rhs2;
             cpx<W> *spec = (cpx<W> *)c->spec;
-            const int KC = c->tune.conv_kc > 0 ? c->tune.conv_kc : std::min(16, N), KZ = c->tune.cnz_kz, KU = c->tune.upd_kz;
+            const int KC = c->tune.conv_kc > 0 ? c->tune.conv_kc : std::min(16, N), KZ = c->tune.cnz_kz, KU = upd_planes(c->tune.upd_kz, L, M, N);
             const int KY3 = cny3_rows(c->tune.cny3_ky, L, M, N);
             const int NLX = c->tune.cnx_nlx > 0 ? c->tune.cnx_nlx : ((2048 / L) < 1 ? 1 : 2048 / L);
             const int TK = c->tune.fftx_tk > 0 ? c->tune.fftx_tk : tk_for(L, N);

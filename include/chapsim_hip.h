@@ -154,14 +154,14 @@ int chs_set_refinement(chs_ctx *ctx, int nref_step, int nref_projection);
  * threads per block of the Poisson y-solve (64 default, 128, 256) and "ytdma_rb" its rows per
  * load batch (8, 16 default), "ytdma_c" rows per chunk of the chunked y-Thomas (-1 = chosen by
  * the mesh, 0 = unchunked), "conv_dma" rows per block of the direct-to-LDS convection kernel
- * (4 default, 2; 0 = off), "cny3_ky" rows per chunk of the fused three-component y-solve (by default 16 to 48 by the mesh;
- * 0 = M, -1 = one launch per component), "cnzy" 1 (default) to run the z and y Crank-Nicolson
- * solves in one pass where L is a multiple of 64 and N of 16, 2 on every mesh (ragged tiles), 0
+ * (4 default, 2; 0 = off), "cny3_ky" rows per chunk of the fused three-component y-solve (by default 9 to 48 by the mesh;
+ * 0 = M, -1 = one launch per component), "cnzy" 1 to run the z and y Crank-Nicolson
+ * solves in one pass where L is a multiple of 64 and N of 16 (the default, in FP64 from 2^22 points), 2 on every mesh (ragged tiles), 0
  * for the two kernels (the pass needs z and y band half-widths of at most 8), "cnzy_ky" its rows
  * per chunk (by default 12 to 48 by the mesh; 0 = M), "cnzy_nxcd" the XCDs its tiles
  * are grouped for (8), "divg_nxcd" and "upd_nxcd" the XCDs the divergence
  * transform's and the correction's tiles are grouped for (8 and 1; 1 = dispatch order), "upd_kz"
- * z-planes each correction thread marches (4) and "upd_by" its rows per block (4), "upd_w2" 1
+ * z-planes each correction thread marches (by default 2 or 4 by the mesh) and "upd_by" its rows per block (4), "upd_w2" 1
  * (default) for the correction with two points per lane where L is a multiple of 128 (0: one).  Results do not
  * depend on the shapes except through the summation order of the mass-flux partials
  * (conv_by, conv_kc, conv_fx) and conv_fx's rounding.  A captured step graph is re-made on

@@ -475,6 +475,27 @@ def test_y_chunks_by_mesh_change_no_bit(pkg, L, M, N, mode):
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
 
 
+@pytest.mark.parametrize("L,M,N", [(16, 4, 18), (64, 64, 64), (18, 80, 96), (12, 71, 120), (10, 35, 256), (30, 100, 36),
+                                   (20, 97, 90), (6, 18, 162), (8, 16, 512), (24, 12, 30)])
+def test_spectral_plane_in_one_block_matches_oracle(pkg, L, M, N):
+    """The z-transforms and the y-Thomas of a kx in one block (planes up to 160 KB of LDS: chunks of 4, 8
+    and 12 rows, the last short or empty, two- and three-pass z-plans) against the oracle (bound as
+    test_poisson_matches_oracle), and both gauges against the separate kernels (ytdma_c = 16),
+    which differ by rounding (bound as test_wide_ytdma_matches_serial_lines)."""
+    mesh = setup.Mesh(L, M, N, STR2=1.9)
+    r = np.random.default_rng(M + N).standard_normal((N, M, L))
+    w = (1.0 / mesh.DYFI)[None, :, None]
+    r -= np.sum(r * w) / (np.sum(w) * L * N)
+    ref = oracle.OracleTG(mesh, 2800.0).poisson(r)
+    ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=1.9), pkg.PLAIN_FP64)
+    got = [ch.poisson(r), ch.FISHPACK_POIS3D_SIMPLE(r)]
+    assert rel(got[0], ref) < 1e-10
+    ch.set_tuning(ytdma_c=16)
+    for a, b in zip(got, [ch.poisson(r), ch.FISHPACK_POIS3D_SIMPLE(r)]):
+        assert rel(a, b) < 1e-10, rel(a, b)
+    ch.close()
+
+
 @pytest.mark.parametrize("L,M,N", [(64, 132, 64), (128, 192, 64), (64, 256, 50), (48, 161, 128)])
 def test_fp32_wide_ytdma_changes_no_bit(pkg, L, M, N):
     """The mixed form's chunked y-solve keeps its 16-row chunks (M = 129 .. 256) in the kernel with 16
