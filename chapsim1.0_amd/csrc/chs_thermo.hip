@@ -26,30 +26,40 @@ std::string g_prop_err;
 struct SplineDev {
     const double *x, *y, *b, *c, *d;
     int imin, imax;   // 1-based, as IMIN_*/IMAX_* of the reference
+    double lo, hi;    // x there (dhh and ht)
 };
 
-// Bucket index over a non-decreasing searched table x: bucket b = floor((xv - x0) inv),
-// clamped to 0..nb-1, holds an index range lohi[2b] .. lohi[2b+1] that contains the
-// bisection's result for every xv of the bucket (the result, the count of x <= xv clamped to
-// 1..n, is monotone in xv; the range has one index of margin either side for the rounding of
-// the bucket edges).  Bisection inside that range gives the same index in one or two steps
-// instead of log2(n).  nb = 0: no index (table not monotone), full bisection.
+// Bucket index over a non-decreasing searched table x: bucket(xv) = floor((xv - x0) inv) clamped to
+// 0..nb-1.  It is monotone in xv, rounding included, so the table values of lower buckets are
+// below xv and those of higher ones above it: the bisection's result (the count of x <= xv, at least 1)
+// is lo plus the count of the bucket's own cnt values that are <= xv.  With 4 n buckets there is
+// mostly one or none, and its first value stands in the record: one 16-byte load per search.
+// nb = 0: no index (table not monotone), full bisection.
+struct BucketRec {
+    int lo, cnt;   // table values in lower buckets, in this one
+    double x1;     // the first of this one's
+};
 struct BucketDev {
-    const int *lohi;
+    const BucketRec *rec;
     double x0, inv;
     int nb;
 };
+// The bucket of xv, -1 for a NaN (the plain bisection).
+__host__ __device__ inline int bucket_of(const BucketDev &bk, double xv)
+{
+    const double f = (xv - bk.x0) * bk.inv;
+    return f == f ? (f <= 0.0 ? 0 : (f >= (double)(bk.nb - 1) ? bk.nb - 1 : (int)f)) : -1;
+}
 
 struct PropDev {
     int n;
     SplineDev dhh, ht, hd, hm, hk, hcp, hb;
     BucketDev bdh, bh;   // over LIST_DH (dhh.x) and LIST_H (ht.x and the other H splines)
-    // The same coefficients as records, one per table index, for the property update's
-    // evaluation (a cell's reads of one index then come in a few 16-byte loads):
-    // recd[8 i] = LIST_DH(i), then H's y, b, c, d (2 doubles of padding);
-    // rech[24 i] = LIST_H(i), then y, b, c, d of the H->T, H->M, H->K, H->D, H->Cp splines
-    // (3 of padding).
-    const double *recd, *rech;
+    // The same coefficients as records, one per table index, for the property update: recd[8 i] =
+    // LIST_DH(i), then H's y, b, c, d; recc[8 i] = LIST_H(i), then Cp's y, b, c, d (both with 3
+    // of padding: 64 bytes); rech[16 i] = y, b of the H->T, H->M, H->K and H->D splines, then their
+    // c, d (2 x 64 bytes).
+    const double *recd, *recc, *rech;
 };
 
 // The bisection of spline_interpolation_* (I = 1, J = N+1, thermo_properties_table_searching.f90:
@@ -57,13 +67,14 @@ struct PropDev {
 __device__ __forceinline__ int spl_index_b(const BucketDev &bk, const double *x, int n, double xv)
 {
     int I = 1, J = n + 1;
-    if (bk.nb > 0) {
-        const double f = (xv - bk.x0) * bk.inv;
-        if (f == f) {   // a NaN searches the whole table, as the plain bisection
-            const int b = f <= 0.0 ? 0 : (f >= (double)(bk.nb - 1) ? bk.nb - 1 : (int)f);
-            const int2 r = reinterpret_cast<const int2 *>(bk.lohi)[b];
-            I = r.x;
-            J = r.y + 1;
+    const int b = bk.nb > 0 ? bucket_of(bk, xv) : -1;
+    if (b >= 0) {
+        const BucketRec r = bk.rec[b];
+        I = r.lo;
+        J = r.lo + r.cnt + 1;
+        if (r.cnt == 1) {
+            if (xv < r.x1) J = I + 1;
+            else I = J - 1;
         }
     }
     while (J > I + 1) {
@@ -71,7 +82,7 @@ __device__ __forceinline__ int spl_index_b(const BucketDev &bk, const double *x,
         if (xv < x[K - 1]) J = K;
         else I = K;
     }
-    return I;
+    return max(I, 1);
 }
 
 // Table-range flags: one int per bit in pinned host memory, written only by a lookup outside its
@@ -446,6 +457,13 @@ __device__ __forceinline__ double spl_at(const SplineDev &s, int I, double xv)
     return s.y[I - 1] + dx * (s.b[I - 1] + dx * (s.c[I - 1] + dx * s.d[I - 1]));
 }
 
+// spline_interpolation_*'s range check.
+__device__ __forceinline__ void eng_range(const SplineDev &s, double v, int *err, int bits)
+{
+    if ((v - s.lo) < -1.0e-8) raise_flags(err, bits);
+    if ((v - s.hi) > 1.0e-8) raise_flags(err, bits << 8);
+}
+
 // spl_at from a record's x and y, b, c, d (the same expression).
 __device__ __forceinline__ double spl_rec(double x, double y, double b, double c, double d, double xv)
 {
@@ -454,112 +472,26 @@ __device__ __forceinline__ double spl_rec(double x, double y, double b, double c
     return y + dx * (b + dx * (c + dx * d));
 }
 
-// spl_index_b for C values in lockstep: the bisection steps are branch-free (a finished search
-// re-reads its own entry and keeps its bounds), so the C searches' loads go out together.
-// Two lockstep steps cover a bucket's index range unless the table clusters; the rest, if
-// any, runs as the plain loop.  Each result equals spl_index_b's.
-template <int C>
-__device__ __forceinline__ void spl_index_lock(const BucketDev &bk, const double *x, int n, const double *xv,
-                                               int *I)
-{
-    int J[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        I[c] = 1;
-        J[c] = n + 1;
-        if (bk.nb > 0) {
-            const double f = (xv[c] - bk.x0) * bk.inv;
-            if (f == f) {
-                const int b = f <= 0.0 ? 0 : (f >= (double)(bk.nb - 1) ? bk.nb - 1 : (int)f);
-                const int2 r = reinterpret_cast<const int2 *>(bk.lohi)[b];
-                I[c] = r.x;
-                J[c] = r.y + 1;
-            }
-        }
-    }
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
-        double xk[C];
-        int K[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            K[c] = (I[c] + J[c]) / 2;   // = I when the search is done (J = I + 1): a valid entry
-            xk[c] = x[K[c] - 1];
-        }
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const bool go = J[c] > I[c] + 1, lt = xv[c] < xk[c];
-            J[c] = (go && lt) ? K[c] : J[c];
-            I[c] = (go && !lt) ? K[c] : I[c];
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-        while (J[c] > I[c] + 1) {
-            const int K = (I[c] + J[c]) / 2;
-            if (xv[c] < x[K - 1]) J[c] = K;
-            else I[c] = K;
-        }
-}
-
-// THERM_PROP_UPDATE_FROM_DH for C cells (h0[c], those with act[c]).  The five H-based splines
-// share their table (LIST_H) and range (IMIN_H, IMAX_H), so one search serves all of them;
-// each result equals spl_eval's.  xdh / xh: LIST_DH / LIST_H (LDS copies or the global
-// tables).  An inactive cell searches the table's first entry and stores nothing.
-template <int C>
-__device__ void eng_cells_props(const EngDev &e, const PropDev &p, const size_t *h0, const bool *act, int *err,
-                                const double *xdh, const double *xh)
-{
-    double dv[C], hv[C];
-    int I[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) dv[c] = act[c] ? e.dh[h0[c]] : p.dhh.x[0];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        if (!act[c]) continue;
-        if ((dv[c] - p.dhh.x[p.dhh.imin - 1]) < -1.0e-8) raise_flags(err, 1);
-        if ((dv[c] - p.dhh.x[p.dhh.imax - 1]) > 1.0e-8) raise_flags(err, 1 << 8);
-    }
-    spl_index_lock<C>(p.bdh, xdh, p.n, dv, I);
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        hv[c] = 0.0;   // an inactive cell searches from any value
-        if (act[c]) {
-            const double2 *r = reinterpret_cast<const double2 *>(p.recd + (size_t)8 * (I[c] - 1));
-            const double2 r0 = r[0], r1 = r[1], r2 = r[2];
-            hv[c] = spl_rec(r0.x, r0.y, r1.x, r1.y, r2.x, dv[c]);
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        if (!act[c]) continue;
-        if ((hv[c] - p.ht.x[p.ht.imin - 1]) < -1.0e-8) raise_flags(err, 2 | 4 | 8 | 16 | 32);
-        if ((hv[c] - p.ht.x[p.ht.imax - 1]) > 1.0e-8) raise_flags(err, (2 | 4 | 8 | 16 | 32) << 8);
-    }
-    spl_index_lock<C>(p.bh, xh, p.n, hv, I);
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        if (!act[c]) continue;
-        const size_t o = h0[c];
-        const double2 *r = reinterpret_cast<const double2 *>(p.rech + (size_t)24 * (I[c] - 1));
-        double2 v[11];
-#pragma unroll
-        for (int q = 0; q < 11; ++q) v[q] = r[q];
-        const double x = v[0].x, h = hv[c];
-        e.h[o] = h;
-        e.t[o] = spl_rec(x, v[0].y, v[1].x, v[1].y, v[2].x, h);
-        e.d[o] = spl_rec(x, v[2].y, v[3].x, v[3].y, v[4].x, h);    // D from H->M, as the reference
-        e.m[o] = spl_rec(x, v[4].y, v[5].x, v[5].y, v[6].x, h);    // M from H->K
-        e.k[o] = spl_rec(x, v[6].y, v[7].x, v[7].y, v[8].x, h);    // K from H->D
-        e.cp[o] = spl_rec(x, v[8].y, v[9].x, v[9].y, v[10].x, h);
-    }
-}
-
-__device__ void eng_cell_props(const EngDev &e, const PropDev &p, size_t h0, int *err, const double *xdh,
+// THERM_PROP_UPDATE_FROM_DH for one cell, each lookup equal to spl_eval's.  The five H-based
+// splines share their table (LIST_H) and range (IMIN_H, IMAX_H), so one search serves all of them.
+// xdh / xh: LIST_DH / LIST_H (LDS copies or the global tables).
+__device__ void eng_cell_props(const EngDev &e, const PropDev &p, size_t o, int *err, const double *xdh,
                                const double *xh)
 {
-    const bool act = true;
-    eng_cells_props<1>(e, p, &h0, &act, err, xdh, xh);
+    const double dv = e.dh[o];
+    eng_range(p.dhh, dv, err, 1);
+    const double *r = p.recd + (size_t)8 * (spl_index_b(p.bdh, xdh, p.n, dv) - 1);
+    const double h = spl_rec(r[0], r[1], r[2], r[3], r[4], dv);
+    eng_range(p.ht, h, err, 2 | 4 | 8 | 16 | 32);
+    const int I = spl_index_b(p.bh, xh, p.n, h) - 1;
+    const double *c = p.recc + (size_t)8 * I, *v = p.rech + (size_t)16 * I;
+    const double x = c[0];
+    e.h[o] = h;
+    e.t[o] = spl_rec(x, v[0], v[1], v[8], v[9], h);
+    e.d[o] = spl_rec(x, v[2], v[3], v[10], v[11], h);  // D from H->M, as the reference
+    e.m[o] = spl_rec(x, v[4], v[5], v[12], v[13], h);  // M from H->K
+    e.k[o] = spl_rec(x, v[6], v[7], v[14], v[15], h);  // K from H->D
+    e.cp[o] = spl_rec(x, c[1], c[2], c[3], c[4], h);
 }
 
 // BC_WALL_THERMAL(IMAIND) (BC_WALL.f90:622-643) at the ghost cell (i, k) of wall w (0 bottom, 1 top):
@@ -589,18 +521,11 @@ __device__ void eng_wall(const EngDev &e, const PropDev &p, int *err, int w, int
     }
 }
 
-// THERM_PROP_UPDATE (THERM_PROP_UPDATE.f90:124-168) over rows j0..j1.  With lds != 0 the two
-// searched tables (2 n doubles of dynamic LDS) are staged per block first.  walls: the launch has one
-// more row of blocks, which does BC_WALL_THERMAL (it reads DH only, which this kernel does not
-// write elsewhere): a launch of its own took 10 to 13 us of latency per stage.
-__global__ __launch_bounds__(256) void k_eng_props(EngDev e, PropDev p, int j0, int j1, int *err, int lds, int walls)
+// THERM_PROP_UPDATE (THERM_PROP_UPDATE.f90:124-168) over rows j0..j1 for tables without a bucket
+// index: the bisections run on LDS copies of the two searched tables (lds != 0; 2 n doubles).
+__global__ __launch_bounds__(256) void k_eng_props_bisect(EngDev e, PropDev p, int j0, int j1, int *err, int lds)
 {
     extern __shared__ double tab[];
-    if (walls && blockIdx.y == gridDim.y - 1) {   // thread rows: wall w = ty & 1 of planes k, k + gridDim.z
-        const int i = blockIdx.x * 64 + threadIdx.x, k = blockIdx.z + (threadIdx.y >> 1) * gridDim.z;
-        if (i < e.L && k < e.N) eng_wall(e, p, err, threadIdx.y & 1, i, k);
-        return;
-    }
     const double *xdh = p.dhh.x, *xh = p.ht.x;
     if (lds) {
         for (int t = threadIdx.x + 64 * threadIdx.y; t < p.n; t += 256) {
@@ -611,14 +536,121 @@ __global__ __launch_bounds__(256) void k_eng_props(EngDev e, PropDev p, int j0, 
         xdh = tab;
         xh = tab + p.n;
     }
-    // two cells per thread, z-planes k and k + gridDim.z, searched in lockstep
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    const int J = j0 + blockIdx.y * 4 + threadIdx.y;
-    const int k = blockIdx.z, k2 = k + gridDim.z;
-    if (i >= e.L || J > j1) return;
-    const size_t h0[2] = {ehx(e, i, J, k), ehx(e, i, J, k2 < e.N ? k2 : k)};
-    const bool act[2] = {true, k2 < e.N};
-    eng_cells_props<2>(e, p, h0, act, err, xdh, xh);
+    const int i = blockIdx.x * 64 + threadIdx.x, J = j0 + blockIdx.y * 4 + threadIdx.y;
+    if (i < e.L && J <= j1) eng_cell_props(e, p, ehx(e, i, J, blockIdx.z), err, xdh, xh);
+}
+
+// The value of lane Q of this lane's quad (DPP; every lane of the wavefront takes part).
+template <int Q>
+__device__ __forceinline__ int quad_i(int v) { return __builtin_amdgcn_mov_dpp(v, 0x55 * Q, 0xf, 0xf, true); }
+template <int Q>
+__device__ __forceinline__ double quad_d(double v)
+{
+    return __hiloint2double(quad_i<Q>(__double2hiint(v)), quad_i<Q>(__double2loint(v)));
+}
+
+// Transposes a quad's 4 x 4 values: lane q's r[j] becomes lane j's r[q].
+__device__ __forceinline__ void quad_transpose(double *r, int q)
+{
+    auto swap = [&](int a, int b, bool up, auto ctrl) {   // with the partner lane: up keeps b and gives a
+        constexpr int P = decltype(ctrl)::value;
+        const double v = up ? r[a] : r[b];
+        const double w = __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), P, 0xf, 0xf, true),
+                                          __builtin_amdgcn_mov_dpp(__double2loint(v), P, 0xf, 0xf, true));
+        r[a] = up ? w : r[a];
+        r[b] = up ? r[b] : w;
+    };
+    constexpr std::integral_constant<int, 0xb1> x1{};   // quad_perm [1, 0, 3, 2]
+    constexpr std::integral_constant<int, 0x4e> x2{};   // quad_perm [2, 3, 0, 1]
+    swap(0, 1, q & 1, x1);
+    swap(2, 3, q & 1, x1);
+    swap(0, 2, q & 2, x2);
+    swap(1, 3, q & 2, x2);
+}
+
+// Cell Q of a quad's four: the quad reads the 64-byte record {x, y, b, c, d} of index I of lane
+// Q, 16 bytes a lane, and every lane evaluates it at lane Q's xv.
+template <int Q>
+__device__ __forceinline__ double quad_rec(const double *rec, int I, double xv, int q, double &x)
+{
+    const double2 v = reinterpret_cast<const double2 *>(rec + (size_t)8 * (quad_i<Q>(I) - 1))[q];
+    x = quad_d<0>(v.x);
+    return spl_rec(x, quad_d<0>(v.y), quad_d<1>(v.x), quad_d<1>(v.y), quad_d<2>(v.x), xv);
+}
+
+// THERM_PROP_UPDATE over rows j0 .. j0 + rows - 1 (one run of memory per plane), each lookup equal to
+// spl_eval's; blocks of 512 cells, two per thread for the latency of the dependent lookups.  Its
+// traffic is one field read and six written (80 us at 256x128x256); what bounds it is the lookups: a
+// wavefront's 64 records are 64 cache lines, a cycle of the cache per lane and load where each lane
+// fetches its own (20 loads a cell).  So a quad of lanes fetches its four cells' records one after
+// the other, 64 bytes at a time; for T, D, M and K lane q evaluates spline q of all four cells and
+// the results are transposed in the quad.  us before / now: 256x128x256 236 / 188 (134 with every
+// lookup in cache), 128x96x128 45 / 34, 90x71x120 33 / 20.  Table copies in LDS (blocks of a whole CU)
+// halved the cache misses and measured 181 and 29.
+// The first wrows block rows do BC_WALL_THERMAL (it reads DH only, which this kernel does not write
+// elsewhere): a launch of its own took 10 to 13 us of latency per stage.
+__global__ __launch_bounds__(256) void k_eng_props(EngDev e, PropDev p, int j0, int rows, int *err, int wrows)
+{
+    constexpr int C = 2;
+    if ((int)blockIdx.y < wrows) {
+        const long t = (long)(blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
+        const int i = (int)(t % e.L), k = (int)(t / e.L % e.N), w = (int)(t / e.L / e.N);
+        if (w < 2) eng_wall(e, p, err, w, i, k);
+        return;
+    }
+    const size_t base = ehx(e, 0, j0, blockIdx.y - wrows);
+    const int R = rows * e.L, c0 = blockIdx.x * (256 * C) + threadIdx.x, q = threadIdx.x & 3;
+    if (c0 - (int)(threadIdx.x & 63) >= R) return;   // a wavefront past the plane's end
+    double dv[C], hv[C], cp[C];
+    int I[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) dv[c] = e.dh[base + min(c0 + 256 * c, R - 1)];   // lanes past the end repeat the last cell
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        eng_range(p.dhh, dv[c], err, 1);
+        I[c] = spl_index_b(p.bdh, p.dhh.x, p.n, dv[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        double x;
+        const double h0 = quad_rec<0>(p.recd, I[c], quad_d<0>(dv[c]), q, x), h1 = quad_rec<1>(p.recd, I[c], quad_d<1>(dv[c]), q, x),
+                     h2 = quad_rec<2>(p.recd, I[c], quad_d<2>(dv[c]), q, x), h3 = quad_rec<3>(p.recd, I[c], quad_d<3>(dv[c]), q, x);
+        hv[c] = q == 0 ? h0 : q == 1 ? h1 : q == 2 ? h2 : h3;
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        eng_range(p.ht, hv[c], err, 2 | 4 | 8 | 16 | 32);
+        I[c] = spl_index_b(p.bh, p.ht.x, p.n, hv[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        double r[4], y[4];
+        auto cell = [&](auto Q) {
+            constexpr int j = decltype(Q)::value;
+            const double2 *s = reinterpret_cast<const double2 *>(p.rech + (size_t)16 * (quad_i<j>(I[c]) - 1));
+            const double2 s0 = s[q], s1 = s[4 + q];
+            double x;
+            const double h = quad_d<j>(hv[c]);
+            y[j] = quad_rec<j>(p.recc, I[c], h, q, x);
+            r[j] = spl_rec(x, s0.x, s0.y, s1.x, s1.y, h);
+        };
+        cell(std::integral_constant<int, 0>{});
+        cell(std::integral_constant<int, 1>{});
+        cell(std::integral_constant<int, 2>{});
+        cell(std::integral_constant<int, 3>{});
+        cp[c] = q == 0 ? y[0] : q == 1 ? y[1] : q == 2 ? y[2] : y[3];
+        quad_transpose(r, q);
+        const int n = c0 + 256 * c;
+        if (n < R) {
+            const size_t o = base + n;
+            e.h[o] = hv[c];
+            e.t[o] = r[0];
+            e.d[o] = r[1];   // D from H->M, as the reference
+            e.m[o] = r[2];   // M from H->K
+            e.k[o] = r[3];   // K from H->D
+            e.cp[o] = q == 0 ? y[0] : q == 1 ? y[1] : q == 2 ? y[2] : y[3];
+        }
+    }
 }
 
 // One thread per ghost cell (i, k) of each wall, for a property update that covered the ghost rows
@@ -635,8 +667,8 @@ __global__ __launch_bounds__(256) void k_eng_walls(EngDev e, PropDev p, int *err
 struct chs_prop {
     int n = 0;
     double *dev = nullptr;   // all table arrays, packed
-    int *buckets = nullptr;  // bucket indexes of LIST_DH and LIST_H
-    double *recs = nullptr;  // PropDev::recd and rech
+    BucketRec *buckets = nullptr;  // bucket indexes of LIST_DH and LIST_H
+    double *recs = nullptr;  // PropDev::rech, recd and recc
     int *err = nullptr;
     PropDev p;
     hipStream_t stream = nullptr;
@@ -692,15 +724,21 @@ void eng_own_g(chs_eng *e)
 
 void eng_props_and_walls(chs_eng *e, int j0, int j1)
 {
-    const bool own = j0 >= 1 && j1 <= e->M;   // the ghost rows are the walls' alone
-    const dim3 blk(64, 4), grd((e->L + 63) / 64, (j1 - j0 + 4) / 4 + (own ? 1 : 0), (e->N + 1) / 2);
-    // without bucket indexes the bisections run on LDS copies of the two searched tables;
-    // with them, a search touches two or three entries, which the caches serve
-    const size_t sh = 2 * sizeof(double) * (size_t)e->prop->p.n;
-    const int lds = sh <= 64 * 1024 && (e->prop->p.bdh.nb == 0 || e->prop->p.bh.nb == 0);
-    hipLaunchKernelGGL(k_eng_props, grd, blk, lds ? sh : 0, e->stream, e->e, e->prop->p, j0, j1, e->err, lds, own);
-    if (!own) hipLaunchKernelGGL(k_eng_walls, dim3((e->L + 255) / 256, e->N), dim3(256), 0, e->stream, e->e, e->prop->p,
-                       e->err);
+    bool own = j0 >= 1 && j1 <= e->M;   // the ghost rows are the walls' alone
+    const int rows = j1 - j0 + 1;
+    const PropDev &p = e->prop->p;
+    if (p.bdh.nb > 0 && p.bh.nb > 0) {
+        const int gx = (int)(((long)rows * e->L + 511) / 512);
+        const int wrows = own ? (int)((2L * e->L * e->N + 256L * gx - 1) / (256L * gx)) : 0;
+        hipLaunchKernelGGL(k_eng_props, dim3(gx, e->N + wrows), dim3(256), 0, e->stream, e->e, p, j0, rows, e->err, wrows);
+    } else {
+        const size_t sh = 2 * sizeof(double) * (size_t)p.n;
+        const int lds = sh <= 64 * 1024;
+        hipLaunchKernelGGL(k_eng_props_bisect, dim3((e->L + 63) / 64, (rows + 3) / 4, e->N), dim3(64, 4), lds ? sh : 0,
+                           e->stream, e->e, p, j0, j1, e->err, lds);
+        own = false;
+    }
+    if (!own) hipLaunchKernelGGL(k_eng_walls, dim3((e->L + 255) / 256, e->N), dim3(256), 0, e->stream, e->e, p, e->err);
 }
 
 }  // namespace
@@ -976,9 +1014,13 @@ int chs_prop_create(const chs_prop_table *t, chs_prop **out)
     const int ys[6] = {2, 3, 4, 5, 6, 7};   // T, D, M, K, Cp, B
     SplineDev *dst[6] = {&p->p.ht, &p->p.hd, &p->p.hm, &p->p.hk, &p->p.hcp, &p->p.hb};
     for (int c = 0; c < 6; ++c) *dst[c] = {A(1), A(ys[c]), A(11 + 3 * c), A(12 + 3 * c), A(13 + 3 * c), t->imin_h, t->imax_h};
-    // bucket indexes (2 n buckets) for the two searched tables where they are non-decreasing
-    const int nb = 2 * n;
-    std::vector<int> bk((size_t)4 * nb);
+    p->p.dhh.lo = t->dh[t->imin_dh - 1];
+    p->p.dhh.hi = t->dh[t->imax_dh - 1];
+    p->p.ht.lo = t->h[t->imin_h - 1];
+    p->p.ht.hi = t->h[t->imax_h - 1];
+    // bucket indexes (4 n buckets) for the two searched tables where they are non-decreasing
+    const int nb = 4 * n;
+    std::vector<BucketRec> bk((size_t)2 * nb);
     BucketDev *bd[2] = {&p->p.bdh, &p->p.bh};
     const double *xs[2] = {t->dh, t->h};
     for (int a = 0; a < 2; ++a) {
@@ -987,46 +1029,40 @@ int chs_prop_create(const chs_prop_table *t, chs_prop **out)
         bool mono = x[n - 1] > x[0];
         for (int i = 1; i < n && mono; ++i) mono = x[i] >= x[i - 1];
         if (!mono) continue;
-        auto bis = [&](double xv) {
-            int I = 1, J = n + 1;
-            while (J > I + 1) {
-                const int K = (I + J) / 2;
-                if (xv < x[K - 1]) J = K;
-                else I = K;
-            }
-            return I;
-        };
-        const double x0 = x[0], w = (x[n - 1] - x[0]) / (double)nb;
-        int *r = bk.data() + (size_t)a * 2 * nb;
-        for (int b = 0; b < nb; ++b) {
-            r[2 * b] = b == 0 ? 1 : std::max(1, bis(x0 + (double)b * w) - 1);
-            r[2 * b + 1] = b == nb - 1 ? n : std::min(n, bis(x0 + (double)(b + 1) * w) + 1);
+        *bd[a] = {nullptr, x[0], (double)nb / (x[n - 1] - x[0]), nb};
+        BucketRec *r = bk.data() + (size_t)a * nb;
+        for (int b = 0; b < nb; ++b) r[b] = {0, 0, 0.0};
+        bool ok = true;
+        for (int i = 0; i < n && ok; ++i) {
+            const int b = bucket_of(*bd[a], x[i]);
+            ok = b >= 0;
+            if (ok && r[b].cnt++ == 0) r[b].x1 = x[i];
         }
-        *bd[a] = {nullptr, x0, (double)nb / (x[n - 1] - x[0]), nb};
+        if (!ok) *bd[a] = {nullptr, 0.0, 0.0, 0};
+        for (int b = 1; b < nb; ++b) r[b].lo = r[b - 1].lo + r[b - 1].cnt;
     }
-    e = hipMalloc(&p->buckets, sizeof(int) * bk.size());
+    e = hipMalloc(&p->buckets, sizeof(BucketRec) * bk.size());
     if (e == hipSuccess)
-        e = hipMemcpyAsync(p->buckets, bk.data(), sizeof(int) * bk.size(), hipMemcpyHostToDevice, p->stream);
+        e = hipMemcpyAsync(p->buckets, bk.data(), sizeof(BucketRec) * bk.size(), hipMemcpyHostToDevice, p->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(p->stream);
     if (e != hipSuccess) {
         g_prop_err = std::string("chs_prop_create: ") + hipGetErrorString(e);
         chs_prop_destroy(p);
         return CHS_E_HIP;
     }
-    p->p.bdh.lohi = p->buckets;
-    p->p.bh.lohi = p->buckets + 2 * (size_t)nb;
-    // evaluation records (PropDev::recd, rech)
+    p->p.bdh.rec = p->buckets;
+    p->p.bh.rec = p->buckets + nb;
+    // evaluation records (PropDev::rech, recd, recc)
     std::vector<double> rec((size_t)32 * n, 0.0);
     for (int i = 0; i < n; ++i) {
-        double *rd = rec.data() + (size_t)8 * i, *rh = rec.data() + (size_t)8 * n + (size_t)24 * i;
+        double *rh = rec.data() + (size_t)16 * i, *rd = rec.data() + (size_t)16 * n + (size_t)8 * i, *rc = rd + (size_t)8 * n;
         const double vd[5] = {t->dh[i], t->h[i], t->dhh_b[i], t->dhh_c[i], t->dhh_d[i]};
-        for (int q = 0; q < 5; ++q) rd[q] = vd[q];
-        rh[0] = t->h[i];
-        const double *hs[5][4] = {{t->t, t->ht_b, t->ht_c, t->ht_d}, {t->m, t->hm_b, t->hm_c, t->hm_d},
-                                  {t->k, t->hk_b, t->hk_c, t->hk_d}, {t->d, t->hd_b, t->hd_c, t->hd_d},
-                                  {t->cp, t->hcp_b, t->hcp_c, t->hcp_d}};
-        for (int sp = 0; sp < 5; ++sp)
-            for (int q = 0; q < 4; ++q) rh[1 + 4 * sp + q] = hs[sp][q][i];
+        const double vc[5] = {t->h[i], t->cp[i], t->hcp_b[i], t->hcp_c[i], t->hcp_d[i]};
+        const double vh[16] = {t->t[i], t->ht_b[i], t->m[i], t->hm_b[i], t->k[i], t->hk_b[i], t->d[i], t->hd_b[i],
+                               t->ht_c[i], t->ht_d[i], t->hm_c[i], t->hm_d[i], t->hk_c[i], t->hk_d[i], t->hd_c[i], t->hd_d[i]};
+        std::copy(vd, vd + 5, rd);
+        std::copy(vc, vc + 5, rc);
+        std::copy(vh, vh + 16, rh);
     }
     e = hipMalloc(&p->recs, sizeof(double) * rec.size());
     if (e == hipSuccess)
@@ -1037,8 +1073,9 @@ int chs_prop_create(const chs_prop_table *t, chs_prop **out)
         chs_prop_destroy(p);
         return CHS_E_HIP;
     }
-    p->p.recd = p->recs;
-    p->p.rech = p->recs + (size_t)8 * n;
+    p->p.rech = p->recs;
+    p->p.recd = p->recs + (size_t)16 * n;
+    p->p.recc = p->recs + (size_t)24 * n;
     *out = p;
     return CHS_OK;
 }

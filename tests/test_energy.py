@@ -203,3 +203,62 @@ def test_gpu_energy_rhs_lds_equals_per_point(pkg, table):
         with pytest.raises(pkg.ChsError):
             e.set_tuning(**bad)
     e.close()
+
+
+def _bisect(x, v):
+    """The reference's table search (I = 1, J = N + 1), 0-based."""
+    lo, hi = np.ones(v.shape, int), np.full(v.shape, len(x) + 1)
+    while np.any(hi > lo + 1):
+        k = (lo + hi) // 2
+        lt, go = v < x[np.maximum(k, 1) - 1], hi > lo + 1
+        hi, lo = np.where(go & lt, k, hi), np.where(go & ~lt, k, lo)
+    return lo - 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,L,M,N", [("clustered", 18, 7, 6), ("clustered", 90, 71, 4), ("clustered", 64, 16, 4),
+                                        ("unordered", 18, 7, 6)])
+def test_gpu_cell_props_on_uneven_tables(pkg, kind, L, M, N):
+    """The property update (start-up and substep) against the plain bisection, bit for bit, on tables
+    whose buckets hold several values or none and on one that is not ordered (no bucket index);
+    meshes whose planes end inside a wavefront, inside a quad and on a block."""
+    from importlib import import_module
+    thermo = import_module(pkg.__name__ + ".thermo")
+    if kind == "clustered":
+        t = thermo.table_setup(thermo.synthetic_table(n=4000)[np.unique((np.linspace(0, 1, 80) ** 4 * 3999).astype(int))], 665.0)
+    else:
+        t = thermo.table_setup(thermo.synthetic_table(n=256), 630.0)
+    x, n = np.asarray(t["DH"]), t["N"]
+    assert (kind == "clustered") == bool(np.all(np.diff(x) > 0))
+
+    def spline(s, tab, y, v):
+        i = _bisect(np.asarray(tab), v)
+        dx = v - np.asarray(tab)[i]
+        return np.asarray(y)[i] + dx * (t[s + "_B"][i] + dx * (t[s + "_C"][i] + dx * t[s + "_D"][i]))
+
+    rng = np.random.default_rng(L + M)
+    i = rng.integers(n // 10, n - n // 10, 40000)
+    v = x[i] + (x[i + 1] - x[i]) * np.where(i % 4 == 0, 0.0, rng.uniform(0.0, 1.0, i.size))
+    lo, hi = t["IMIN_DH"] - 1, t["IMAX_DH"] - 1
+    hv = spline("DHH", x, t["H"], v)
+    hr = np.asarray(t["H"])[[t["IMIN_H"] - 1, t["IMAX_H"] - 1]]
+    v = v[(v > x[lo]) & (v < x[hi]) & (hv > hr[0]) & (hv < hr[1])]
+    dh = np.zeros((N, M + 2, L))
+    dh[:, 1:M + 1] = np.resize(v, N * M * L).reshape(N, M, L)
+    dh[:, 0], dh[:, M + 1] = dh[:, 1], dh[:, M]
+    h0 = float(np.median(hv))
+    ws = [[1.0, h0, 1.0, 1.0, 1.0]] * 2
+    e = thermo.EnergyTG(pkg.channel_setup(L, M, N, STR2=1.9), t, (2, 2), 1e-12, x[lo], x[hi], (0.0, 0.0), wall_state=ws)
+    e.upload(dh, np.zeros((3, N, M + 2, L)))
+    for step in range(2):
+        if step:
+            e.SOLVERRK3_ENG_io(1, 1e-9)
+        out = e.download()
+        d = out["DH"][:, 1:M + 1]
+        h = spline("DHH", x, t["H"], d)
+        want = {"H": h, "T": spline("HT", t["H"], t["T"], h), "D": spline("HM", t["H"], t["M"], h),
+                "M": spline("HK", t["H"], t["K"], h), "K": spline("HD", t["H"], t["D"], h),
+                "CP": spline("HCp", t["H"], t["CP"], h)}
+        for k, w in want.items():
+            np.testing.assert_array_equal(out[k][:, 1:M + 1], w, err_msg=k)
+    e.close()
