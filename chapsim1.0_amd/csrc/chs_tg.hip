@@ -2105,7 +2105,9 @@ __global__ __launch_bounds__(64) void k_fftz_r(Geo g, const cpx<T> *__restrict__
     });
 }
 
-// x forward: block = row J and TK = 2 LPW consecutive z-planes (plane pair per line).
+// x forward: block = row J and TK = 2 LPW consecutive z-planes (plane pair per line).  Bound by
+// memory: 98 us at 256x192x256 (4 TB/s), 7.5 at 64x64x64; with a branch between one point's loads and
+// the next's the points went one after the other (105 and 12 us).
 template <typename T, int L>
 __global__ __launch_bounds__(64) void k_divg_fftx_r(Geo g, const cpx<T> *__restrict__ tw, const double *__restrict__ dv,
                                                     double talp,
@@ -2121,32 +2123,38 @@ __global__ __launch_bounds__(64) void k_divg_fftx_r(Geo g, const cpx<T> *__restr
     const int tile = __builtin_amdgcn_readfirstlane(xcd_tile(nxcd, own_blk()));
     const int J = tile % gridDim.x + 1, k0 = (tile / gridDim.x) * TK, ka = k0 + 2 * li;
     const size_t hs = (size_t)g.N * (g.M + 2) * L;
-    const double *u = q, *v = q + hs, *w = q + 2 * hs;
     const double dyf = g.dyfi[J - 1];
     const double coe0 = dv ? 1.0 / (dv[0] * talp) : 1.0;   // 1 / (alpha DT) (DIVG_tg)
     cpx<T> x[G::E];
+    double d[2][G::E];
+    const size_t c0 = cix(g, 0, J, ka), c1 = c0 + (size_t)g.M * L, ps = (size_t)(g.M + 2) * L;
+    auto pt = [&](int e) { return t + e / G::R0 * G::TL + e % G::R0 * (L / G::R0); };
+    if (src) {
 #pragma unroll
-    for (int b = 0; b < G::E / G::R0; ++b)
-#pragma unroll
-        for (int r = 0; r < G::R0; ++r) {
-            const int i = t + b * G::TL + r * (L / G::R0);
-            double d[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int k = ka + h;
-                if (src) {
-                    d[h] = src[cix(g, i, J, k)];
-                } else {
-                    const int ip = (i == L - 1) ? 0 : i + 1, kp = (k == g.N - 1) ? 0 : k + 1;
-                    const double dd = divg_cell(u[hix(g, ip, J, k)], u[hix(g, i, J, k)], v[hix(g, i, J + 1, k)],
-                                                v[hix(g, i, J, k)], w[hix(g, i, J, kp)], w[hix(g, i, J, k)], g.dxi,
-                                                dyf, g.dzi);
-                    d[h] = dd * coe0;
-                    if (div) div[cix(g, i, J, k)] = d[h];
-                }
-            }
-            x[b * G::R0 + r] = {(T)d[0], (T)d[1]};
+        for (int e = 0; e < G::E; ++e) {
+            d[0][e] = src[c0 + pt(e)];
+            d[1][e] = src[c1 + pt(e)];
         }
+    } else {
+        const double *u = q + ka * ps + (size_t)J * L, *v = u + hs, *w = v + hs;
+        const double *w2 = q + 2 * hs + (size_t)(ka + 2 >= g.N ? 0 : ka + 2) * ps + (size_t)J * L;
+#pragma unroll
+        for (int e = 0; e < G::E; ++e) {
+            const int i = pt(e), ip = (i == L - 1) ? 0 : i + 1;
+            const double wm = w[ps + i];
+            d[0][e] = divg_cell(u[ip], u[i], v[L + i], v[i], wm, w[i], g.dxi, dyf, g.dzi) * coe0;
+            d[1][e] = divg_cell(u[ps + ip], u[ps + i], v[ps + L + i], v[ps + i], w2[i], wm, g.dxi, dyf, g.dzi) * coe0;
+        }
+        if (div) {
+#pragma unroll
+            for (int e = 0; e < G::E; ++e) {
+                div[c0 + pt(e)] = d[0][e];
+                div[c1 + pt(e)] = d[1][e];
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < G::E; ++e) x[e] = {(T)d[0][e], (T)d[1][e]};
     cpx<T> *line = lds + li * G::LS;
     chs::rfft_line<T, L>(x, line, t, tw, -1, [&](int idx, const cpx<T> &z) { line[chs::rpad<G::PS>(idx)] = z; });
     chs::wave_lds_sync();
@@ -2165,7 +2173,8 @@ __global__ __launch_bounds__(64) void k_divg_fftx_r(Geo g, const cpx<T> *__restr
 }
 
 // x inverse: Hermitian extension of the plane pair of each line, complex inverse transform,
-// real parts to the solution rows (CELLS: of a cell field, else of the halo field; PhiOut).
+// real parts to the solution rows.  Five loads of each plane in flight per lane: 256x192x256 37 us
+// (42 with one at a time), FP32 28 (31), 64x64x64 6.5 (7.1).  (CELLS: of a cell field, else of the halo field; PhiOut).
 template <typename T, int L, bool CELLS>
 __global__ __launch_bounds__(64) void k_fftx_inv_r(Geo g, const cpx<T> *__restrict__ tw,
                                                    const cpx<T> *__restrict__ spec, double *__restrict__ phi)
@@ -2177,11 +2186,23 @@ __global__ __launch_bounds__(64) void k_fftx_inv_r(Geo g, const cpx<T> *__restri
     {
         const int p = threadIdx.x % G::LPW;
         cpx<T> *zl = lds + p * G::LS;
-        for (int kx = threadIdx.x / G::LPW; kx < g.H; kx += 64 / G::LPW) {
-            cpx<T> A = spec[six(g, J, kx, k0 + 2 * p)], B = spec[six(g, J, kx, k0 + 2 * p + 1)];
+        auto put = [&](int kx, cpx<T> A, cpx<T> B) {
             if (kx == 0 || kx == L / 2) { A.y = T(0); B.y = T(0); }
             zl[chs::rpad<G::PS>(kx)] = {A.x - B.y, A.y + B.x};
             if (kx > 0 && kx < L / 2) zl[chs::rpad<G::PS>(L - kx)] = {A.x + B.y, B.x - A.y};
+        };
+        constexpr int ST = 64 / G::LPW, U = 5;   // the five loads of each plane that 8 points a lane make
+        for (int kb = threadIdx.x / G::LPW; kb < g.H; kb += U * ST) {
+            cpx<T> A[U], B[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const size_t o = six(g, J, min(kb + u * ST, g.H - 1), k0 + 2 * p);
+                A[u] = spec[o];
+                B[u] = spec[o + 1];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (kb + u * ST < g.H) put(kb + u * ST, A[u], B[u]);
         }
     }
     chs::wave_lds_sync();
@@ -2343,8 +2364,10 @@ __global__ __launch_bounds__(1024) void k_spec_plane(Geo g, chs::GPlan P, const 
 // x forward: block = row J and TK consecutive z-planes (a plane pair per line; planes past N - 1
 // of the last block have no line).  TK = 16 or 8 gives spec runs of 256 or 128 bytes per kx; a
 // block's lines take 20 to 37 KB of LDS and its threads at most 128 VGPRs, so four blocks share a
-// CU.  512x192x512: 348 us (4.6 TB/s) against 562 of the register plan's 32-byte runs.
-template <typename T>
+// CU.  512x192x512: 349 us (4.6 TB/s) against 552 of the register plan's 32-byte runs.  MODE 0: the
+// divergence of q; 1: also stored to div; 2: the field src (no branch between two points' loads:
+// 96x80x96 14 -> 12.5 us).
+template <typename T, int MODE>
 __global__ __launch_bounds__(256, 4) void k_divg_fftx_g(Geo g, chs::GPlan P, const cpx<T> *__restrict__ tw,
                                                         const double *__restrict__ dv, double talp,
                                                         const double *__restrict__ q, double *__restrict__ div,
@@ -2370,13 +2393,13 @@ __global__ __launch_bounds__(256, 4) void k_divg_fftx_g(Geo g, chs::GPlan P, con
     chs::gfft_lines<T, -1, false, true>(
         P, line, j, act, tw,
         [&](int i) -> cpx<T> {
-            if (src) return {(T)src[c0 + i], (T)src[c1 + i]};
+            if constexpr (MODE == 2) return {(T)src[c0 + i], (T)src[c1 + i]};
             const int ip = (i == L - 1) ? 0 : i + 1;
             const double wm = w[ps + i];
             const double d0 = divg_cell(u[ip], u[i], v[L + i], v[i], wm, w[i], g.dxi, dyf, g.dzi) * coe0;
             const double d1 = divg_cell(u[ps + ip], u[ps + i], v[ps + L + i], v[ps + i], w2[i], wm, g.dxi, dyf,
                                         g.dzi) * coe0;
-            if (div) {
+            if constexpr (MODE == 1) {
                 div[c0 + i] = d0;
                 div[c1 + i] = d1;
             }
@@ -2399,7 +2422,8 @@ __global__ __launch_bounds__(256, 4) void k_divg_fftx_g(Geo g, chs::GPlan P, con
 }
 
 // x inverse: Hermitian extension of the plane pair of each line, complex inverse transform,
-// real parts to the solution rows (PhiOut).
+// real parts to the solution rows (PhiOut).  512x192x512 208 us (221 with one load of each plane in
+// flight at a time), 96x80x96 9 (10).
 template <typename T>
 __global__ __launch_bounds__(256, 4) void k_fftx_inv_g(Geo g, chs::GPlan P, const cpx<T> *__restrict__ tw,
                                                        const cpx<T> *__restrict__ spec, PhiOut out, int TK)
@@ -2410,13 +2434,24 @@ __global__ __launch_bounds__(256, 4) void k_fftx_inv_g(Geo g, chs::GPlan P, cons
     {
         const int np = TK / 2, sh = 31 - __builtin_clz(np), p = threadIdx.x & (np - 1);
         cpx<T> *zl = lds + p * P.ls;
+        const int st = blockDim.x >> sh;
         if (k0 + 2 * p < N)
-            for (int kx = threadIdx.x >> sh; kx < g.H; kx += blockDim.x >> sh) {
-                cpx<T> A = spec[six(g, J, kx, k0 + 2 * p)], B = spec[six(g, J, kx, k0 + 2 * p + 1)];
-                const int kc2 = L - kx;
-                if (kx == 0 || kx == L / 2) { A.y = T(0); B.y = T(0); }
-                zl[kx + (kx >> P.ps)] = {A.x - B.y, A.y + B.x};
-                if (kx > 0 && kx < L / 2) zl[kc2 + (kc2 >> P.ps)] = {A.x + B.y, B.x - A.y};
+            for (int kb = threadIdx.x >> sh; kb < g.H; kb += 4 * st) {   // four loads of each plane in flight
+                cpx<T> A[4], B[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const size_t o = six(g, J, min(kb + u * st, g.H - 1), k0 + 2 * p);
+                    A[u] = spec[o];
+                    B[u] = spec[o + 1];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int kx = kb + u * st, kc2 = L - kx;
+                    if (kx >= g.H) break;
+                    if (kx == 0 || kx == L / 2) { A[u].y = T(0); B[u].y = T(0); }
+                    zl[kx + (kx >> P.ps)] = {A[u].x - B[u].y, A[u].y + B[u].x};
+                    if (kx > 0 && kx < L / 2) zl[kc2 + (kc2 >> P.ps)] = {A[u].x + B[u].y, B[u].x - A[u].y};
+                }
             }
     }
     __syncthreads();
@@ -3796,15 +3831,15 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
     //        (N = 120: 20 / - / 13);
     //  x     register plan where L has one, except where mixed radix is faster: L >= 512, whose plan
     //        holds one line, so two planes or 32-byte runs of the spectrum, per wavefront
-    //        (512x192x512 forward 520 / 562 / 348, inverse 340 / 270 / 221; the FP32 inverse 188 /
-    //        164 / 182 keeps the plan), and the FP64 forward transform with the divergence of
-    //        L = 128 (128x96x128: 22.3 / 22.3 / 17.2; of a given field the plan is faster); else mixed
+    //        (512x192x512 forward 520 / 552 / 349, inverse 340 / 263 / 208; FP32 inverse
+    //        188 / 162 / 145), and the FP64 forward transform with the divergence of L = 128
+    //        (128x96x128: 22.3 / 19.9 / 17.0; of a given field the plan is faster); else mixed
     //        radix (144x103x180 forward 48 / - / 29, inverse 35 / - / 17).
     // The LDS transforms remain for lengths with no plan of two or three passes of at most 256
     // threads a line, for fft_reg = 0 and for the batched ensemble.
     const bool f64 = sizeof(T) == 8, fr = c->tune.fft_reg != 0, gxok = c->gtwx && c->gtwxi;
     const bool rx = fr && c->rtwx && !(gxok && (L >= 512 || (f64 && L == 128 && !src)));
-    const bool rxi = fr && c->rtwx && !(gxok && f64 && L >= 512);
+    const bool rxi = fr && c->rtwx && !(gxok && L >= 512);
     const bool rz = fr && c->rtwz;
     const bool mx = fr && !rx && gxok, mxi = fr && !rxi && gxok, mz = fr && !rz && c->gtwz;
     const int TKR = 2 * (c->rtwx ? chs::rplan_lpw(L) : 1), LPZ = rz ? chs::rplan_lpw(N) : 1;
@@ -3824,9 +3859,9 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
             divg_fftx_r<T>(L, dim3(M, N / TKR), c->stream, g, (const cpx<T> *)c->rtwx, dv, talp, qv, dvo, spec, src,
                            c->tune.divg_nxcd);
         else if (mx)
-            hipLaunchKernelGGL(k_divg_fftx_g<T>, gxg, dim3(block_threads(TKG / 2 * c->gx.tpl)),
-                               sizeof(cpx<T>) * (TKG / 2) * c->gx.ls, c->stream, g, c->gx, (const cpx<T> *)c->gtwx, dv,
-                               talp, qv, dvo, spec, src, TKG, c->tune.divg_nxcd);
+            hipLaunchKernelGGL((src ? k_divg_fftx_g<T, 2> : dvo ? k_divg_fftx_g<T, 1> : k_divg_fftx_g<T, 0>), gxg,
+                               dim3(block_threads(TKG / 2 * c->gx.tpl)), sizeof(cpx<T>) * (TKG / 2) * c->gx.ls, c->stream,
+                               g, c->gx, (const cpx<T> *)c->gtwx, dv, talp, qv, dvo, spec, src, TKG, c->tune.divg_nxcd);
         else
             hipLaunchKernelGGL(k_divg_fftx<T>, dim3(M, N / TK), dim3(256), shx, c->stream, g, pa, dv, talp, qv, dvo,
                                spec, TK, src);
