@@ -3727,10 +3727,11 @@ int gz_lines(const chs::GPlan &P, size_t cs, int lines)
 // with the least rounds x (planes + 2), the longest of equals.  256x192x256 52 planes (240 blocks in one
 // round, 6 % fewer plane loads than 16 planes in three: 285 -> 250 us, FP32 189 -> 182); 64x64x64
 // 4 (34 -> 17 us with 256 blocks in place of 64); 144x103x180 20 (118 -> 83 us with 234 blocks in
-// place of 312).
+// place of 312).  A CU holds four blocks of one wavefront's width within 128 VGPRs, three of the FP32
+// kernel's on whole tiles (167 VGPRs; counted as two, 64x192x256 marched 26 planes in 61 us, where 16 take 50).
 int conv_march(int M, int N, int bxw, int waves)
 {
-    const long long cap = 256LL * (waves == 4 ? (bxw == 1 ? 4 : 2) : (bxw == 1 ? 2 : 1));
+    const long long cap = 256LL * (waves == 4 ? (bxw == 1 ? 4 : 2) : (bxw == 1 ? 3 : 1));
     const long long rows = (M + 3) / 4;
     int best = 4;
     long long cost = -1;

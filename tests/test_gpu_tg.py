@@ -511,3 +511,27 @@ def test_fp32_wide_ytdma_changes_no_bit(pkg, L, M, N):
         out.append(ch.download())
         ch.close()
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("L,M,N,mode", [(64, 192, 256, "mixed"), (64, 160, 256, "mixed"), (64, 64, 64, "plain")])
+def test_convection_march_by_mesh_is_near_the_best(pkg, L, M, N, mode):
+    """The planes per march that the mesh chooses: within 12 % of the fastest of a few set by hand
+    (kernel times; a march too long for the blocks a CU holds cost 23 % at 64x192x256)."""
+    ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=1.8), pkg.MIXED if mode == "mixed" else pkg.PLAIN_FP64)
+    ch.upload(*oracle.initial_field(setup.Mesh(L, M, N, STR2=1.8), 3))
+
+    def kernel_ms():
+        for _ in range(3):
+            ch.rk3_step(5.0e-4, 1.0 / 2800.0)
+        ch.profile_reset("conv_rhs")
+        for _ in range(20):
+            ch.rk3_step(5.0e-4, 1.0 / 2800.0)
+        return ch.profile_get("conv_rhs")[0]
+
+    auto, by_hand = kernel_ms(), {}
+    for kc in (4, 8, 16, 26):
+        ch.set_tuning(conv_kc=kc)
+        by_hand[kc] = kernel_ms()
+    print(f"  by the mesh {auto:.4f} ms, by hand {by_hand}")
+    assert auto < 1.12 * min(by_hand.values())
+    ch.close()
