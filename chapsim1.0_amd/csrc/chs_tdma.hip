@@ -11,6 +11,7 @@
 #include <string>
 
 #include "../../include/chapsim_hip.h"
+#include "chs_tdma_rule.h"
 
 namespace {
 
@@ -207,7 +208,8 @@ __global__ __launch_bounds__(64, 1) void k_tdma_lines_ck(int n, int nl, const do
     }
 }
 
-// The launch for lines of n points (at most 1280: 157 KB of LDS); false: longer lines.
+// The launch for lines of n points (at most 1280: 157 KB of LDS); false: longer lines, and the batches
+// that chs_tdma_rule.h leaves to k_tdma_lines (alloc: its work array would be allocated).
 template <int NCH>
 void launch_ck(int kind, int n, int nl, const double *a, const double *b, const double *c, double *r, const double *bc)
 {
@@ -217,16 +219,18 @@ void launch_ck(int kind, int n, int nl, const double *a, const double *b, const 
     else if (kind == 2) hipLaunchKernelGGL((k_tdma_lines_ck<false, true, NCH>), g, t, 0, 0, n, nl, a, b, c, r, bc);
     else hipLaunchKernelGGL((k_tdma_lines_ck<true, false, NCH>), g, t, 0, 0, n, nl, a, b, c, r, bc);
 }
-bool tdma_ck(int kind, int n, int nl, const double *a, const double *b, const double *c, double *r, const double *bc)
+bool tdma_ck(int kind, int n, int nl, const double *a, const double *b, const double *c, double *r, const double *bc,
+             bool alloc)
 {
+    if (chs::tdma_thread_per_line(kind, n, nl, alloc)) return false;
     if (n <= 20 * kCk) launch_ck<20>(kind, n, nl, a, b, c, r, bc);        // 65 KB: two blocks on a CU
     else if (n <= 80 * kCk) launch_ck<80>(kind, n, nl, a, b, c, r, bc);
     else return false;
     return true;
 }
 
-// Lines longer than k_tdma_lines_ck's, one thread per line.  work: 3 n doubles per line, element-major
-// ([i][line]) so that consecutive lines coalesce.
+// The other batches (lines longer than k_tdma_lines_ck's, and short ones), one thread per line.  work:
+// 3 n doubles per line, element-major ([i][line]) so that consecutive lines coalesce.
 __global__ __launch_bounds__(256) void k_tdma_lines(int kind, int isz, int jsz, const double *__restrict__ A,
                                                     const double *__restrict__ B, const double *__restrict__ C,
                                                     double *__restrict__ R, const double *__restrict__ bc,
@@ -340,7 +344,7 @@ int chs_tdma_lines(int kind, int isz, int jsz, const double *a, const double *b,
     }
     double *work = nullptr;
     hipError_t e = hipSuccess;
-    if (tdma_ck(kind, n, nl, a, b, c, r, bc)) {
+    if (tdma_ck(kind, n, nl, a, b, c, r, bc, true)) {
         e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(0);
     } else if ((e = hipMalloc(&work, sizeof(double) * 3 * (size_t)n * nl)) == hipSuccess) {
@@ -378,7 +382,7 @@ int chs_tdma_lines_noalloc(int kind, int isz, int jsz, const double *a, const do
     // every work entry a line reads was written earlier by the same line: nothing to clear
     double *work = nullptr;
     hipError_t e = hipSuccess;
-    if (tdma_ck(kind, n, nl, a, b, c, r, bc)) {
+    if (tdma_ck(kind, n, nl, a, b, c, r, bc, false)) {
         e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(0);
     } else if ((e = scratch_ptr(&work)) == hipSuccess) {
