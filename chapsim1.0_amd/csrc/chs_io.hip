@@ -1274,6 +1274,15 @@ __device__ __forceinline__ void io_cn_z_line(const IoDev &d, int l, double facoe
     thomas_cyc(N, coef, rhs, out, Wk, Wk + cs, Wk + 2 * cs, (size_t)nl);
 }
 
+template <typename W>
+__global__ __launch_bounds__(128) void k_io_cn_z(IoDev d, double facoe)
+{
+    const int l = blockIdx.x * 128 + threadIdx.x;
+    if (blockIdx.y == 0) io_cn_z_line<0, W>(d, l, facoe);
+    else if (blockIdx.y == 1) io_cn_z_line<1, W>(d, l, facoe);
+    else io_cn_z_line<2, W>(d, l, facoe);
+}
+
 // MOMFA3_Y_io (MOMFA_io.f90:268-406): y-lines over rows 1..M with zero boundary values, then
 // G = increment + G0 for rows N2I..M (MOMFA_io.f90:38-44) with BC_WALL_G_io: every row of the
 // line's new G.  u, w: the wall rows' viscosity is the mean of the wall cell and its ghost in
@@ -1772,6 +1781,7 @@ struct chs_io {
     int props_kc = 4;   // z-planes per block of the LDS-staged staggered properties (0: per-point kernel; 4
                         // against 16: 256x128x256 252 and 256 us, 90x71x120 22 and 29)
     int cnz_cols = 0, cny_cols = 0;   // cn_cols for the z or the y solve alone (0: cn_cols)
+    double ymax = 0.0;                // largest (AMVR + APVR) / 2
     int cnz_p = 8, cny_p = 8;         // line points per thread of the z and y solves (4 or 8; 8:
                                       // 6.21 -> 6.09 (z) and 6.14 (y) ms per heated CN step)
     int cnx_wave = 1;     // x-lines of the Crank-Nicolson solve one per wavefront (L = 64, 128, 256, 512)
@@ -1900,6 +1910,8 @@ int chs_io_create(const chs_coeffs *c, const chs_io_params *p, chs_io **out)
         d.amvr1 = ucaj * (2.0 * c->dyfi[0]);
         ucaj = 4.0 / (2.0 / c->dyci[M - 1] + 1.0 / c->dyfi[M - 1]);
         d.apvrn = ucaj * (2.0 * c->dyfi[M - 1]);
+        for (int r = 0; r < 3; ++r)
+            for (int J = 1; J <= M; ++J) m->ymax = std::max(m->ymax, 0.5 * (ha[r * (M + 2) + J] + ha[na + r * (M + 2) + J]));
     }
     d.dxqi = c->dxqi; d.dzqi = c->dzqi;
     d.L = L; d.M = M; d.N = N;
@@ -2134,13 +2146,23 @@ void io_momentum_launch(chs_io *m, const double *gs, double tg, double tr, doubl
         // here (each reads Q, the properties and its own increment), so they run side by side.
         const double facoe = 0.5 * ta * dt * d.cvisc;
         const int L = m->L, M = m->M, N = m->N;
+        // Lines that a wavefront or a padded block solves (L no power of two, z and y blocks that are not
+        // whole wavefronts) go to one thread per line where the sweeps would not be used: a line
+        // handed over inside such a block has at most 16 lanes of a wavefront, one in x
+        // (rho > 1/4 at 90x71x120, all three directions: 395 us of one thread per line, 1346 handed over).
+        // The host's estimate of rho = 2 lam / (1 + 2 lam) takes viscosity / density as 4 times the
+        // reference state's, so that few lines are handed over below it; above it 15 sweeps and more still
+        // gain a little (90x71x120 at lam = 1/20 on the walls alone 223 us against 279).
+        auto sweeps = [&](double coe) { return facoe * (4.0 / 3.0) * coe <= 1.0 / 24.0; };
+        auto padded = [](int T, int NT) { return T < 64 / std::gcd(NT, 64); };
         // x: one wavefront per line where L is a multiple n P of at most 64 lanes (the fewest points
         // per lane); else a block per line for powers of two, else a thread per line
         int PX = 0;
         if (m->cnx_wave && L <= 640)
             for (int q : {1, 2, 3, 4, 5, 6, 8, 9, 10})
                 if (PX == 0 && L % q == 0 && L / q <= 64) PX = q;
-        if (PX && !(L < 32 && (L & (L - 1)) == 0)) {
+        const bool pow2 = (L & (L - 1)) == 0;
+        if (PX && !(pow2 ? L < 32 : !sweeps(d.dxqi))) {
             const dim3 gx((M * N + 3) / 4, 3);
 #define CHS_IOX(q) \
     case q: \
@@ -2151,7 +2173,7 @@ void io_momentum_launch(chs_io *m, const double *gs, double tg, double tr, doubl
                 CHS_IOX(1) CHS_IOX(2) CHS_IOX(3) CHS_IOX(4) CHS_IOX(5) CHS_IOX(6) CHS_IOX(8) CHS_IOX(9) CHS_IOX(10)
             }
 #undef CHS_IOX
-        } else if ((L & (L - 1)) == 0 && L >= 4 && L <= 512) {
+        } else if (pow2 && L >= 4 && L <= 512) {
             const int T = L >= 256 ? 1 : 256 / L;   // x-lines per block
             hipLaunchKernelGGL(k_io_cn_x_jac<W>, dim3((M * N + T - 1) / T, 3), dim3(T * L),
                                sizeof(double) * (2 * T * L + 1), m->stream, d, dpg_dev, dpg, facoe);
@@ -2160,10 +2182,13 @@ void io_momentum_launch(chs_io *m, const double *gs, double tg, double tr, doubl
                                facoe);
         }
         // z and y: T x-columns by NT chunks of P line points per thread (4 or 8), rounded up to whole
-        // wavefronts; N <= 2048 leaves z at most 512 chunks
+        // wavefronts; N <= 2048 leaves z at most 512 chunks.  Lines of more than 1024 chunks: a thread per line.
         const int Pz = m->cnz_p, Py = m->cny_p;
-        {
-            const int NT = (N + Pz - 1) / Pz, T = std::min(m->cnz_cols ? m->cnz_cols : m->cn_cols, 1024 / NT);
+        const int NTz = (N + Pz - 1) / Pz, Tz = std::min(m->cnz_cols ? m->cnz_cols : m->cn_cols, 1024 / NTz);
+        if ((N % Pz || NTz < 2 || padded(Tz, NTz)) && !sweeps(d.dzqi)) {
+            hipLaunchKernelGGL(k_io_cn_z<W>, dim3((M * L + 127) / 128, 3), dim3(128), 0, m->stream, d, facoe);
+        } else {
+            const int NT = NTz, T = Tz;
             const int S = (T * NT + 63) / 64 * 64;
             const dim3 gz((L + T - 1) / T * M, 3), bz(S);
             const size_t sz = sizeof(double) * (4 * S + 1);
@@ -2181,9 +2206,9 @@ void io_momentum_launch(chs_io *m, const double *gs, double tg, double tr, doubl
 #undef CHS_IOZ
             }
         }
-        const int NTy = (M + Py - 1) / Py;
-        if (NTy <= 1024) {
-            const int Ty = std::min(m->cny_cols ? m->cny_cols : m->cn_cols, 1024 / NTy), S = (Ty * NTy + 63) / 64 * 64;
+        const int NTy = (M + Py - 1) / Py, Ty = NTy <= 1024 ? std::min(m->cny_cols ? m->cny_cols : m->cn_cols, 1024 / NTy) : 0;
+        if (Ty > 0 && !(padded(Ty, NTy) && !sweeps(m->ymax))) {
+            const int S = (Ty * NTy + 63) / 64 * 64;
             const int ng = (L + Ty - 1) / Ty;
             const dim3 gy(ng * N, 3), by(S);
             const size_t sy = sizeof(double) * (4 * S + 1 + 2 * (M + 2));

@@ -622,3 +622,63 @@ def test_gpu_cn_ragged_line_solves(pkg, L, M, N, kv):
             assert rel(f[k][c], o.f[k][c]) < 1e-11, (k, c, rel(f[k][c], o.f[k][c]))
     assert rel(f["PR"], o.f["PR"]) < 1e-10, rel(f["PR"], o.f["PR"])
     ch.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,M,N,kv", [(36, 18, 30, {}), (90, 9, 20, {}), (54, 13, 50, dict(cnz_p=4, cny_p=4)), (150, 6, 36, {}),
+                                      (36, 17, 20, dict(cn_cols=1))])
+@pytest.mark.parametrize("REN,dt,visc", [(1.0, 0.5, 1.0), (400.0, 0.5, 400.0), (400.0, 0.02, 400.0)])
+def test_gpu_cn_ragged_line_regimes(pkg, L, M, N, kv, REN, dt, visc):
+    """test_gpu_cn_line_solve_regimes on padded blocks and short wavefronts.  REN = 1: the host's
+    estimate of rho sends every direction to one thread per line; REN = 400 with 400 times the
+    viscosity: rho is the same, the estimate is small, and the line kernels hand over blocks
+    with rho > 1/4 themselves (dt = 0.02: the walls' alone).  Momentum part against the oracle."""
+    print(f"io cn ragged regimes {L}x{M}x{N} {kv} REN {REN} dt {dt}", flush=True)
+    mesh = setup.Mesh(L, M, N, STR2=2.0)
+    st = oracle.io_initial_field(mesh, 95)
+    m1 = visc * cn_viscosity(st, 95, False)
+    o = oracle.OracleIO(mesh, REN, flow_driven=1, vis_scheme=1)
+    o.set_state(dict(st, M1=m1))
+    o.props(1)
+    o.momentum_cn(1, dt)
+    ch = pkg.ChannelIO(pkg.channel_setup(L, M, N, STR2=2.0), REN, flow_driven=1, vis_scheme=1)
+    ch.set_tuning(**kv)
+    ch.upload(**st, M1=m1)
+    ch.ioprops(1)
+    ch.momentum(1, dt)
+    f = ch.download()
+    for c in range(3):
+        assert rel(f["G"][c], o.f["G"][c]) < TOL, (c, rel(f["G"][c], o.f["G"][c]))
+    ch.close()
+
+
+@pytest.mark.gpu
+def test_gpu_cn_stiff_lines_keep_their_lanes(pkg):
+    """Where no line can be solved by sweeps (REN = 1, dt = 0.5) a ragged mesh takes the kernels with a
+    thread per line: at most 5 times a small step's time (2.6 on MI355X; 9.5 with the lines handed
+    over inside padded blocks)."""
+    import time
+    L, M, N = 90, 71, 120
+    co = pkg.channel_setup(L, M, N, STR2=1.8)
+    rng = np.random.default_rng(1)
+    prop = 1.0 + 0.01 * rng.random((N, M + 2, L))
+    G = np.zeros((3, N, M + 2, L))
+    G[0, :, 1:M + 1] = 1.0 + 0.05 * rng.standard_normal((N, M, L))
+    took = []
+    for REN, dt in ((2800.0, 1e-3), (1.0, 0.5)):
+        ch = pkg.ChannelIO(co, REN, flow_driven=1, vis_scheme=1)
+        ch.upload(G=G, PR=np.zeros_like(prop), D0=prop, M0=prop, M1=prop)
+        ch.ioprops(1)
+        ch.momentum(1, dt)
+        ch.sync()
+        best = 1.0
+        for _ in range(5):
+            t0 = time.perf_counter()
+            for _ in range(5):
+                ch.momentum(1, dt)
+            ch.sync()
+            best = min(best, time.perf_counter() - t0)
+        took.append(best / 5)
+        ch.close()
+    print(f"  sweeps {1e6 * took[0]:.0f} us, thread per line {1e6 * took[1]:.0f} us")
+    assert took[1] < 5.0 * took[0]
