@@ -2039,6 +2039,20 @@ int chs_io_set_tuning(chs_io *m, const char *key, int value)
 {
     if (!m || !key) return io_fail(m, CHS_E_ARG, "chs_io_set_tuning: bad argument");
     const std::string k(key);
+    if (value == CHS_TUNE_DEFAULT) {
+        const struct {
+            const char *key;
+            int chs_io::*field;
+        } keys[] = {{"mom_rows", &chs_io::mom_rows}, {"mom_kz", &chs_io::mom_kz}, {"props_kc", &chs_io::props_kc},
+                    {"mom_nxcd", &chs_io::mom_nxcd}, {"mom_by", &chs_io::mom_by}, {"cnz_p", &chs_io::cnz_p},
+                    {"cny_p", &chs_io::cny_p}, {"cnz_cols", &chs_io::cnz_cols}, {"cny_cols", &chs_io::cny_cols},
+                    {"cn_fastdiv", &chs_io::cn_fastdiv}, {"cnx_wave", &chs_io::cnx_wave}, {"cn_cols", &chs_io::cn_cols}};
+        for (const auto &t : keys)
+            if (k == t.key) {
+                m->*t.field = chs_io().*t.field;
+                return CHS_OK;
+            }
+    }
     if (k == "mom_rows") {
         if (value != 1 && value != 2 && value != 4) return io_fail(m, CHS_E_ARG, "chs_io_set_tuning: mom_rows must be 1, 2 or 4");
         m->mom_rows = value;

@@ -3273,6 +3273,51 @@ struct CnTab {
     void *gx = nullptr, *gz = nullptr, *by[3] = {nullptr, nullptr, nullptr};
 };
 
+// Launch shapes (chs_set_tuning); 0 = derived from the mesh
+// (defaults: the fastest shapes on MI355X for a 256 x 192 x 256 channel; cnx_nlx 0 means
+// 2048 / L lines)
+struct Tune {
+    int conv_by = 4, conv_kc = 0;   // k_conv_rhs rows per block, z-planes per thread (0: by the mesh)
+    int conv_bx = 1;                // k_conv_rhs wavefronts along x per block (1 or 4)
+    int conv_fence = 0;             // 1: all of a plane's loads stay ahead of its arithmetic
+    int cnx_nlx = 0;                // k_cn_x lines per block
+    int cnz_kz = 16, cny_ky = 48;   // march lengths of the z and y CN stencils (FP64)
+    int fftx_tk = 0, fftz_nl = 0;   // z-planes per x-transform block, z-lines per block
+    int nxcd = 1;                   // XCDs the stencil tiles are grouped for (1 = off)
+    int fft_reg = 1;                // register FFTs where L / N have a plan (0 = LDS Stockham)
+    int cn_xz = 0, cnxz_by = 1;     // fused x+z CN kernel (1; slower on MI355X), rows per block
+    int conv_fx = 1;                // x-solve inside k_conv_rhs (rows per block; 0 = off)
+    int ytdma_bs = 64, ytdma_rb = 16;   // k_ytdma threads per block, rows per load batch
+    int ytdma_c = -1;                   // k_ytdma_chunk rows per chunk (-1 auto = 16, 0 = k_ytdma)
+    int conv_lds = 2;                   // k_conv_rhs_lds rows per block (1, 2, 4; 0 = k_conv_rhs)
+    int conv_dma = 4;                   // k_conv_rhs_dma rows per block (2, 4; 0 = k_conv_rhs_lds)
+    int divg_nxcd = 8;                  // XCDs the k_divg_fftx_r rows are grouped for (1 = off)
+    int cny3_ky = -2;                   // k_cn_y3_march rows per chunk (-2 by the mesh; 0 = M; -1 = one launch per component)
+    int upd_kz = 0;                     // k_update z-planes per thread (0: by the mesh)
+    int upd_by = 4;                     // k_update rows per block (1, 2, 4, 8, 16)
+    int upd_nxcd = 1;                   // k_update tiles grouped for this many XCDs (1: launch order;
+                                        // 8 measured equal at 256x192x256)
+    int upd_w2 = 1;                     // k_update2 (two points per lane) where L % 128 == 0 (0 = k_update)
+    int cnzy = -1;                      // z and y solves fused (k_cn_zy_march): -1 by the mesh, 1 where
+                                        // L % 64 == 0 and N % 16 == 0, 2 on every mesh, 0 = two kernels
+    int cnzy_ky = -1;                   // k_cn_zy_march rows per chunk (-1 by the mesh; 0 = M)
+    int cnzy_nxcd = 8;                  // k_cn_zy_march tiles grouped for this many XCDs
+};
+const struct {
+    const char *key;
+    int Tune::*field;
+} kTuneKeys[] = {
+    {"conv_by", &Tune::conv_by}, {"conv_kc", &Tune::conv_kc}, {"conv_bx", &Tune::conv_bx},
+    {"conv_fence", &Tune::conv_fence}, {"cnx_nlx", &Tune::cnx_nlx}, {"cnz_kz", &Tune::cnz_kz},
+    {"cny_ky", &Tune::cny_ky}, {"fftx_tk", &Tune::fftx_tk}, {"fftz_nl", &Tune::fftz_nl}, {"nxcd", &Tune::nxcd},
+    {"fft_reg", &Tune::fft_reg}, {"cn_xz", &Tune::cn_xz}, {"cnxz_by", &Tune::cnxz_by}, {"conv_fx", &Tune::conv_fx},
+    {"ytdma_bs", &Tune::ytdma_bs}, {"ytdma_rb", &Tune::ytdma_rb}, {"ytdma_c", &Tune::ytdma_c},
+    {"conv_lds", &Tune::conv_lds}, {"conv_dma", &Tune::conv_dma}, {"divg_nxcd", &Tune::divg_nxcd},
+    {"cny3_ky", &Tune::cny3_ky}, {"upd_kz", &Tune::upd_kz}, {"upd_by", &Tune::upd_by},
+    {"upd_nxcd", &Tune::upd_nxcd}, {"upd_w2", &Tune::upd_w2}, {"cnzy", &Tune::cnzy}, {"cnzy_ky", &Tune::cnzy_ky},
+    {"cnzy_nxcd", &Tune::cnzy_nxcd},
+};
+
 }  // namespace
 
 struct chs_ctx {
@@ -3306,36 +3351,7 @@ struct chs_ctx {
     void *gtw = nullptr, *gtwx = nullptr, *gtwxi = nullptr, *gtwz = nullptr;   // their twiddles (null: not served)
     chs::FftPlan px, pz;
     CnTab cn[4];
-    // launch shapes (chs_set_tuning); 0 = derived from the mesh
-    // (defaults: the fastest shapes on MI355X for a 256 x 192 x 256 channel; cnx_nlx 0 means
-    // 2048 / L lines)
-    struct {
-        int conv_by = 4, conv_kc = 0;   // k_conv_rhs rows per block, z-planes per thread (0: by the mesh)
-        int conv_bx = 1;                // k_conv_rhs wavefronts along x per block (1 or 4)
-        int conv_fence = 0;             // 1: all of a plane's loads stay ahead of its arithmetic
-        int cnx_nlx = 0;                // k_cn_x lines per block
-        int cnz_kz = 16, cny_ky = 48;   // march lengths of the z and y CN stencils (FP64)
-        int fftx_tk = 0, fftz_nl = 0;   // z-planes per x-transform block, z-lines per block
-        int nxcd = 1;                   // XCDs the stencil tiles are grouped for (1 = off)
-        int fft_reg = 1;                // register FFTs where L / N have a plan (0 = LDS Stockham)
-        int cn_xz = 0, cnxz_by = 1;     // fused x+z CN kernel (1; slower on MI355X), rows per block
-        int conv_fx = 1;                // x-solve inside k_conv_rhs (rows per block; 0 = off)
-        int ytdma_bs = 64, ytdma_rb = 16;   // k_ytdma threads per block, rows per load batch
-        int ytdma_c = -1;                   // k_ytdma_chunk rows per chunk (-1 auto = 16, 0 = k_ytdma)
-        int conv_lds = 2;                   // k_conv_rhs_lds rows per block (1, 2, 4; 0 = k_conv_rhs)
-        int conv_dma = 4;                   // k_conv_rhs_dma rows per block (2, 4; 0 = k_conv_rhs_lds)
-        int divg_nxcd = 8;                  // XCDs the k_divg_fftx_r rows are grouped for (1 = off)
-        int cny3_ky = -2;                   // k_cn_y3_march rows per chunk (-2 by the mesh; 0 = M; -1 = one launch per component)
-        int upd_kz = 0;                     // k_update z-planes per thread (0: by the mesh)
-        int upd_by = 4;                     // k_update rows per block (1, 2, 4, 8, 16)
-        int upd_nxcd = 1;                   // k_update tiles grouped for this many XCDs (1: launch order;
-                                            // 8 measured equal at 256x192x256)
-        int upd_w2 = 1;                     // k_update2 (two points per lane) where L % 128 == 0 (0 = k_update)
-        int cnzy = -1;                      // z and y solves fused (k_cn_zy_march): -1 by the mesh, 1 where
-                                            // L % 64 == 0 and N % 16 == 0, 2 on every mesh, 0 = two kernels
-        int cnzy_ky = -1;                   // k_cn_zy_march rows per chunk (-1 by the mesh; 0 = M)
-        int cnzy_nxcd = 8;                  // k_cn_zy_march tiles grouped for this many XCDs
-    } tune;
+    Tune tune, tune_default;   // tune_default: as the context was made
     int tune_gen = 0;   // bumped by every chs_set_tuning / chs_set_refinement (graphs are re-made)
     int cn_gen = 0;     // bumped by every rebuild of a Crank-Nicolson table (its memory may move)
     bool have_fields = false;
@@ -4537,6 +4553,7 @@ static int create_impl(const chs_coeffs *cf, int mode, hipStream_t shared, chs_c
         e = (mode == CHS_MIXED) ? upload_rtw<float>(c, N, &c->rtwz) : upload_rtw<double>(c, N, &c->rtwz);
     if (e) return bad(e);
 #undef CK
+    c->tune_default = c->tune;
     *out = c;
     return 0;
 }
@@ -4809,7 +4826,15 @@ int chs_set_tuning(chs_ctx *c, const char *key, int value)
     const std::string k(key);
     const int L = c->L, M = c->M, N = c->N;
     auto bad = [&](const char *why) { return fail(c, CHS_E_ARG, "chs_set_tuning " + k + ": " + why); };
-    if (k == "conv_by") {
+    if (value == CHS_TUNE_DEFAULT) {   // every pair of defaults satisfies the limits between keys
+        bool known = false;
+        for (const auto &t : kTuneKeys)
+            if (k == t.key) {
+                c->tune.*t.field = c->tune_default.*t.field;
+                known = true;
+            }
+        if (!known) return bad("unknown key");
+    } else if (k == "conv_by") {
         if (value != 1 && value != 2 && value != 4 && value != 8 && value != 16) return bad("must be 1, 2, 4, 8 or 16");
         if (c->tune.conv_bx * value > 16) return bad("conv_bx * conv_by must be <= 16");
         c->tune.conv_by = value;

@@ -881,7 +881,10 @@ int chs_eng_set_tuning(chs_eng *e, const char *key, int value)
 {
     if (!e || !key) return eng_fail(e, CHS_E_ARG, "chs_eng_set_tuning: bad argument");
     const std::string k(key);
-    if (k == "rhs_lds" && (value == 0 || value == 1)) e->rhs_lds = value;
+    if (value == CHS_TUNE_DEFAULT && k == "rhs_lds") e->rhs_lds = chs_eng().rhs_lds;
+    else if (value == CHS_TUNE_DEFAULT && k == "rhs_kc") e->rhs_kc = chs_eng().rhs_kc;
+    else if (value == CHS_TUNE_DEFAULT && k == "rhs_nxcd") e->rhs_nxcd = chs_eng().rhs_nxcd;
+    else if (k == "rhs_lds" && (value == 0 || value == 1)) e->rhs_lds = value;
     else if (k == "rhs_kc" && value >= 1 && value <= 1024) e->rhs_kc = value;
     else if (k == "rhs_nxcd" && value >= 1 && value <= 64) e->rhs_nxcd = value;
     else return eng_fail(e, CHS_E_ARG, "chs_eng_set_tuning: unknown key or value out of range (" + k + ")");

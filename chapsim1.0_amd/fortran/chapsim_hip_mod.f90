@@ -15,6 +15,7 @@ MODULE chapsim_hip
     INTEGER(C_INT), PARAMETER :: CHS_OK = 0
     INTEGER(C_INT), PARAMETER :: CHS_PLAIN_FP64 = 0
     INTEGER(C_INT), PARAMETER :: CHS_MIXED = 1
+    INTEGER(C_INT), PARAMETER :: CHS_TUNE_DEFAULT = -1000000   ! a tuning key's default
 
     ! mirror of chs_coeffs
     TYPE, BIND(C) :: chs_coeffs

@@ -24,6 +24,7 @@ LIB_PATH = os.path.join(HERE, "libchapsim_hip.so")
 
 PLAIN_FP64 = 0
 MIXED = 1
+TUNE_DEFAULT = -1000000   # CHS_TUNE_DEFAULT
 
 _dp = C.POINTER(C.c_double)
 _lib = None
@@ -285,9 +286,10 @@ class ChannelTG:
         _check(lib().chs_set_refinement(self._h, int(nref_step), int(nref_projection)), self._h)
 
     def set_tuning(self, **shapes):
-        """Launch shapes, e.g. set_tuning(conv_by=8, conv_kc=16) (keys of chs_set_tuning)."""
+        """Launch shapes, e.g. set_tuning(conv_by=8, conv_kc=16) (keys of chs_set_tuning); None is a
+        key's default."""
         for k, v in shapes.items():
-            _check(lib().chs_set_tuning(self._h, k.encode(), int(v)), self._h)
+            _check(lib().chs_set_tuning(self._h, k.encode(), TUNE_DEFAULT if v is None else int(v)), self._h)
 
     def poisson(self, rhs):
         L, M, N = self.L, self.M, self.N
@@ -519,9 +521,10 @@ class ChannelIO:
         self._check(lib().chs_io_set_mixed(self._h, int(bool(mixed))), "chs_io_set_mixed")
 
     def set_tuning(self, **kv):
-        """Launch shapes (chs_io_set_tuning), e.g. mom_rows=2."""
+        """Launch shapes (chs_io_set_tuning), e.g. mom_rows=2; None is a key's default."""
         for k, v in kv.items():
-            self._check(lib().chs_io_set_tuning(self._h, k.encode(), int(v)), "chs_io_set_tuning")
+            self._check(lib().chs_io_set_tuning(self._h, k.encode(), TUNE_DEFAULT if v is None else int(v)),
+                        "chs_io_set_tuning")
 
     def sync(self):
         self._check(lib().chs_io_sync(self._h), "chs_io_sync")

@@ -13,7 +13,7 @@ import math
 
 import numpy as np
 
-from .tg import _check, _coeff_struct, _dp, _p, lib, ChsError
+from .tg import TUNE_DEFAULT, _check, _coeff_struct, _dp, _p, lib, ChsError
 
 
 def synthetic_table(n=2048, T_lo=600.0, T_hi=720.0, T_pc=660.0, cp_base=5.0e3, peak=8.0,
@@ -207,9 +207,10 @@ class EnergyTG:
         self._check(lib().chs_eng_set_mass_flux(self._h, C.c_void_p(g_dev_ptr)), "chs_eng_set_mass_flux")
 
     def set_tuning(self, **kv):
-        """Launch shapes (chs_eng_set_tuning), e.g. rhs_lds=0."""
+        """Launch shapes (chs_eng_set_tuning), e.g. rhs_lds=0; None is a key's default."""
         for k, v in kv.items():
-            self._check(lib().chs_eng_set_tuning(self._h, k.encode(), int(v)), "chs_eng_set_tuning")
+            self._check(lib().chs_eng_set_tuning(self._h, k.encode(), TUNE_DEFAULT if v is None else int(v)),
+                        "chs_eng_set_tuning")
 
     def SOLVERRK3_ENG_io(self, ns, dt):
         self._check(lib().chs_substep_eng(self._h, int(ns), float(dt)), "chs_substep_eng")

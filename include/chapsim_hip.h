@@ -41,6 +41,10 @@ enum {
                               reductions and divergence refinement                        */
 };
 
+/* As the value of a key of chs_set_tuning, chs_io_set_tuning or chs_eng_set_tuning: back to its
+ * default, which for many keys is a choice by the mesh that no other value stands for. */
+enum { CHS_TUNE_DEFAULT = -1000000 };
+
 /* Mesh and coefficient arrays as the reference's set-up computes them (CONSPARA,
  * COORDJR, TDMA_COEF, FFT99_ROOT, CONS_RKCOEF).  Index base as in the reference array,
  * counts in brackets:
@@ -164,8 +168,8 @@ int chs_set_refinement(chs_ctx *ctx, int nref_step, int nref_projection);
  * z-planes each correction thread marches (by default 2 or 4 by the mesh) and "upd_by" its rows per block (4), "upd_w2" 1
  * (default) for the correction with two points per lane where L is a multiple of 128 (0: one).  Results do not
  * depend on the shapes except through the summation order of the mass-flux partials
- * (conv_by, conv_kc, conv_fx) and conv_fx's rounding.  A captured step graph is re-made on
- * the next step.  CHS_E_ARG for an unknown key or a value out of range. */
+ * (conv_by, conv_kc, conv_fx) and conv_fx's rounding.  CHS_TUNE_DEFAULT is taken for every key.  A captured
+ * step graph is re-made on the next step.  CHS_E_ARG for an unknown key or a value out of range. */
 int chs_set_tuning(chs_ctx *ctx, const char *key, int value);
 
 /* ---- Batched tridiagonal solvers ------------------------------------------------------ */
@@ -362,7 +366,7 @@ int chs_substep_eng(chs_eng *e, int ns, double dt);
  * "rhs_lds" 1 (default) for the kernel that stages H, K, T, G_x, G_y per z-plane in LDS, 0 for
  * the one reading them per point (identical results); "rhs_kc" its z-planes per block (1..1024,
  * by default 8 to 32 by the mesh); "rhs_nxcd" the XCDs its tiles are grouped for (1..64, default 8).  CHS_E_ARG for
- * an unknown key or a value out of range. */
+ * an unknown key or a value out of range (CHS_TUNE_DEFAULT is taken for each). */
 int chs_eng_set_tuning(chs_eng *e, const char *key, int value);
 
 /* Copy fields back (NULL skips one): halo arrays (N, M+2, L), rhs0 (N, M, L). */
@@ -521,8 +525,8 @@ int chs_substep_io_momentum(chs_io *m, int ns, double dt);
  * (powers of two up to 512) or thread per line (0); "cn_fastdiv":
  * the z and y solves' coefficients by Newton reciprocals (1, default) or IEEE division (0),
  * which changes them by an ulp, below the 1e-17 the sweeps resolve.  Otherwise results change
- * only through the summation order of the mass-flux partials.  CHS_E_ARG for an unknown key
- * or value. */
+ * only through the summation order of the mass-flux partials.  CHS_TUNE_DEFAULT is taken for every key.
+ * CHS_E_ARG for an unknown key or value. */
 int chs_io_set_tuning(chs_io *m, const char *key, int value);
 
 /* Mixed form of the main-domain momentum substep (mixed = 1): EXPLT0_io (the RK history of

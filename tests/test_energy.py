@@ -262,3 +262,17 @@ def test_gpu_cell_props_on_uneven_tables(pkg, kind, L, M, N):
         for k, w in want.items():
             np.testing.assert_array_equal(out[k][:, 1:M + 1], w, err_msg=k)
     e.close()
+
+
+@pytest.mark.gpu
+def test_gpu_rhs_default_shapes_are_taken(pkg):
+    """None (CHS_TUNE_DEFAULT) is taken for each key of the energy substep, and for no other."""
+    from chapsim_amd import thermo
+    t = thermo.table_setup(thermo.synthetic_table(), 665.0)
+    e = thermo.EnergyTG(pkg.channel_setup(16, 9, 6, STR2=1.8), t, (1, 1), 1e-3, t["DH"][t["IMIN_DH"] - 1],
+                        t["DH"][t["IMAX_DH"] - 1], (0.1, -0.1))
+    e.set_tuning(rhs_lds=0, rhs_kc=3, rhs_nxcd=1)
+    e.set_tuning(rhs_lds=None, rhs_kc=None, rhs_nxcd=None)
+    with pytest.raises(pkg.ChsError):
+        e.set_tuning(no_such_key=None)
+    e.close()

@@ -535,3 +535,35 @@ def test_convection_march_by_mesh_is_near_the_best(pkg, L, M, N, mode):
     print(f"  by the mesh {auto:.4f} ms, by hand {by_hand}")
     assert auto < 1.12 * min(by_hand.values())
     ch.close()
+
+
+def test_default_shapes_can_be_set_again(pkg):
+    """None (CHS_TUNE_DEFAULT) puts back what a context was made with, the choices by the mesh among
+    them: after other values for every key and None again, a step gives a fresh channel's bits
+    (conv_kc, conv_by and conv_fx change the mass flux's last bits, ytdma_c and fft_reg the solve's)."""
+    L, M, N = 48, 36, 40
+    q, p = oracle.initial_field(setup.Mesh(L, M, N, STR2=2.0), 3)
+    other = dict(conv_by=16, conv_kc=3, conv_fence=1, conv_fx=0, conv_lds=1, conv_dma=0, cnx_nlx=3, cnz_kz=5, cny_ky=7,
+                 cn_xz=1, cnxz_by=2, fftx_tk=2, fftz_nl=1, nxcd=3, fft_reg=0, ytdma_bs=128, ytdma_rb=8, ytdma_c=0,
+                 divg_nxcd=1, cny3_ky=-1, upd_kz=7, upd_by=2, upd_nxcd=3, upd_w2=0, cnzy=2, cnzy_ky=20, cnzy_nxcd=1)
+    for mode in (pkg.PLAIN_FP64, pkg.MIXED):
+        out = []
+        for reset in (False, True):
+            ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=2.0), mode)
+            ch.upload(q, p)
+            if reset:
+                ch.set_tuning(**other)
+                ch.rk3_step(8.0e-4, 1.0 / 4000.0)
+                ch.upload(q, p, np.zeros((3, N, M, L)))
+                ch.set_tuning(**{k: None for k in other}, conv_bx=None)
+            for _ in range(2):
+                ch.rk3_step(8.0e-4, 1.0 / 4000.0)
+            ch.profile_reset(None)
+            ch.rk3_step(8.0e-4, 1.0 / 4000.0)
+            out.append((*ch.download(), [ch.profile_get(k)[1] for k in ("conv_rhs", "cn_x", "cn_xz", "cn_z", "cn_y", "cn_zy",
+                                                                         "spec_plane", "ytdma")]))
+            with pytest.raises(pkg.ChsError):
+                ch.set_tuning(no_such_key=None)
+            ch.close()
+        assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+        assert out[0][2] == out[1][2]

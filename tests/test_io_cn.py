@@ -682,3 +682,29 @@ def test_gpu_cn_stiff_lines_keep_their_lanes(pkg):
         ch.close()
     print(f"  sweeps {1e6 * took[0]:.0f} us, thread per line {1e6 * took[1]:.0f} us")
     assert took[1] < 5.0 * took[0]
+
+
+@pytest.mark.gpu
+def test_gpu_io_default_shapes_can_be_set_again(pkg):
+    """None (CHS_TUNE_DEFAULT) puts back what a context was made with: the momentum part gives a fresh
+    context's bits again (mom_kz changes the mass flux's last bits, cn_fastdiv the line solves')."""
+    L, M, N, REN, dt = 48, 37, 30, 4000.0, 5e-4
+    mesh = setup.Mesh(L, M, N, STR2=2.0)
+    st = oracle.io_initial_field(mesh, 96)
+    m1 = cn_viscosity(st, 96, False)
+    other = dict(mom_rows=2, mom_kz=0, props_kc=0, mom_nxcd=1, mom_by=8, cnz_p=4, cny_p=4, cnz_cols=3, cny_cols=5,
+                 cn_fastdiv=0, cnx_wave=0, cn_cols=2)
+    out = []
+    for reset in (False, True):
+        ch = pkg.ChannelIO(pkg.channel_setup(L, M, N, STR2=2.0), REN, flow_driven=1, vis_scheme=1)
+        if reset:
+            ch.set_tuning(**other)
+            ch.set_tuning(**{k: None for k in other})
+        ch.upload(**st, M1=m1)
+        ch.ioprops(1)
+        ch.momentum(1, dt)
+        out.append(ch.download()["G"])
+        with pytest.raises(pkg.ChsError):
+            ch.set_tuning(no_such_key=None)
+        ch.close()
+    assert np.array_equal(out[0], out[1])
