@@ -71,6 +71,8 @@ def alg_bytes(kernel: str, L: int, M: int, N: int, wbytes: int) -> float:
         # R spectrum + pivots (work precision; FP64 for six low modes), W spectrum
         "ytdma": 2 * S * 2 * wbytes + S * wbytes,
         "fftz_inv": 2 * S * 2 * wbytes,
+        # both z-transforms and the y-solve in one pass: R spectrum + pivots, W spectrum
+        "spec_plane": 2 * S * 2 * wbytes + S * wbytes,
         # R spectrum, W phi
         "fftx_inv": S * 2 * wbytes + F * 8,
         # R phi, predicted u, v, w, p; W u, v, w, p
@@ -95,7 +97,7 @@ def canonical_step_bytes(L: int, M: int, N: int, wbytes: int) -> float:
 
 
 KERNELS = ["conv_rhs", "cn_x", "cn_z", "cn_xz", "cn_y", "cn_zy", "divg_fftx", "fftz_fwd", "ytdma",
-           "fftz_inv", "fftx_inv", "update", "refine_update"]
+           "fftz_inv", "spec_plane", "fftx_inv", "update", "refine_update"]
 
 
 def load_pkg():
