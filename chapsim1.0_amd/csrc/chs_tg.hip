@@ -3849,9 +3849,12 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
     //  x     register plan where L has one, except where mixed radix is faster: L >= 512, whose plan
     //        holds one line, so two planes or 32-byte runs of the spectrum, per wavefront
     //        (512x192x512 forward 520 / 552 / 349, inverse 340 / 263 / 208; FP32 inverse
-    //        188 / 162 / 145), and the FP64 forward transform with the divergence of L = 128
-    //        (128x96x128: 22.3 / 19.9 / 17.0; of a given field the plan is faster); else mixed
-    //        radix (144x103x180 forward 48 / - / 29, inverse 35 / - / 17).
+    //        188 / 162 / 145), and the FP64 forward transform with the divergence of L = 128, whose
+    //        plan takes 18 us on any small mesh.  Plan / mixed radix over 11 meshes: L = 128 1.00 to 1.66
+    //        (128x16x64 18.2 / 11.0, 128x96x128 20.5 / 17.7, 128x192x256 72.5 / 54.3), L = 64 0.76 to
+    //        1.01, L = 256 0.88 to 1.04 (1.15 and 1.23 with 48 and 16 rows of 64).  Of a given field the
+    //        plan is the faster at 128 too.  Else mixed radix (144x103x180 forward 48 / - / 29, inverse
+    //        35 / - / 17).
     // The LDS transforms remain for lengths with no plan of two or three passes of at most 256
     // threads a line, for fft_reg = 0 and for the batched ensemble.
     const bool f64 = sizeof(T) == 8, fr = c->tune.fft_reg != 0, gxok = c->gtwx && c->gtwxi;
@@ -4024,7 +4027,8 @@ int substep_impl(chs_ctx *c, int ns, double dt, double cvisc, bool host_dt = tru
     const int FY = c->tune.conv_fx;   // rows per block of the fused kernel (0: not fused)
     const bool fx0 = FY > 0 && M % FY == 0 && !xz && zmarch && L % 64 == 0 && L * FY <= 512 && !t.fullx &&
                     t.Dx <= 16;
-    // state staged through LDS (k_conv_rhs_lds): LY rows of whole x-lines per block
+    // state staged through LDS (k_conv_rhs_lds): LY rows of whole x-lines per block; only with conv_dma = 0, as
+    // one of the two below takes every mesh that it could
     const int LY = c->tune.conv_lds;
     // state planes moved into LDS by direct loads (k_conv_rhs_dma): DY rows per block
     const int DY = c->tune.conv_dma;

@@ -136,39 +136,46 @@ int chs_set_graph(chs_ctx *ctx, int enable);
 int chs_set_refinement(chs_ctx *ctx, int nref_step, int nref_projection);
 
 /* Launch shapes of the substep kernels (no counterpart in the reference, whose loops have no
- * tiling).  Keys and limits: "conv_by" rows per k_conv_rhs block (1, 2, 4, 8, 16; default 4),
- * "conv_bx" wavefronts along x per k_conv_rhs block (1 or 4, conv_bx * conv_by <= 16; 1),
- * "conv_fence" 1 to keep all of a z-plane's loads ahead of its arithmetic in k_conv_rhs (FP64 0,
- * mixed 1),
- * "conv_kc" z-planes marched per k_conv_rhs thread (1..N; by default chosen by the mesh for the
- * direct-to-LDS kernel, else 16), "cnx_nlx" x-lines per CN-x
- * block (0 = 2048/L), "cnz_kz" / "cny_ky" march lengths of the z / y CN stencils (FP64 16 / 48,
- * mixed 8 / 32),
- * "fftx_tk" z-planes per x-transform block (0 = derived; even, divides N, TK/2*L <= 2048),
- * "fftz_nl" z-lines per z-transform block (0 = 2048/N; NL*N <= 2048), "nxcd" number of L2
- * domains (XCDs) the k_conv_rhs tiles are grouped for (1..64; FP64 1 = dispatch order, mixed 8),
- * "fft_reg" 1 (default) to run the register-resident FFTs for line lengths 64 ... 1024, 0 for
- * the LDS Stockham transforms, "cn_xz" 1 to run the x and z Crank-Nicolson solves in one kernel
- * where a block can hold whole x-lines (default 0: two kernels, faster on MI355X at 256^2 x
- * 192), "cnxz_by" x-lines per block of that kernel (1, 2, 4; 1), "conv_fx" rows per block
- * (1 default, 2) of k_conv_rhs applying the x Crank-Nicolson inverse itself where L is 64,
- * 128, 192 or 256 (L * conv_fx <= 512, M divisible by conv_fx) and the inverse's band is
- * short, 0 for the separate x kernel (with conv_fx > 0, conv_bx / conv_by do not apply; the
- * mass-flux correction moves after the z-solve, which changes rounding only), "ytdma_bs"
- * threads per block of the Poisson y-solve (64 default, 128, 256) and "ytdma_rb" its rows per
- * load batch (8, 16 default), "ytdma_c" rows per chunk of the chunked y-Thomas (-1 = chosen by
- * the mesh, 0 = unchunked), "conv_dma" rows per block of the direct-to-LDS convection kernel
- * (4 default, 2; 0 = off), "cny3_ky" rows per chunk of the fused three-component y-solve (by default 9 to 48 by the mesh;
- * 0 = M, -1 = one launch per component), "cnzy" 1 to run the z and y Crank-Nicolson
- * solves in one pass where L is a multiple of 64 and N of 16 (the default, in FP64 from 2^22 points), 2 on every mesh (ragged tiles), 0
- * for the two kernels (the pass needs z and y band half-widths of at most 8), "cnzy_ky" its rows
- * per chunk (by default 12 to 48 by the mesh; 0 = M), "cnzy_nxcd" the XCDs its tiles
- * are grouped for (8), "divg_nxcd" and "upd_nxcd" the XCDs the divergence
- * transform's and the correction's tiles are grouped for (8 and 1; 1 = dispatch order), "upd_kz"
- * z-planes each correction thread marches (by default 2 or 4 by the mesh) and "upd_by" its rows per block (4), "upd_w2" 1
- * (default) for the correction with two points per lane where L is a multiple of 128 (0: one).  Results do not
- * depend on the shapes except through the summation order of the mass-flux partials
- * (conv_by, conv_kc, conv_fx) and conv_fx's rounding.  CHS_TUNE_DEFAULT is taken for every key.  A captured
+ * tiling).  Several keys shape a kernel that others stand in for on most meshes; they are taken
+ * always and act where their kernel runs.
+ * Convection: "conv_dma" rows per block of the direct-to-LDS kernel (4 default, 2; 0 = off), which
+ * applies the x Crank-Nicolson inverse itself: with 4 rows every L from 32 to 256, with 2 L = 64,
+ * 128, 192 or 256 and even M; "conv_fx" 1 (default) or 2 to let a convection kernel apply that
+ * inverse, 0 for the separate x kernel (the inverse's band must be short; the mass-flux
+ * correction moves after the z-solve, which changes rounding only); "conv_kc" its z-planes per march
+ * (1..N; by default by the mesh for conv_dma = 4, else 16); "nxcd" number of L2 domains (XCDs) its
+ * tiles are grouped for (1..64; FP64 1 = dispatch order, mixed 8).  With conv_dma = 0: "conv_lds"
+ * rows per block of the kernel staged through registers (2 default, 1, 4; 0 = off; L = 64, 128, 192 or
+ * 256, M a multiple of it).  Else, and for other L: conv_fx rows per block of k_conv_rhs (L a
+ * multiple of 64, L * conv_fx <= 512, M divisible by conv_fx), and where it does not apply the
+ * inverse itself (conv_fx = 0, other L or M) "conv_by" its rows per block (1, 2, 4, 8, 16; default 4),
+ * "conv_bx" its wavefronts along x (1 or 4, conv_bx * conv_by <= 16; 1); "conv_fence" 1 to keep all
+ * of a z-plane's loads ahead of its arithmetic in k_conv_rhs (FP64 0, mixed 1).
+ * Crank-Nicolson: "cnx_nlx" x-lines per block of the separate x kernel (0 = 2048/L), "cnz_kz" /
+ * "cny_ky" march lengths of the z / y stencils (FP64 16 / 48, mixed 8 / 32), "cn_xz" 1 to run the x
+ * and z solves in one kernel where a block can hold whole x-lines (default 0: two kernels, faster on
+ * MI355X at 256^2 x 192), "cnxz_by" x-lines per block of that kernel (1, 2, 4; 1), "cny3_ky" rows per
+ * chunk of the fused three-component y-solve (by default 9 to 48 by the mesh; 0 = M, -1 = one launch
+ * per component), "cnzy" 1 to run the z and y solves in one pass where L is a multiple of 64 and N of
+ * 16 (the default, in FP64 from 2^22 points), 2 on every mesh (ragged tiles), 0 for the two
+ * kernels (the pass needs z and y band half-widths of at most 8), "cnzy_ky" its rows per chunk (by
+ * default 12 to 48 by the mesh; 0 = M), "cnzy_nxcd" the XCDs its tiles are grouped for (8).
+ * Poisson: "fft_reg" 1 (default) for the transforms whose passes run in registers: line lengths 64,
+ * 128, 256, 512 and 1024, and every other length with a plan of two or three passes of radices up to
+ * 16, at most 256 threads a line; 0, and the other lengths, for the LDS Stockham transforms,
+ * which alone have "fftx_tk" z-planes per x-transform block (0 = derived; even, divides N, TK/2*L <=
+ * 2048) and "fftz_nl" z-lines per z-transform block (0 = 2048/N; NL*N <= 2048); "ytdma_c" rows per
+ * chunk of the y-Thomas (-1 = by the mesh: in FP64 the z-transforms and the y-Thomas of a kx in one
+ * block where its plane fits, else chunks of 4 to 16 rows; 4, 8, 16; 0 = unchunked); "ytdma_bs"
+ * threads per block of the unchunked y-solve (64 default, 128, 256) and "ytdma_rb" its rows per
+ * load batch (8, 16 default); "divg_nxcd" the XCDs the divergence transform's tiles are grouped
+ * for (8; 1 = dispatch order).
+ * Correction: "upd_kz" z-planes each thread marches (by default 2 or 4 by the mesh) and "upd_by" its
+ * rows per block (4), "upd_nxcd" the XCDs its tiles are grouped for (1), "upd_w2" 1 (default) for two
+ * points per lane where L is a multiple of 128 (0: one).
+ * Results do not depend on the shapes except through the summation order of the mass-flux partials
+ * (conv_by, conv_kc, conv_fx, conv_lds, conv_dma), conv_fx's rounding, and the rounding of the pressure
+ * solve (fft_reg, ytdma_c).  CHS_TUNE_DEFAULT is taken for every key.  A captured
  * step graph is re-made on the next step.  CHS_E_ARG for an unknown key or a value out of range. */
 int chs_set_tuning(chs_ctx *ctx, const char *key, int value);
 

@@ -567,3 +567,60 @@ def test_default_shapes_can_be_set_again(pkg):
             ch.close()
         assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
         assert out[0][2] == out[1][2]
+
+
+@pytest.mark.parametrize("L,M,N", [(48, 9, 90), (90, 6, 48), (120, 5, 150), (150, 7, 120), (250, 4, 54), (12, 5, 486), (96, 80, 96)])
+def test_lds_transforms_match_oracle(pkg, L, M, N):
+    """The LDS transforms (fft_reg = 0; what batched ensembles launch, and lengths without a plan)
+    at lengths with factors 3 and 5 that the mixed-radix plans otherwise take, bounds as
+    test_poisson_matches_oracle."""
+    print(f"lds poisson {L}x{M}x{N}", flush=True)
+    mesh = setup.Mesh(L, M, N, STR2=1.9)
+    r = np.random.default_rng(L + N).standard_normal((N, M, L))
+    w = (1.0 / mesh.DYFI)[None, :, None]
+    r -= np.sum(r * w) / (np.sum(w) * L * N)
+    ref = oracle.OracleTG(mesh, 2800.0).poisson(r)
+    for mode, tol in ((pkg.PLAIN_FP64, 1e-10), (pkg.MIXED, 1e-5)):
+        ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=1.9), mode)
+        ch.set_tuning(fft_reg=0)
+        phi = ch.poisson(r)
+        assert rel(phi, ref) < tol, (mode, rel(phi, ref))
+        ch.close()
+
+
+@pytest.mark.parametrize("kv", [dict(fftx_tk=2, fftz_nl=1), dict(fftx_tk=8, fftz_nl=5), dict(fftx_tk=4, fftz_nl=51)])
+def test_lds_transform_tilings_match_oracle(pkg, kv):
+    """fftx_tk and fftz_nl shape the LDS transforms alone (fft_reg = 0): other tilings give the oracle's
+    step to test_launch_shapes_keep_results' bounds."""
+    L, M, N, STR2, REN, dt = 48, 36, 40, 2.0, 4000.0, 8.0e-4
+    print(f"lds tilings {kv}", flush=True)
+    mesh, ch, o = make(pkg, L, M, N, STR2, REN)
+    ch.set_tuning(fft_reg=0, **kv)
+    ch.SOLVERRK3_MOM_tg(0, dt, 1.0 / REN)
+    o.substep(0, dt)
+    for _ in range(2):
+        ch.rk3_step(dt, 1.0 / REN)
+        for ns in (1, 2, 3):
+            o.substep(ns, dt)
+    gq, gp = ch.download()
+    assert max(rel(gq[c], o.q[c]) for c in range(3)) < 1e-10 and rel(gp, o.pr) < 1e-10
+    ch.close()
+
+
+@pytest.mark.parametrize("L,M,N", [(128, 20, 16), (192, 12, 18), (64, 24, 32)])
+def test_lds_convection_matches_oracle(pkg, L, M, N):
+    """The convection kernel that stages its rows through registers (conv_lds rows), which the
+    direct-to-LDS one stands in for unless conv_dma = 0."""
+    STR2, REN, dt = 2.0, 4000.0, 8.0e-4
+    for rows in (1, 2, 4):
+        print(f"lds convection {L}x{M}x{N} rows {rows}", flush=True)
+        mesh, ch, o = make(pkg, L, M, N, STR2, REN)
+        ch.set_tuning(conv_dma=0, conv_lds=rows)
+        ch.SOLVERRK3_MOM_tg(0, dt, 1.0 / REN)
+        o.substep(0, dt)
+        ch.rk3_step(dt, 1.0 / REN)
+        for ns in (1, 2, 3):
+            o.substep(ns, dt)
+        gq, gp = ch.download()
+        assert max(rel(gq[c], o.q[c]) for c in range(3)) < 1e-10 and rel(gp, o.pr) < 1e-10
+        ch.close()
