@@ -3345,6 +3345,7 @@ struct chs_ctx {
     double *pp00 = nullptr;  // (0,0)-mode pivots without FFT99's decoupling (FISHPACK gauge)
     int npartial = 0;
     double *mean_part = nullptr, *mean_host = nullptr;   // chs_mean_zx_tg: tile sums, pinned result
+    std::mutex mean_mu;                                  // held while a call uses them
     void *twx = nullptr, *twz = nullptr;
     void *rtwx = nullptr, *rtwz = nullptr;   // register-FFT pass twiddles (chs_fftr.h), if planned
     chs::GPlan gx{}, gxi{}, gz{};            // mixed-radix plans: x forward, x inverse, z (chs_fftg.h)
@@ -5494,6 +5495,7 @@ extern "C" int chs_mean_zx_tg(chs_ctx *c, double *stats, double *scal)
 {
     if (!c || (!stats && !scal)) return fail(c, CHS_E_ARG, "chs_mean_zx_tg: null argument");
     const int L = c->L, M = c->M, N = c->N;
+    const std::lock_guard<std::mutex> lock(c->mean_mu);
     const double vl = 1.0 / (double)(L * N);
     const MeanCoef mc = {vl, {vl * c->dxi, vl * 0.25, vl * 0.25 * c->dzi, vl * 0.25 * c->dxi, vl, vl * 0.25 * c->dzi,
                               vl * 0.25 * c->dxi, vl * 0.25, vl * c->dzi}};

@@ -96,3 +96,21 @@ def test_gpu_lane_and_run_edges(pkg, L, M, N):
     ch.upload(q, p)
     check(*ch.PP_MEAN_ZX_FLOW_TG(), *o.mean_zx())
     ch.close()
+
+
+@pytest.mark.gpu
+def test_gpu_threads_share_a_channel(pkg):
+    """Calls of several threads on one channel, the first of which lays out the buffers that they share:
+    each returns the same bits as a call on its own."""
+    from concurrent.futures import ThreadPoolExecutor
+    L, M, N = 96, 40, 54
+    q, p = pkg.poiseuille_perturbed(pkg.channel_setup(L, M, N, STR2=1.8), seed=3, amp=0.2)
+    ref = None
+    for _ in range(3):
+        ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=1.8), pkg.PLAIN_FP64)
+        ch.upload(q, p)
+        with ThreadPoolExecutor(8) as ex:
+            got = list(ex.map(lambda _: ch.PP_MEAN_ZX_FLOW_TG(), range(64)))
+        ref = ref or ch.PP_MEAN_ZX_FLOW_TG()
+        assert all(np.array_equal(a, b) for g in got for a, b in zip(g, ref))
+        ch.close()
