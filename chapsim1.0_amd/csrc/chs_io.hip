@@ -1046,9 +1046,11 @@ __device__ __forceinline__ double block_max_nonneg(double v, unsigned long long 
 // rho = max (|a| + |c|) / |b| (about 1e-4 in x and z and 2e-3 at the walls in y on the
 // channel meshes).  Starting from x0 = r / b, K Jacobi sweeps x <- (r - a x_- - c x_+) / b leave
 // an error of at most rho^(K+1) max|x| (|x0 - x| <= rho |x|, each sweep contracts by rho); K is
-// the least count with rho^(K+1) <= 1e-17, e.g. 3 sweeps at rho = 1e-4.  The line kernels below
-// solve this way and hand a block whose rho exceeds 1/4 to the thread-per-line recurrences
-// (io_cn_x_line, io_cn_z_line, io_cn_y_line).
+// the least count with rho^(K+1) <= 1e-17, e.g. 3 sweeps at rho = 1e-4.  Their error against long
+// double is 0.7 to 1.6e-16 max|x|, the recurrences' 1.3 to 2.3e-16 (lines of 10 to 500 points, rho up
+// to 1/4).  The line kernels below solve this way and hand a block whose rho exceeds 1/4 to the
+// recurrences, a lane per line (io_cn_x_line, io_cn_z_line, io_cn_y_line; the launch sends padded
+// blocks of stiff lines to the thread-per-line kernels).
 // 1/x from the hardware estimate and two Newton-Raphson steps r <- r + r (1 - x r), each of
 // which doubles the correct bits: within about an ulp of the correctly rounded reciprocal.
 __device__ __forceinline__ double rcp_nr(double x)
@@ -1784,7 +1786,7 @@ struct chs_io {
     double ymax = 0.0;                // largest (AMVR + APVR) / 2
     int cnz_p = 8, cny_p = 8;         // line points per thread of the z and y solves (4 or 8; 8:
                                       // 6.21 -> 6.09 (z) and 6.14 (y) ms per heated CN step)
-    int cnx_wave = 1;     // x-lines of the Crank-Nicolson solve one per wavefront (L = 64, 128, 256, 512)
+    int cnx_wave = 1;     // x-lines of the Crank-Nicolson solve one per wavefront (L a multiple of at most 64 lanes)
     int cn_fastdiv = 1;   // z and y Jacobi coefficients by Newton reciprocals (the sweeps resolve
                           // no finer; 0.26 -> 0.24 and 0.29 -> 0.28 ms per stage at 256 x 128 x 256)
     int cn_cols = 16;   // most x-columns per block of the z and y Jacobi line solves (16: 1.7 %

@@ -601,7 +601,7 @@ __global__ __launch_bounds__(256) void k_eng_props(EngDev e, PropDev p, int j0, 
     const size_t base = ehx(e, 0, j0, blockIdx.y - wrows);
     const int R = rows * e.L, c0 = blockIdx.x * (256 * C) + threadIdx.x, q = threadIdx.x & 3;
     if (c0 - (int)(threadIdx.x & 63) >= R) return;   // a wavefront past the plane's end
-    double dv[C], hv[C], cp[C];
+    double dv[C], hv[C];
     int I[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) dv[c] = e.dh[base + min(c0 + 256 * c, R - 1)];   // lanes past the end repeat the last cell
@@ -638,7 +638,6 @@ __global__ __launch_bounds__(256) void k_eng_props(EngDev e, PropDev p, int j0, 
         cell(std::integral_constant<int, 1>{});
         cell(std::integral_constant<int, 2>{});
         cell(std::integral_constant<int, 3>{});
-        cp[c] = q == 0 ? y[0] : q == 1 ? y[1] : q == 2 ? y[2] : y[3];
         quad_transpose(r, q);
         const int n = c0 + 256 * c;
         if (n < R) {
