@@ -472,26 +472,58 @@ __device__ __forceinline__ double spl_rec(double x, double y, double b, double c
     return y + dx * (b + dx * (c + dx * d));
 }
 
-// THERM_PROP_UPDATE_FROM_DH for one cell, each lookup equal to spl_eval's.  The five H-based
-// splines share their table (LIST_H) and range (IMIN_H, IMAX_H), so one search serves all of them.
-// xdh / xh: LIST_DH / LIST_H (LDS copies or the global tables).
+// THERM_PROP_UPDATE_FROM_DH for C cells (o[c], those with act[c]), each lookup equal to spl_eval's.  The
+// five H-based splines share their table (LIST_H) and range (IMIN_H, IMAX_H), so one search serves
+// all of them, and a cell's records come in 16-byte loads.  xdh / xh: LIST_DH / LIST_H (LDS copies
+// or the global tables).  An inactive cell stores nothing.
+template <int C>
+__device__ void eng_cells_props(const EngDev &e, const PropDev &p, const size_t *o, const bool *act, int *err,
+                                const double *xdh, const double *xh)
+{
+    double dv[C], h[C];
+    int I[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) dv[c] = act[c] ? e.dh[o[c]] : xdh[0];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        if (act[c]) eng_range(p.dhh, dv[c], err, 1);
+        I[c] = spl_index_b(p.bdh, xdh, p.n, dv[c]) - 1;
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const double2 *r = reinterpret_cast<const double2 *>(p.recd + (size_t)8 * I[c]);
+        const double2 r0 = r[0], r1 = r[1], r2 = r[2];
+        h[c] = spl_rec(r0.x, r0.y, r1.x, r1.y, r2.x, dv[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        if (act[c]) eng_range(p.ht, h[c], err, 2 | 4 | 8 | 16 | 32);
+        I[c] = spl_index_b(p.bh, xh, p.n, h[c]) - 1;
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        if (!act[c]) continue;
+        const double2 *rc = reinterpret_cast<const double2 *>(p.recc + (size_t)8 * I[c]);
+        const double2 *rh = reinterpret_cast<const double2 *>(p.rech + (size_t)16 * I[c]);
+        const double2 c0 = rc[0], c1 = rc[1], c2 = rc[2];
+        double2 v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = rh[q];
+        const double x = c0.x, hv = h[c];
+        e.h[o[c]] = hv;
+        e.t[o[c]] = spl_rec(x, v[0].x, v[0].y, v[4].x, v[4].y, hv);
+        e.d[o[c]] = spl_rec(x, v[1].x, v[1].y, v[5].x, v[5].y, hv);  // D from H->M, as the reference
+        e.m[o[c]] = spl_rec(x, v[2].x, v[2].y, v[6].x, v[6].y, hv);  // M from H->K
+        e.k[o[c]] = spl_rec(x, v[3].x, v[3].y, v[7].x, v[7].y, hv);  // K from H->D
+        e.cp[o[c]] = spl_rec(x, c0.y, c1.x, c1.y, c2.x, hv);
+    }
+}
+
 __device__ void eng_cell_props(const EngDev &e, const PropDev &p, size_t o, int *err, const double *xdh,
                                const double *xh)
 {
-    const double dv = e.dh[o];
-    eng_range(p.dhh, dv, err, 1);
-    const double *r = p.recd + (size_t)8 * (spl_index_b(p.bdh, xdh, p.n, dv) - 1);
-    const double h = spl_rec(r[0], r[1], r[2], r[3], r[4], dv);
-    eng_range(p.ht, h, err, 2 | 4 | 8 | 16 | 32);
-    const int I = spl_index_b(p.bh, xh, p.n, h) - 1;
-    const double *c = p.recc + (size_t)8 * I, *v = p.rech + (size_t)16 * I;
-    const double x = c[0];
-    e.h[o] = h;
-    e.t[o] = spl_rec(x, v[0], v[1], v[8], v[9], h);
-    e.d[o] = spl_rec(x, v[2], v[3], v[10], v[11], h);  // D from H->M, as the reference
-    e.m[o] = spl_rec(x, v[4], v[5], v[12], v[13], h);  // M from H->K
-    e.k[o] = spl_rec(x, v[6], v[7], v[14], v[15], h);  // K from H->D
-    e.cp[o] = spl_rec(x, c[1], c[2], c[3], c[4], h);
+    const bool act = true;
+    eng_cells_props<1>(e, p, &o, &act, err, xdh, xh);
 }
 
 // BC_WALL_THERMAL(IMAIND) (BC_WALL.f90:622-643) at the ghost cell (i, k) of wall w (0 bottom, 1 top):
@@ -522,7 +554,8 @@ __device__ void eng_wall(const EngDev &e, const PropDev &p, int *err, int w, int
 }
 
 // THERM_PROP_UPDATE (THERM_PROP_UPDATE.f90:124-168) over rows j0..j1 for tables without a bucket
-// index: the bisections run on LDS copies of the two searched tables (lds != 0; 2 n doubles).
+// index: the bisections run on LDS copies of the two searched tables (lds != 0; 2 n doubles), two cells
+// per thread (z-planes k and k + gridDim.z) for the copies' cost and the records' latency.
 __global__ __launch_bounds__(256) void k_eng_props_bisect(EngDev e, PropDev p, int j0, int j1, int *err, int lds)
 {
     extern __shared__ double tab[];
@@ -537,7 +570,11 @@ __global__ __launch_bounds__(256) void k_eng_props_bisect(EngDev e, PropDev p, i
         xh = tab + p.n;
     }
     const int i = blockIdx.x * 64 + threadIdx.x, J = j0 + blockIdx.y * 4 + threadIdx.y;
-    if (i < e.L && J <= j1) eng_cell_props(e, p, ehx(e, i, J, blockIdx.z), err, xdh, xh);
+    const int k = blockIdx.z, k2 = k + gridDim.z;
+    if (i >= e.L || J > j1) return;
+    const size_t o[2] = {ehx(e, i, J, k), ehx(e, i, J, k2 < e.N ? k2 : k)};
+    const bool act[2] = {true, k2 < e.N};
+    eng_cells_props<2>(e, p, o, act, err, xdh, xh);
 }
 
 // The value of lane Q of this lane's quad (DPP; every lane of the wavefront takes part).
@@ -733,7 +770,7 @@ void eng_props_and_walls(chs_eng *e, int j0, int j1)
     } else {
         const size_t sh = 2 * sizeof(double) * (size_t)p.n;
         const int lds = sh <= 64 * 1024;
-        hipLaunchKernelGGL(k_eng_props_bisect, dim3((e->L + 63) / 64, (rows + 3) / 4, e->N), dim3(64, 4), lds ? sh : 0,
+        hipLaunchKernelGGL(k_eng_props_bisect, dim3((e->L + 63) / 64, (rows + 3) / 4, (e->N + 1) / 2), dim3(64, 4), lds ? sh : 0,
                            e->stream, e->e, p, j0, j1, e->err, lds);
         own = false;
     }

@@ -276,3 +276,40 @@ def test_gpu_rhs_default_shapes_are_taken(pkg):
     with pytest.raises(pkg.ChsError):
         e.set_tuning(no_such_key=None)
     e.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,M,N", [(70, 6, 5), (64, 5, 4), (6, 4, 7)])
+def test_gpu_cell_props_by_bisection_on_plane_pairs(pkg, L, M, N):
+    """The update of tables without a bucket index takes two z-planes per thread: odd plane counts, rows and
+    columns past the mesh, as test_gpu_cell_props_on_uneven_tables."""
+    test_gpu_cell_props_on_uneven_tables(pkg, "unordered", L, M, N)
+
+
+@pytest.mark.gpu
+def test_gpu_unordered_table_costs_its_bisections_only(pkg):
+    """An energy substep on a table that is not ordered against one on an ordered table, 256x128x256: 1.26 on
+    MI355X (1.37 with a cell per thread and its records in 8-byte loads)."""
+    import time
+    from chapsim_amd import thermo
+    L, M, N = 256, 128, 256
+    rng = np.random.default_rng(3)
+    took = []
+    for T0 in (665.0, 630.0):
+        t = thermo.table_setup(thermo.synthetic_table(), T0)
+        assert (T0 == 665.0) == bool(np.all(np.diff(t["DH"]) >= 0))
+        v = [t["DH"][t[k] - 1] for k in ("IMIN_DH", "IMAX_DH")]
+        dh = min(v) + abs(v[1] - v[0]) * (0.35 + 0.3 * rng.random((N, M + 2, L)))
+        e = thermo.EnergyTG(pkg.channel_setup(L, M, N, STR2=1.8), t, (1, 1), 1e-9, *v, (0.0, 0.0))
+        e.upload(dh, np.zeros((3, N, M + 2, L)))
+        best = 1.0
+        for _ in range(5):
+            e.SOLVERRK3_ENG_io(1, 1e-6)
+            t0 = time.perf_counter()
+            for _ in range(20):
+                e.SOLVERRK3_ENG_io(1, 1e-6)
+            best = min(best, (time.perf_counter() - t0) / 20)
+        took.append(best)
+        e.close()
+    print(f"  ordered {1e6 * took[0]:.0f} us, unordered {1e6 * took[1]:.0f} us")
+    assert took[1] < 1.32 * took[0]
