@@ -2174,11 +2174,14 @@ __global__ __launch_bounds__(64) void k_divg_fftx_r(Geo g, const cpx<T> *__restr
 
 // x inverse: Hermitian extension of the plane pair of each line, complex inverse transform,
 // real parts to the solution rows.  Five loads of each plane in flight per lane: 256x192x256 37 us
-// (42 with one at a time), FP32 28 (31), 64x64x64 6.5 (7.1).  (CELLS: of a cell field, else of the halo field; PhiOut).
-template <typename T, int L, bool CELLS>
+// (42 with one at a time), FP32 28 (31), 64x64x64 6.5 (7.1).  FP64: one instance for halo and cell
+// fields, whose addresses it takes from out, so that every caller gets the same rounding (the
+// compiler contracts other instances' products differently); FP32 writes the halo field alone.
+template <typename T, int L>
 __global__ __launch_bounds__(64) void k_fftx_inv_r(Geo g, const cpx<T> *__restrict__ tw,
-                                                   const cpx<T> *__restrict__ spec, double *__restrict__ phi)
+                                                   const cpx<T> *__restrict__ spec, PhiOut out)
 {
+    constexpr bool RT = sizeof(T) == 8;
     using G = RGeom<L>;
     constexpr int TK = 2 * G::LPW;
     __shared__ cpx<T> lds[G::LPW * G::LS];
@@ -2215,17 +2218,19 @@ __global__ __launch_bounds__(64) void k_fftx_inv_r(Geo g, const cpx<T> *__restri
         for (int r = 0; r < G::R0; ++r) x[b * G::R0 + r] = line[chs::rpad<G::PS>(t + b * G::TL + r * (L / G::R0))];
     chs::wave_lds_sync();
     // the block's planes k0 .. k0+TK-1 from one wave-uniform base: a lane's offset is 32-bit
-    constexpr int G2 = CELLS ? 0 : 2;   // ghost rows of a plane
-    const auto pb = uniform(phi + (size_t)k0 * (M + G2) * L);
-    const unsigned pl = (unsigned)(2 * li) * (unsigned)((M + G2) * L), ps = (unsigned)((M + G2) * L);
+    const int row0 = RT ? out.row0 : 0;
+    const unsigned ps = (unsigned)((M + 2 - 2 * row0) * L);   // a plane
+    const bool lo = J == 1 && row0 == 0, hi = J == M && row0 == 0;   // ghost rows
+    const auto pb = uniform(out.phi + (size_t)k0 * ps), pr = uniform(out.phi + (size_t)k0 * ps + (size_t)(J - row0) * L);
+    const unsigned pl = (unsigned)(2 * li) * ps;
     chs::rfft_line<T, L>(x, line, t, tw, +1, [&](int i, const cpx<T> &z) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const unsigned o = pl + h * ps + (unsigned)i;
             const double val = h == 0 ? (double)z.x : (double)z.y;
-            pb[o + (unsigned)((CELLS ? J - 1 : J) * L)] = val;
-            if (!CELLS && J == 1) pb[o] = val;
-            if (!CELLS && J == M) pb[o + (unsigned)((M + 1) * L)] = val;
+            pr[o] = val;
+            if (lo) pb[o] = val;
+            if (hi) pb[o + (unsigned)((M + 1) * L)] = val;
         }
     });
 }
@@ -3713,8 +3718,7 @@ void fftx_inv_r(int L, dim3 grid, hipStream_t st, const Geo &g, const cpx<T> *tw
     switch (L) {
 #define X(n) \
     case n: \
-        if (out.row0) hipLaunchKernelGGL((k_fftx_inv_r<T, n, sizeof(T) == 8>), grid, dim3(64), 0, st, g, tw, spec, out.phi); \
-        else hipLaunchKernelGGL((k_fftx_inv_r<T, n, false>), grid, dim3(64), 0, st, g, tw, spec, out.phi); \
+        hipLaunchKernelGGL((k_fftx_inv_r<T, n>), grid, dim3(64), 0, st, g, tw, spec, out); \
         break;
         CHS_RCASES(X)
 #undef X

@@ -624,3 +624,22 @@ def test_lds_convection_matches_oracle(pkg, L, M, N):
         gq, gp = ch.download()
         assert max(rel(gq[c], o.q[c]) for c in range(3)) < 1e-10 and rel(gp, o.pr) < 1e-10
         ch.close()
+
+
+@pytest.mark.parametrize("L,M,N", [(64, 64, 64), (64, 20, 96), (128, 12, 64), (256, 12, 256), (512, 8, 512), (1024, 6, 64),
+                                   (96, 80, 96), (256, 192, 64), (16, 16, 16)])
+def test_poisson_entry_points_agree_to_the_bit(pkg, L, M, N):
+    """The host entry point's solution (through the halo field) and the device one's (cells) are the same
+    bits for each kind of x-transform, in both forms."""
+    co = pkg.channel_setup(L, M, N, STR2=1.9)
+    r = np.random.default_rng(L + N).standard_normal((N, M, L))
+    for mode in (pkg.PLAIN_FP64, pkg.MIXED):
+        ch = pkg.ChannelTG(co, mode)
+        phi = ch.poisson(r)
+        d_r, d_p = pkg.DeviceArray.from_host(r), pkg.DeviceArray(r.shape)
+        ch.poisson_device(d_r.ptr, d_p.ptr, 0, False)
+        ch.sync()
+        assert np.array_equal(d_p.to_host(), phi), mode
+        for d in (d_r, d_p):
+            d.free()
+        ch.close()
