@@ -3296,7 +3296,8 @@ struct Tune {
     int ytdma_c = -1;                   // k_ytdma_chunk rows per chunk (-1 auto = 16, 0 = k_ytdma)
     int conv_lds = 2;                   // k_conv_rhs_lds rows per block (1, 2, 4; 0 = k_conv_rhs)
     int conv_dma = 4;                   // k_conv_rhs_dma rows per block (2, 4; 0 = k_conv_rhs_lds)
-    int divg_nxcd = 8;                  // XCDs the k_divg_fftx_r rows are grouped for (1 = off)
+    int divg_nxcd = 0;                  // XCDs the forward x-transform's rows are grouped for (1 = off; 0: 8,
+                                        // or off where its runs of the spectrum are short)
     int cny3_ky = -2;                   // k_cn_y3_march rows per chunk (-2 by the mesh; 0 = M; -1 = one launch per component)
     int upd_kz = 0;                     // k_update z-planes per thread (0: by the mesh)
     int upd_by = 4;                     // k_update rows per block (1, 2, 4, 8, 16)
@@ -3852,9 +3853,14 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
     //  z     register plan where N has one (256x192x256: 78 / 34 / 39), else mixed radix
     //        (N = 120: 20 / - / 13);
     //  x     register plan where L has one, except where mixed radix is faster: L >= 512, whose plan
-    //        holds one line, so two planes or 32-byte runs of the spectrum, per wavefront
-    //        (512x192x512 forward 520 / 552 / 349, inverse 340 / 263 / 208; FP32 inverse
-    //        188 / 162 / 145), and the FP64 forward transform with the divergence of L = 128, whose
+    //        holds one line, so two planes or 32-byte runs of the spectrum, per wavefront, on meshes
+    //        whose spectrum does not stay in the caches between those runs (plan / mixed radix, FP64
+    //        and FP32; forward 512x48x64 14.5 / 17.0 and 13.4 / 16.5, 512x96x90 52 / 49 and 43 / 37,
+    //        1024x64x128 75 / 71 and 83 / 68, 512x192x512 552 / 348 and 491 / 377; inverse 512x64x128
+    //        18 / 22 and 15 / 21, 512x128x256 50 / 55 and 42 / 45, 512x192x256 106 / 91 and 73 / 69,
+    //        512x192x512 261 / 184 and 163 / 144; 512x97x250, whose planes are not 128-byte lines,
+    //        75 / 53 and 75 / 47, 1024x96x90 33 / 40 and 28 / 33);
+    //        and the FP64 forward transform with the divergence of L = 128, whose
     //        plan takes 18 us on any small mesh.  Plan / mixed radix over 11 meshes: L = 128 1.00 to 1.66
     //        (128x16x64 18.2 / 11.0, 128x96x128 20.5 / 17.7, 128x192x256 72.5 / 54.3), L = 64 0.76 to
     //        1.01, L = 256 0.88 to 1.04 (1.15 and 1.23 with 48 and 16 rows of 64).  Of a given field the
@@ -3863,12 +3869,20 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
     // The LDS transforms remain for lengths with no plan of two or three passes of at most 256
     // threads a line, for fft_reg = 0 and for the batched ensemble.
     const bool f64 = sizeof(T) == 8, fr = c->tune.fft_reg != 0, gxok = c->gtwx && c->gtwxi;
-    const bool rx = fr && c->rtwx && !(gxok && (L >= 512 || (f64 && L == 128 && !src)));
-    const bool rxi = fr && c->rtwx && !(gxok && L >= 512);
+    const double points = (double)L * M * N;
+    const bool far = L >= 512 && points > 4.2e6, fari = L >= 512 && points > (N % 16 ? 1.0e7 : 1.7e7);
+    const bool rx = fr && c->rtwx && !(gxok && (far || (f64 && L == 128 && !src)));
+    const bool rxi = fr && c->rtwx && !(gxok && fari);
     const bool rz = fr && c->rtwz;
     const bool mx = fr && !rx && gxok, mxi = fr && !rxi && gxok, mz = fr && !rz && c->gtwz;
     const int TKR = 2 * (c->rtwx ? chs::rplan_lpw(L) : 1), LPZ = rz ? chs::rplan_lpw(N) : 1;
     const int TKG = gxok ? gx_planes(c->gx, sizeof(cpx<T>), M, N) : 2;
+    // Rows grouped by XCD share the v row between two of them in one L2.  A block that writes a part of
+    // the spectrum's 128-byte lines leaves the rest to the next planes' blocks, which then come all of
+    // M rows later, when those lines have left the L2: runs of 16 and 32 bytes (FP32 also 64) in dispatch
+    // order (us, grouped / not: 1280x64x128 FP32 133 / 96, FP64 127 / 101; 1024x64x128 FP32 80 / 68;
+    // 512x128x256 FP32 124 / 115, FP64 120 / 124; 1024x128x256 FP64 276 / 290).
+    const int NXG = c->tune.divg_nxcd > 0 ? c->tune.divg_nxcd : TKG * sizeof(cpx<T>) >= (f64 ? 64 : 128) ? 8 : 1;
     const dim3 gxg(M, (N + TKG - 1) / TKG);
     const int NLG = mz ? gz_lines(c->gz, sizeof(cpx<T>), M * H) : 1;
     const dim3 gzg((M * H + NLG - 1) / NLG);
@@ -3882,11 +3896,11 @@ void poisson_launch(chs_ctx *c, const double *dv, double talp, const double *src
         EvScope ev(c, "divg_fftx");
         if (rx)
             divg_fftx_r<T>(L, dim3(M, N / TKR), c->stream, g, (const cpx<T> *)c->rtwx, dv, talp, qv, dvo, spec, src,
-                           c->tune.divg_nxcd);
+                           c->tune.divg_nxcd > 0 ? c->tune.divg_nxcd : 8);
         else if (mx)
             hipLaunchKernelGGL((src ? k_divg_fftx_g<T, 2> : dvo ? k_divg_fftx_g<T, 1> : k_divg_fftx_g<T, 0>), gxg,
                                dim3(block_threads(TKG / 2 * c->gx.tpl)), sizeof(cpx<T>) * (TKG / 2) * c->gx.ls, c->stream,
-                               g, c->gx, (const cpx<T> *)c->gtwx, dv, talp, qv, dvo, spec, src, TKG, c->tune.divg_nxcd);
+                               g, c->gx, (const cpx<T> *)c->gtwx, dv, talp, qv, dvo, spec, src, TKG, NXG);
         else
             hipLaunchKernelGGL(k_divg_fftx<T>, dim3(M, N / TK), dim3(256), shx, c->stream, g, pa, dv, talp, qv, dvo,
                                spec, TK, src);

@@ -169,7 +169,7 @@ int chs_set_refinement(chs_ctx *ctx, int nref_step, int nref_projection);
  * block where its plane fits, else chunks of 4 to 16 rows; 4, 8, 16; 0 = unchunked); "ytdma_bs"
  * threads per block of the unchunked y-solve (64 default, 128, 256) and "ytdma_rb" its rows per
  * load batch (8, 16 default); "divg_nxcd" the XCDs the divergence transform's tiles are grouped
- * for (8; 1 = dispatch order).
+ * for (1..64, 1 = dispatch order; by default 8, or 1 where the tiles' runs of the spectrum are short).
  * Correction: "upd_kz" z-planes each thread marches (by default 2 or 4 by the mesh) and "upd_by" its
  * rows per block (4), "upd_nxcd" the XCDs its tiles are grouped for (1), "upd_w2" 1 (default) for two
  * points per lane where L is a multiple of 128 (0: one).

@@ -643,3 +643,37 @@ def test_poisson_entry_points_agree_to_the_bit(pkg, L, M, N):
         for d in (d_r, d_p):
             d.free()
         ch.close()
+
+
+@pytest.mark.parametrize("L,M,N", [(512, 20, 512), (512, 84, 250), (1024, 22, 200), (512, 16, 500)])
+def test_long_x_lines_each_side_of_the_rule(pkg, L, M, N):
+    """L >= 512 takes the register plan's x-transforms on small meshes and the mixed-radix ones on large, the
+    forward and the inverse each from a size of its own: both mixes against the oracle, bounds as
+    test_poisson_matches_oracle."""
+    print(f"long x lines {L}x{M}x{N}", flush=True)
+    test_mixed_radix_poisson_matches_oracle_and_device_output(pkg, L, M, N)
+
+
+@pytest.mark.parametrize("L,M,N,mode", [(1280, 64, 128, "mixed"), (1280, 64, 128, "plain"), (1024, 96, 128, "mixed")])
+def test_forward_transform_tile_order_is_the_faster(pkg, L, M, N, mode):
+    """Rows grouped by XCD or in dispatch order, whichever the mesh chose: within 8 % of the faster of the
+    two (short runs of the spectrum grouped cost 28 to 38 % at 1280x64x128)."""
+    ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=1.8), pkg.MIXED if mode == "mixed" else pkg.PLAIN_FP64)
+    rng = np.random.default_rng(1)
+    ch.upload(1e-3 * rng.standard_normal((3, N, M + 2, L)), np.zeros((N, M + 2, L)))
+
+    def kernel_ms():
+        for _ in range(2):
+            ch.rk3_step(1.0e-6, 1.0 / 2800.0)
+        ch.profile_reset("divg_fftx")
+        for _ in range(10):
+            ch.rk3_step(1.0e-6, 1.0 / 2800.0)
+        return ch.profile_get("divg_fftx")[0]
+
+    auto, by_hand = kernel_ms(), []
+    for nx in (1, 8):
+        ch.set_tuning(divg_nxcd=nx)
+        by_hand.append(kernel_ms())
+    print(f"  by the mesh {auto:.4f} ms, dispatch order and grouped {by_hand}")
+    assert auto < 1.08 * min(by_hand)
+    ch.close()
