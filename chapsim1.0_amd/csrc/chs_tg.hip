@@ -3796,10 +3796,15 @@ int upd_planes(int want, int L, int M, int N)
 int block_threads(int n) { return (n + 63) / 64 * 64; }
 
 // Rows per chunk of k_ytdma_wide, 0 where k_ytdma_chunk or k_ytdma runs: automatic (want = -1)
-// only, and M <= 1024 (64 chunks of 16).  k_ytdma_chunk keeps M <= 128 (128x96x128: 15.8 us
-// against 16.4 to 21.5 with 4 to 16 rows) and, up to the 256 rows it covers, fft_reg = 0, whose
-// steps the batched launches reproduce.  us by rows per chunk 8 / 12 / 16, and before:
-// 256x192x256 68 / 48 / 57, 70; 250x300x250 108 / 94 / 122; 512x384x512 425 / 449 / 545, 886.
+// only, and M <= 1024 (64 chunks of 16).  k_ytdma_chunk keeps M <= 128 and, up to the 256 rows it
+// covers, fft_reg = 0, whose steps the batched launches reproduce.  A block's wavefronts (four
+// chunks each) have to fill the 16 that a CU holds at these registers: 4 with 12 rows at M = 192, 8
+// with 8 rows at M = 256, where 12 rows make 6 and leave four places empty.  us by rows per chunk
+// 8 / 12 / 16, and before: 128x128x128 17 / 18 / 22, 17; 256x128x256 38 / 40 / 43, 43; 128x144x128
+// 17 / 17 / 21, 20; 256x192x256 71 / 53 / 63, 76; 256x224x256 80 / 83 / 82, 83; 128x256x128
+// 24 / 31 / 24, 26; 256x256x256 82 / 103 / 89, 89; 256x300x256 116 / 111 / 144, 149; 90x400x120
+// 35 / 33 / 26, 87; 128x512x128 61 / 59 / 50, 108; 512x384x512 425 / 449 / 545, 886; 128x600x128
+// - / 73 / 78, 129; 128x768x128 - / 84 / 88, 177; 128x900x128 - / - / 98, 208.
 // The FP32 spectrum keeps 16 rows up to M = 256, as k_ytdma_chunk: the FP64 sweeps round to FP32 at the
 // end, and other chunks move a few of those roundings, which p shows by 3e-6 of its size
 // (256x192x256: 77 us in k_ytdma_chunk, 58 here).
@@ -3807,10 +3812,14 @@ int ytdma_wide_rows(int want, int fft_reg, int M, bool f64)
 {
     if (want >= 0 || M > 1024 || M <= 128 || (M <= 256 && !fft_reg)) return 0;
     if (!f64 && M <= 256) return 16;
-    return M <= 320 || (M > 512 && M <= 768) ? 12 : (M <= 512 ? 8 : 16);
+    return M <= 192 || (M > 256 && M <= 320) || (M > 512 && M <= 768) ? 12 : (M <= 512 ? 8 : 16);
 }
 
-// Rows per chunk of k_spec_plane (4, 8 or 12; 1024 / N chunks), 0 where a plane does not fit.
+// Rows per chunk of k_spec_plane (4, 8 or 12; 1024 / N chunks), 0 where a plane does not fit.  Any L: the
+// whole solve takes, by this kernel / the three (us), 64x64 planes L = 64 20 / 24, 384 42 / 54, and
+// from 512 on, where its blocks need a second round of the 256 CUs, 512 56 / 59, 1024 77 / 77,
+// 2048 137 / 148; 80x96 planes 1.02 to 1.24 to L = 2048.  Small planes lose there (16x30 512 33 / 27,
+// 2048 73 / 47), and N = 250 a little everywhere (36x250 L = 256 71 / 67).
 int plane_rows(const chs::GPlan &P, int M, int N)
 {
     if (N > 512 || M * P.tpl > 1024 || M * P.ls > kPlaneCpx) return 0;

@@ -677,3 +677,29 @@ def test_forward_transform_tile_order_is_the_faster(pkg, L, M, N, mode):
     print(f"  by the mesh {auto:.4f} ms, dispatch order and grouped {by_hand}")
     assert auto < 1.08 * min(by_hand)
     ch.close()
+
+
+@pytest.mark.parametrize("L,M,N", [(128, 256, 128), (128, 224, 128), (128, 144, 128), (64, 250, 64)])
+def test_wide_ytdma_is_no_slower_than_the_chunks_it_replaces(pkg, L, M, N):
+    """The y-Thomas that the mesh chooses against 16-row chunks of 64 lines (ytdma_c = 16), kernel times
+    within 8 % (12-row chunks at M = 256, six wavefronts a block, took 23 % longer)."""
+    ch = pkg.ChannelTG(pkg.channel_setup(L, M, N, STR2=1.9), pkg.PLAIN_FP64)
+    d_r = pkg.DeviceArray.from_host(np.random.default_rng(1).standard_normal((N, M, L)))
+    d_p = pkg.DeviceArray((N, M, L))
+
+    def kernel_ms():
+        for _ in range(3):
+            ch.poisson_device(d_r.ptr, d_p.ptr, 0, False)
+        ch.profile_reset("ytdma")
+        for _ in range(20):
+            ch.poisson_device(d_r.ptr, d_p.ptr, 0, False)
+        return ch.profile_get("ytdma")[0]
+
+    auto = kernel_ms()
+    ch.set_tuning(ytdma_c=16)
+    chunks = kernel_ms()
+    print(f"  {L}x{M}x{N}: by the mesh {auto:.4f} ms, 16-row chunks {chunks:.4f} ms")
+    assert auto < 1.08 * chunks
+    for d in (d_r, d_p):
+        d.free()
+    ch.close()
